@@ -14,6 +14,7 @@
 //          so the result does not depend on timing)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "m3_common.h"
@@ -132,47 +133,112 @@ int launch_silu_mul(const void* gu, void* out, int64_t rows, int dff, int64_t st
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-template <typename TX, typename TW, typename TG>
-__global__ __launch_bounds__(kNormThreads) void rmsnorm_dx_kernel(
+// dx and the column partials of dw in one launch: the first ndw blocks sum 64 columns of one
+// partial's kNormRowsPerPart rows at a time (16 waves, every 16th row each, met in LDS in wave
+// order), the others take 16 rows of dx, one per wave, in pieces of four elements when VEC.
+// Bound by HBM and, at a few thousand rows, by launch and memory latency. One thread per column
+// walking a partial's 256 rows in turn (three dozen blocks) took 71 us at (3002, 768) bf16, the
+// scalar dx pass 10 us and the sum 5 us; this launch and its sum take 10 us together.
+constexpr int kNormBwdThreads = 1024;
+
+template <typename T>
+struct __align__(4 * sizeof(T)) NormPiece {
+    T v[4];
+};
+
+template <typename TX, typename TW, typename TG, bool VEC>
+__global__ __launch_bounds__(kNormBwdThreads) void rmsnorm_bwd_kernel(
     const void* __restrict__ x, const void* __restrict__ w, const float* __restrict__ rstd,
-    const void* __restrict__ g, void* __restrict__ dx, int64_t rows, int d) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * (kNormThreads / 64) + (threadIdx.x >> 6);
+    const void* __restrict__ g, void* __restrict__ dx, float* __restrict__ part, int64_t rows,
+    int d, int nparts, unsigned ndw) {
+    constexpr int W = kNormBwdThreads / 64;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (blockIdx.x < ndw) {
+        __shared__ float acc_s[W][64];
+        const int64_t njobs = (int64_t)nparts * ((d + 63) / 64);
+        for (int64_t job = blockIdx.x; job < njobs; job += ndw) {
+            const int64_t i = job % nparts;
+            const int j = (int)(job / nparts) * 64 + lane;
+            const int jc = j < d ? j : d - 1;
+            const int64_t r0 = i * kNormRowsPerPart;
+            const int64_t r1 = r0 + kNormRowsPerPart < rows ? r0 + kNormRowsPerPart : rows;
+            float acc = 0.f;
+#pragma unroll 8
+            for (int64_t r = r0 + wave; r < r1; r += W)
+                acc += ldf<TG>(g, r * d + jc) * ldf<TX>(x, r * d + jc) * rstd[r];
+            acc_s[wave][lane] = acc;
+            __syncthreads();
+            if (wave == 0 && j < d) {
+                float v = acc_s[0][lane];
+                for (int k = 1; k < W; ++k) v += acc_s[k][lane];
+                part[i * d + j] = v;
+            }
+            __syncthreads();  // the sums are read before the next job's are written
+        }
+        return;
+    }
+    const int64_t row = (int64_t)(blockIdx.x - ndw) * W + wave;
     if (row >= rows) return;
     const int64_t base = row * d;
     const float s = rstd[row];
     float acc = 0.f;
-    for (int j = lane; j < d; j += 64)
-        acc += ldf<TW>(w, j) * ldf<TG>(g, base + j) * ldf<TX>(x, base + j);
-    acc = group_sum<64>(acc);
-    const float c = s * s * s * acc / (float)d;
-    for (int j = lane; j < d; j += 64)
-        stf<TX>(dx, base + j, s * ldf<TW>(w, j) * ldf<TG>(g, base + j) - ldf<TX>(x, base + j) * c);
+    if constexpr (VEC) {
+        const NormPiece<TX>* xr = reinterpret_cast<const NormPiece<TX>*>(x) + base / 4;
+        const NormPiece<TG>* gr = reinterpret_cast<const NormPiece<TG>*>(g) + base / 4;
+        const NormPiece<TW>* wr = reinterpret_cast<const NormPiece<TW>*>(w);
+        NormPiece<TX>* dr = reinterpret_cast<NormPiece<TX>*>(dx) + base / 4;
+        const int pieces = d / 4;
+#pragma unroll 4
+        for (int c = lane; c < pieces; c += 64) {
+            const NormPiece<TX> xp = xr[c];
+            const NormPiece<TG> gp = gr[c];
+            const NormPiece<TW> wp = wr[c];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc += (float)wp.v[e] * (float)gp.v[e] * (float)xp.v[e];
+        }
+        acc = lane_sum<64>(acc);
+        const float c3 = s * s * s * acc / (float)d;
+#pragma unroll 4
+        for (int c = lane; c < pieces; c += 64) {
+            const NormPiece<TX> xp = xr[c];
+            const NormPiece<TG> gp = gr[c];
+            const NormPiece<TW> wp = wr[c];
+            NormPiece<TX> o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                o.v[e] = (TX)(s * (float)wp.v[e] * (float)gp.v[e] - (float)xp.v[e] * c3);
+            dr[c] = o;
+        }
+    } else {
+        for (int j = lane; j < d; j += 64)
+            acc += ldf<TW>(w, j) * ldf<TG>(g, base + j) * ldf<TX>(x, base + j);
+        acc = lane_sum<64>(acc);
+        const float c3 = s * s * s * acc / (float)d;
+        for (int j = lane; j < d; j += 64)
+            stf<TX>(dx, base + j, s * ldf<TW>(w, j) * ldf<TG>(g, base + j) - ldf<TX>(x, base + j) * c3);
+    }
 }
 
-// Column partials of dw: block (i, c) sums rows i*kNormRowsPerPart .. +kNormRowsPerPart-1 for
-// columns c*256 .. c*256+255, one column per thread.
-template <typename TX, typename TG>
-__global__ __launch_bounds__(kNormThreads) void rmsnorm_dw_part_kernel(
-    const void* __restrict__ x, const float* __restrict__ rstd, const void* __restrict__ g,
-    float* __restrict__ part, int64_t rows, int d) {
-    const int j = blockIdx.y * kNormThreads + threadIdx.x;
-    if (j >= d) return;
-    const int64_t r0 = (int64_t)blockIdx.x * kNormRowsPerPart;
-    const int64_t r1 = r0 + kNormRowsPerPart < rows ? r0 + kNormRowsPerPart : rows;
-    float acc = 0.f;
-    for (int64_t r = r0; r < r1; ++r) acc += ldf<TG>(g, r * d + j) * ldf<TX>(x, r * d + j) * rstd[r];
-    part[(int64_t)blockIdx.x * d + j] = acc;
-}
-
+// dw = the sum of the partials in order: 64 columns per block, its 4 waves take every 4th
+// partial, then meet in LDS in wave order.
 template <typename TW>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_dw_sum_kernel(
     const float* __restrict__ part, void* __restrict__ dw, int nparts, int d) {
-    const int j = blockIdx.x * kNormThreads + threadIdx.x;
-    if (j >= d) return;
+    constexpr int W = kNormThreads / 64;
+    __shared__ float acc_s[W][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int j = blockIdx.x * 64 + lane;
+    const int jc = j < d ? j : d - 1;
     float acc = 0.f;
-    for (int i = 0; i < nparts; ++i) acc += part[(int64_t)i * d + j];
-    stf<TW>(dw, j, acc);
+#pragma unroll 8
+    for (int i = wave; i < nparts; i += W) acc += part[(int64_t)i * d + jc];
+    acc_s[wave][lane] = acc;
+    __syncthreads();
+    if (wave == 0 && j < d) {
+        float v = acc_s[0][lane];
+        for (int k = 1; k < W; ++k) v += acc_s[k][lane];
+        stf<TW>(dw, j, v);
+    }
 }
 
 size_t rmsnorm_bwd_workspace(int64_t rows, int d) {
@@ -221,14 +287,25 @@ int launch_rmsnorm_fwd(const void* x, int xdtype, const void* w, int wdtype, voi
 template <typename TX, typename TW, typename TG>
 static void launch_bwd_t(const void* x, const void* w, const float* rstd, const void* g,
                          void* dx, void* dw, float* part, int64_t rows, int d, hipStream_t stream) {
-    hipLaunchKernelGGL((rmsnorm_dx_kernel<TX, TW, TG>), dim3((unsigned)((rows + 3) / 4)),
-                       dim3(kNormThreads), 0, stream, x, w, rstd, g, dx, rows, d);
     const int64_t nparts = (rows + kNormRowsPerPart - 1) / kNormRowsPerPart;
-    const unsigned cb = (unsigned)((d + kNormThreads - 1) / kNormThreads);
-    hipLaunchKernelGGL((rmsnorm_dw_part_kernel<TX, TG>), dim3((unsigned)nparts, cb),
-                       dim3(kNormThreads), 0, stream, x, rstd, g, part, rows, d);
-    hipLaunchKernelGGL((rmsnorm_dw_sum_kernel<TW>), dim3(cb), dim3(kNormThreads), 0, stream, part,
-                       dw, (int)nparts, d);
+    const int64_t cb = (d + 63) / 64;
+    constexpr int W = kNormBwdThreads / 64;
+    // at most 65536 dw blocks, so that the grid stays within 2^32 threads for every row count
+    // that dx alone allows
+    const unsigned ndw = (unsigned)std::min<int64_t>(nparts * cb, 65536);
+    const dim3 grid((unsigned)(ndw + (rows + W - 1) / W));
+    // four-element pieces need whole, aligned pieces in every row
+    auto al = [](const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; };
+    const bool vec = d % 4 == 0 && al(x, 4 * sizeof(TX)) && al(dx, 4 * sizeof(TX)) &&
+                     al(w, 4 * sizeof(TW)) && al(g, 4 * sizeof(TG));
+    if (vec)
+        hipLaunchKernelGGL((rmsnorm_bwd_kernel<TX, TW, TG, true>), grid, dim3(kNormBwdThreads), 0,
+                           stream, x, w, rstd, g, dx, part, rows, d, (int)nparts, ndw);
+    else
+        hipLaunchKernelGGL((rmsnorm_bwd_kernel<TX, TW, TG, false>), grid, dim3(kNormBwdThreads), 0,
+                           stream, x, w, rstd, g, dx, part, rows, d, (int)nparts, ndw);
+    hipLaunchKernelGGL((rmsnorm_dw_sum_kernel<TW>), dim3((unsigned)cb), dim3(kNormThreads), 0, stream,
+                       part, dw, (int)nparts, d);
 }
 
 template <typename TX, typename TW>

@@ -57,6 +57,33 @@ def test_rmsnorm_fp32_forward_and_gradients_match_oracle(rows, d, cuda_device):
     assert max_rel(rstd, want) < 1e-6
 
 
+# (rows, d) at the backward's edges: one row past a partial's 256, one past a wave pass of 16,
+# a last block of 64 columns with one valid, rows of whole pieces and rows of none, and a
+# storage offset that leaves rows of whole pieces unaligned. (Not d = 1: there dx is the
+# difference of two equal terms, eps / (x^2 + eps) ~ 1e-5 of either, so their roundings of
+# 6e-8 alone are 1e-2 of it.)
+@pytest.mark.parametrize("rows,d,offset", [(257, 65, 0), (17, 4, 0), (256, 64, 0), (255, 768, 1),
+                                           (513, 260, 0), (1, 5, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rmsnorm_backward_edges_match_oracle(rows, d, offset, dtype, cuda_device):
+    """dx and dw against the fp64 oracle on the same rounded inputs: one rounding to the
+    dtype of a result whose fp32 sums of at most 513 terms err by less than 1e-5 of its
+    largest entry (bf16: half an ulp, 2^-9, of the entry)."""
+    print(f"rmsnorm backward rows {rows} d {d} offset {offset} {dtype}", flush=True)
+    g = torch.Generator().manual_seed(rows + 3 * d)
+    flat = [torch.randn(rows * d + offset, generator=g).to(dtype) for _ in range(2)]
+    w = torch.randn(d, generator=g).to(dtype)
+    x, gy = (t[offset:].view(rows, d) for t in flat)
+    xr, wr = x.double().requires_grad_(), w.double().requires_grad_()
+    (ref.rmsnorm(xr, wr, 1e-5) * gy.double()).sum().backward()
+    xd, gd = (t.to(cuda_device)[offset:].view(rows, d) for t in flat)
+    rstd = torch.rsqrt(xd.float().square().mean(-1) + 1e-5)
+    dx, dw = ops.rmsnorm_bwd(xd, w.to(cuda_device), rstd, gd)
+    tol = 1e-5 if dtype == torch.float32 else 2.0 ** -8
+    assert max_rel(dx, xr.grad) < tol
+    assert max_rel(dw, wr.grad) < tol
+
+
 def test_rmsnorm_over_a_leading_dimension(cuda_device):
     """RMSNorm(d, dim=1) on (B, d, T) normalises over dim 1, as the reference's dim argument
     does (mamba3/mamba3.py:27-35)."""
