@@ -120,8 +120,9 @@ const char* m3_status_string(int status);
 int m3_version(void);
 
 /*
- * Name of the prefill kernel m3_prefill_fwd would run for these arguments (the dispatch
- * depends on the shape, dtype, flags and the pointers' alignment): "mfma_d128_p64_r2",
+ * Name of the prefill kernel m3_prefill_fwd would run for these arguments, given the workspace
+ * that m3_prefill_workspace_size asks for (the dispatch depends on the shape, dtype, flags, the
+ * pointers' alignment and, for bf16 layers outside the MFMA kernels, the workspace): "mfma_d128_p64_r2",
  * "mfma_general", "fp32_fused", "fp32_fused_train", "fp32_layer" or "generic"; NULL for an
  * invalid descriptor. No counterpart in the reference (one ATen path). A static string.
  */
@@ -183,7 +184,10 @@ int m3_layer_bwd(const m3_layer_desc* desc, const m3_layer_params* params, const
                  size_t workspace_bytes, void* stream);
 
 /*
- * Bytes of device workspace m3_prefill_fwd needs for `desc` (0 is possible).
+ * Bytes of device workspace m3_prefill_fwd needs for `desc` (0 is possible). bf16 layers that
+ * no bf16 MFMA kernel takes run the fp32 layer path in this workspace ("fp32_layer"), in
+ * slices of the batch where it is smaller, and the generic kernel, which needs none, where it
+ * does not hold one batch row; all of them compute in fp32, so results agree to its rounding.
  * No counterpart in the reference, which allocates inside ATen.
  */
 int m3_prefill_workspace_size(const m3_layer_desc* desc, size_t* bytes);
@@ -213,7 +217,8 @@ int m3_prefill_fwd(const m3_layer_desc* desc, const m3_layer_params* params,
  * harnesses that forbid hipMalloc). Same arguments, dispatch, kernels and results as
  * m3_prefill_fwd, but the workspace is a static array of the library on each GPU
  * (M3_NOALLOC_SCRATCH_BYTES, held from the first call on that GPU until the process
- * ends); calls needing more return M3_ERR_SCRATCH_LIMIT and launch nothing. It calls no
+ * ends; bf16 layers outside the MFMA kernels take what it holds, see
+ * m3_prefill_workspace_size); calls needing more return M3_ERR_SCRATCH_LIMIT and launch nothing. It calls no
  * allocator. M3_FLAG_FOR_BACKWARD is refused (M3_ERR_UNSUPPORTED): the backward's operands
  * would be left in the shared scratch, which the next call overwrites. The scratch keeps the last call's contents and needs no clearing (every
  * kernel writes what it later reads). All calls on one GPU share the array: calls that

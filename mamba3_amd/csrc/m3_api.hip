@@ -57,11 +57,12 @@ int check_scan_bwd_shape(int64_t batch, int64_t nchunks, int64_t nheads, int64_t
 // fused fp32 kernel
 // (fp32, d_state 128 / headdim 64 / rank 2; under M3_FLAG_FOR_BACKWARD it also writes the
 // staged operands of the layer backward into the fp32 layer workspace), the fp32 layer path
-// on the fp32-MFMA chunk kernels (fp32, rank 1..8) or the generic one.
-enum class PrefillPath { kMfma, kWide, kFp32Fused, kFp32FusedTrain, kFp32, kGeneric };
+// on the fp32-MFMA chunk kernels (fp32, rank 1..8; also bf16 layers outside the bf16 kernels,
+// where `limit` bytes of workspace hold its operands) or the generic one.
+enum class PrefillPath { kMfma, kWide, kFp32Fused, kFp32FusedTrain, kFp32, kStagedBf16, kGeneric };
 
 PrefillPath prefill_path(const m3_layer_desc& d, const void* proj, const void* y_out,
-                         const void* h_final, const void* prev_bx) {
+                         const void* h_final, const void* prev_bx, size_t limit) {
     const bool f16_ok = !(d.flags & M3_FLAG_NO_F16_OPERANDS);
     if (f16_ok && m3::mfma_prefill_supported(d, proj, y_out)) return PrefillPath::kMfma;
     if (f16_ok && m3::wide_prefill_supported(d) && aligned(h_final, 16)) return PrefillPath::kWide;
@@ -69,16 +70,18 @@ PrefillPath prefill_path(const m3_layer_desc& d, const void* proj, const void* y
     if ((d.flags & M3_FLAG_FOR_BACKWARD) && m3::fused_fp32_train_supported(d, proj, y_out, h_final, prev_bx))
         return PrefillPath::kFp32FusedTrain;
     if (m3::fp32_layer_supported(d)) return PrefillPath::kFp32;
+    if (m3::staged_bf16_workspace(d, limit) > 0) return PrefillPath::kStagedBf16;
     return PrefillPath::kGeneric;
 }
 
-size_t prefill_path_workspace(const m3_layer_desc& d, PrefillPath path) {
+size_t prefill_path_workspace(const m3_layer_desc& d, PrefillPath path, size_t limit) {
     switch (path) {
         case PrefillPath::kMfma: return m3::mfma_prefill_workspace(d);
         case PrefillPath::kWide: return m3::wide_prefill_workspace(d);
         case PrefillPath::kFp32Fused: return m3::fused_fp32_prefill_workspace(d);
         case PrefillPath::kFp32FusedTrain:
         case PrefillPath::kFp32: return m3::fp32_layer_workspace(d);
+        case PrefillPath::kStagedBf16: return m3::staged_bf16_workspace(d, limit);
         default: return m3::generic_prefill_workspace(d);
     }
 }
@@ -95,7 +98,8 @@ int check_prefill_args(const m3_layer_desc* desc, const m3_layer_params* params,
 
 int launch_prefill_path(PrefillPath path, const m3_layer_desc& d, const m3_layer_params& p,
                         const void* proj, const float* dt_scale, void* y_out, float* h_final,
-                        float* angle, float* prev_bx, void* ws, hipStream_t stream) {
+                        float* angle, float* prev_bx, void* ws, size_t limit,
+                        hipStream_t stream) {
     switch (path) {
         case PrefillPath::kMfma:
             return m3::launch_mfma_prefill(d, p, proj, dt_scale, y_out, h_final, angle, prev_bx,
@@ -116,6 +120,11 @@ int launch_prefill_path(PrefillPath path, const m3_layer_desc& d, const m3_layer
         case PrefillPath::kFp32:
             return m3::launch_fp32_layer(d, p, proj, dt_scale, y_out, h_final, angle, prev_bx,
                                          ws, stream) == 0
+                       ? M3_OK
+                       : M3_ERR_LAUNCH;
+        case PrefillPath::kStagedBf16:
+            return m3::launch_staged_bf16(d, p, proj, dt_scale, y_out, h_final, angle, prev_bx,
+                                          ws, limit, stream) == 0
                        ? M3_OK
                        : M3_ERR_LAUNCH;
         default:
@@ -184,12 +193,13 @@ int m3_version(void) { return 200; }
 const char* m3_prefill_kernel_name(const m3_layer_desc* desc, const void* proj, const void* y_out,
                                    const float* h_final, const float* prev_bx) {
     if (check_desc(desc) != M3_OK) return nullptr;
-    switch (prefill_path(*desc, proj, y_out, h_final, prev_bx)) {
+    switch (prefill_path(*desc, proj, y_out, h_final, prev_bx, SIZE_MAX)) {
         case PrefillPath::kMfma: return "mfma_d128_p64_r2";
         case PrefillPath::kWide: return "mfma_general";
         case PrefillPath::kFp32Fused: return "fp32_fused";
         case PrefillPath::kFp32FusedTrain: return "fp32_fused_train";
-        case PrefillPath::kFp32: return "fp32_layer";
+        case PrefillPath::kFp32:
+        case PrefillPath::kStagedBf16: return "fp32_layer";
         default: return "generic";
     }
 }
@@ -241,6 +251,7 @@ static size_t prefill_workspace(const m3_layer_desc& d) {
         n = std::max(n, m3::fused_fp32_prefill_workspace(d));
     if (m3::mfma_prefill_supported(d, nullptr, nullptr)) n = std::max(n, m3::mfma_prefill_workspace(d));
     if (m3::wide_prefill_supported(d)) n = std::max(n, m3::wide_prefill_workspace(d));
+    else n = std::max(n, m3::staged_bf16_workspace(d, SIZE_MAX));
     return n;
 }
 
@@ -257,12 +268,15 @@ int m3_prefill_fwd(const m3_layer_desc* desc, const m3_layer_params* params, con
                    float* prev_bx, void* workspace, size_t workspace_bytes, void* stream) {
     int st = check_prefill_args(desc, params, proj, y_out);
     if (st != M3_OK) return st;
-    const PrefillPath path = prefill_path(*desc, proj, y_out, h_final, prev_bx);
-    const size_t need = prefill_path_workspace(*desc, path);
+    // bf16 layers outside the bf16 MFMA kernels need no workspace: a caller's smaller one (or
+    // none) takes the slices, or the kernel, that it holds.
+    const size_t limit = workspace ? workspace_bytes : 0;
+    const PrefillPath path = prefill_path(*desc, proj, y_out, h_final, prev_bx, limit);
+    const size_t need = prefill_path_workspace(*desc, path, limit);
     if (need > 0 && (!workspace || workspace_bytes < need)) return M3_ERR_WORKSPACE;
     if (workspace && !aligned(workspace, 256)) return M3_ERR_MISALIGNED;
     return launch_prefill_path(path, *desc, *params, proj, dt_scale, y_out, h_final, angle,
-                               prev_bx, workspace, as_stream(stream));
+                               prev_bx, workspace, limit, as_stream(stream));
 }
 
 int m3_prefill_fwd_noalloc(const m3_layer_desc* desc, const m3_layer_params* params,
@@ -273,8 +287,9 @@ int m3_prefill_fwd_noalloc(const m3_layer_desc* desc, const m3_layer_params* par
     // The backward's operands would land in the shared scratch, which the next call
     // overwrites and no caller can hand to m3_layer_bwd.
     if (desc->flags & M3_FLAG_FOR_BACKWARD) return M3_ERR_UNSUPPORTED;
-    const PrefillPath path = prefill_path(*desc, proj, y_out, h_final, prev_bx);
-    const size_t need = prefill_path_workspace(*desc, path);
+    const size_t limit = M3_NOALLOC_SCRATCH_BYTES;
+    const PrefillPath path = prefill_path(*desc, proj, y_out, h_final, prev_bx, limit);
+    const size_t need = prefill_path_workspace(*desc, path, limit);
     if (need > M3_NOALLOC_SCRATCH_BYTES) return M3_ERR_SCRATCH_LIMIT;
     void* ws = nullptr;
     if (need > 0) {
@@ -282,7 +297,7 @@ int m3_prefill_fwd_noalloc(const m3_layer_desc* desc, const m3_layer_params* par
         if (st != M3_OK) return st;
     }
     return launch_prefill_path(path, *desc, *params, proj, dt_scale, y_out, h_final, angle,
-                               prev_bx, ws, as_stream(stream));
+                               prev_bx, ws, limit, as_stream(stream));
 }
 
 int m3_layer_bwd_workspace_size(const m3_layer_desc* desc, size_t* bytes) {

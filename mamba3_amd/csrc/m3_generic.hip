@@ -359,18 +359,36 @@ size_t generic_prefill_workspace(const m3_layer_desc&) {
     return 0;  // the running state lives in LDS
 }
 
+// The shape, headdim split and chunk of a layer under an LDS limit (Qi = 0: it does not fit).
+static GenShape gen_layer_shape(const m3_layer_desc& d, int max_lds) {
+    GenShape s;
+    s.B = d.batch; s.T = d.seqlen; s.H = d.nheads; s.P = d.headdim; s.N = d.d_state;
+    s.R = d.mimo_rank; s.Rb = d.mimo_rank; s.G = d.ngroups;
+    // Split headdim over workgroups while there are idle CUs (256) and blocks keep at
+    // least 16 columns: everything but the per-chunk preparation and the scores divides.
+    int PS = 1;
+    while (s.P % (2 * PS) == 0 && s.P / (2 * PS) >= 16 && (int64_t)d.batch * d.nheads * 2 * PS <= 256) PS *= 2;
+    s.PS = PS;
+    s.Pb = s.P / PS;
+    s.Qi = gen_pick_chunk(s.N, s.Pb, s.R, s.Rb, d.use_complex != 0, true, max_lds);
+    // A block's state rows that do not fit the LDS even at one token per chunk (d_state 512
+    // with headdim 256 at large batch x heads): narrower column blocks, PS the next divisor
+    // of P.
+    for (int ps = PS + 1; s.Qi == 0 && ps <= s.P; ++ps) {
+        if (s.P % ps != 0) continue;
+        s.PS = ps;
+        s.Pb = s.P / ps;
+        s.Qi = gen_pick_chunk(s.N, s.Pb, s.R, s.Rb, d.use_complex != 0, true, max_lds);
+    }
+    return s;
+}
+
+int generic_prefill_chunk(const m3_layer_desc& d) { return gen_layer_shape(d, kGenMaxLdsBig).Qi; }
+
 int launch_generic_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                            const float* dt_scale, void* y_out, float* h_final, float* angle,
                            float* prev_bx, void* workspace, hipStream_t stream) {
     GenLayerArgs A;
-    A.s.B = d.batch; A.s.T = d.seqlen; A.s.H = d.nheads; A.s.P = d.headdim; A.s.N = d.d_state;
-    A.s.R = d.mimo_rank; A.s.Rb = d.mimo_rank; A.s.G = d.ngroups;
-    // Split headdim over workgroups while there are idle CUs (256) and blocks keep at
-    // least 16 columns: everything but the per-chunk preparation and the scores divides.
-    int PS = 1;
-    while (A.s.P % (2 * PS) == 0 && A.s.P / (2 * PS) >= 16 && (int64_t)d.batch * d.nheads * 2 * PS <= 256) PS *= 2;
-    A.s.PS = PS;
-    A.s.Pb = A.s.P / PS;
     // Up to the CU's full LDS (one workgroup per CU): raise the kernel's dynamic-LDS limit.
     int max_lds = kGenMaxLds;
     if (d.dtype == M3_DTYPE_BF16)
@@ -381,18 +399,9 @@ int launch_generic_prefill(const m3_layer_desc& d, const m3_layer_params& p, con
         max_lds = hipFuncSetAttribute(reinterpret_cast<const void*>(&gen_layer_prefill<float>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, kGenMaxLdsBig) == hipSuccess
                       ? kGenMaxLdsBig : kGenMaxLds;
-    A.s.Qi = gen_pick_chunk(A.s.N, A.s.Pb, A.s.R, A.s.Rb, d.use_complex != 0, true, max_lds);
-    // A block's state rows that do not fit the LDS even at one token per chunk (d_state 512
-    // with headdim 256 at large batch x heads): narrower column blocks, PS the next divisor
-    // of P.
-    for (int ps = PS + 1; A.s.Qi == 0 && ps <= A.s.P; ++ps) {
-        if (A.s.P % ps != 0) continue;
-        A.s.PS = ps;
-        A.s.Pb = A.s.P / ps;
-        A.s.Qi = gen_pick_chunk(A.s.N, A.s.Pb, A.s.R, A.s.Rb, d.use_complex != 0, true, max_lds);
-    }
+    A.s = gen_layer_shape(d, max_lds);
     if (A.s.Qi == 0) return M3_ERR_UNSUPPORTED;
-    PS = A.s.PS;
+    const int PS = A.s.PS;
     A.L = gen_lds_plan(A.s.Qi, A.s.N, A.s.Pb, A.s.R, A.s.Rb, d.use_complex != 0, true);
     A.pl = proj_layout(d);
     A.row_stride = d.proj_row_stride;

@@ -46,6 +46,8 @@ int launch_scan_bwd(const float* decay, const float* h_states, const float* grad
 
 // Generic (fp32 VALU) fused layer prefill: any supported shape, any dtype.
 size_t generic_prefill_workspace(const m3_layer_desc& d);
+// Tokens per chunk of that kernel for a shape (0: the shape does not fit it).
+int generic_prefill_chunk(const m3_layer_desc& d);
 int launch_generic_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                            const float* dt_scale, void* y_out, float* h_final, float* angle,
                            float* prev_bx, void* workspace, hipStream_t stream);
@@ -137,6 +139,13 @@ size_t fp32_layer_workspace(const m3_layer_desc& d);
 int launch_fp32_layer(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                       const float* dt_scale, void* y_out, float* h_final, float* angle,
                       float* prev_bx, void* workspace, hipStream_t stream);
+// The same pipeline for bf16 layers the bf16 MFMA kernels do not take, fp32 in between, in
+// slices of the batch whose workspace stays within `limit` (and an own bound): workspace bytes
+// (0: not taken) and launcher (with the same limit).
+size_t staged_bf16_workspace(const m3_layer_desc& d, size_t limit);
+int launch_staged_bf16(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
+                       const float* dt_scale, void* y_out, float* h_final, float* angle,
+                       float* prev_bx, void* workspace, size_t limit, hipStream_t stream);
 
 // Backward of the fp32 layer prefill (gate, chunked SSD, preparation) from the forward's
 // workspace: workspace bytes and launcher.

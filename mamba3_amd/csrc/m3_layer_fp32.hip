@@ -1,5 +1,7 @@
-// fp32 layer prefill on the fp32-MFMA chunk kernels: the region between in_proj and out_proj
-// (mamba3/mamba3.py:199-256) for fp32 layers, as
+// Layer prefill on the fp32-MFMA chunk kernels: the region between in_proj and out_proj
+// (mamba3/mamba3.py:199-256) in fp32 arithmetic, for fp32 layers and for the bf16 layers no
+// bf16 MFMA kernel takes (T below is the type of the in_proj output and of y; everything in
+// between is fp32), as
 //   lp_dt      dt = softplus(dt_raw + dt_bias) [* dt_scale], A = -exp(A_log)
 //              (mamba3/mamba3.py:200-204)
 //   lp_angle_sums, lp_angles
@@ -18,6 +20,7 @@
 
 #include <algorithm>
 
+#include "m3_common.h"
 #include "m3_kernels.h"
 
 namespace m3 {
@@ -30,24 +33,29 @@ struct Args {
     ProjLayout pl;
     float eps;
     m3_layer_params prm;
-    const float* proj;
+    const void* proj;
     const float* dt_scale;
     float *dt, *A, *phi, *phi_sum, *xg, *xb, *xr, *Bt, *Bb, *Ct, *ys;  // workspace
-    float *y, *h_final, *angle, *prev_bx;                     // outputs
+    void* y;                                                           // outputs
+    float *h_final, *angle, *prev_bx;
 };
+
+template <typename T>
+__device__ __forceinline__ const T* proj_of(const Args& a) { return reinterpret_cast<const T*>(a.proj); }
 
 constexpr int NTH = 256;
 
 __device__ __forceinline__ float softplus(float v) { return v > 20.f ? v : log1pf(expf(v)); }
 
 // dt[b,t,h] and A[h].
+template <typename T>
 __global__ __launch_bounds__(NTH) void lp_dt(Args a) {
     const int64_t n = (int64_t)a.B * a.T * a.H;
     const int64_t e = (int64_t)blockIdx.x * NTH + threadIdx.x;
     if (e < a.H) a.A[e] = -expf(a.prm.A_log[e]);
     if (e >= n) return;
     const int h = (int)(e % a.H);
-    float d = softplus(a.proj[(e / a.H) * a.rs + a.pl.dt + h] + a.prm.dt_bias[h]);
+    float d = softplus(ld_f32(proj_of<T>(a) + (e / a.H) * a.rs + a.pl.dt + h) + a.prm.dt_bias[h]);
     if (a.dt_scale) d *= a.dt_scale[e];
     a.dt[e] = d;
 }
@@ -67,6 +75,7 @@ __device__ __forceinline__ void angle_job(const Args& a, int64_t e, int& b, int&
     b = (int)(bc / nc);
 }
 
+template <typename T>
 __global__ __launch_bounds__(NTH) void lp_angle_sums(Args a) {
     const int nc = (a.T + kAC - 1) / kAC;
     const int64_t n = (int64_t)a.B * nc * a.H * (a.N / 2);
@@ -77,22 +86,23 @@ __global__ __launch_bounds__(NTH) void lp_angle_sums(Args a) {
     float s = 0.f;
     const int t1 = min(a.T, (c + 1) * kAC);
     const float* dtp = a.dt + (int64_t)b * a.T * a.H + h;                  // stride H
-    const float* thp = a.proj + (int64_t)b * a.T * a.rs + a.pl.theta + i;  // stride rs
+    const T* thp = proj_of<T>(a) + (int64_t)b * a.T * a.rs + a.pl.theta + i;  // stride rs
     int t = c * kAC;
     for (; t + 8 <= t1; t += 8) {  // tokens added in order; eight loads ahead of their products
         float dv[8], tv[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             dv[u] = dtp[(int64_t)(t + u) * a.H];
-            tv[u] = thp[(int64_t)(t + u) * a.rs];
+            tv[u] = ld_f32(thp + (int64_t)(t + u) * a.rs);
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) s += dv[u] * tv[u];
     }
-    for (; t < t1; ++t) s += dtp[(int64_t)t * a.H] * thp[(int64_t)t * a.rs];
+    for (; t < t1; ++t) s += dtp[(int64_t)t * a.H] * ld_f32(thp + (int64_t)t * a.rs);
     a.phi_sum[e] = s;
 }
 
+template <typename T>
 __global__ __launch_bounds__(NTH) void lp_angles(Args a) {
     const int nc = (a.T + kAC - 1) / kAC;
     const int NH = a.N / 2;
@@ -105,7 +115,7 @@ __global__ __launch_bounds__(NTH) void lp_angles(Args a) {
     for (int cc = 0; cc < c; ++cc) s += a.phi_sum[(((int64_t)b * nc + cc) * a.H + h) * NH + i];
     const int t1 = min(a.T, (c + 1) * kAC);
     const float* dtp = a.dt + (int64_t)b * a.T * a.H + h;                  // stride H
-    const float* thp = a.proj + (int64_t)b * a.T * a.rs + a.pl.theta + i;  // stride rs
+    const T* thp = proj_of<T>(a) + (int64_t)b * a.T * a.rs + a.pl.theta + i;  // stride rs
     float* php = a.phi + ((int64_t)b * a.T * a.H + h) * NH + i;            // stride H*NH
     const int64_t ps = (int64_t)a.H * NH;
     // tokens in order; phi is a buffer of its own, so eight tokens' loads go out ahead of the
@@ -116,7 +126,7 @@ __global__ __launch_bounds__(NTH) void lp_angles(Args a) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             dv[u] = dtp[(int64_t)(t + u) * a.H];
-            tv[u] = thp[(int64_t)(t + u) * a.rs];
+            tv[u] = ld_f32(thp + (int64_t)(t + u) * a.rs);
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
@@ -125,7 +135,7 @@ __global__ __launch_bounds__(NTH) void lp_angles(Args a) {
         }
     }
     for (; t < t1; ++t) {
-        s += dtp[(int64_t)t * a.H] * thp[(int64_t)t * a.rs];
+        s += dtp[(int64_t)t * a.H] * ld_f32(thp + (int64_t)t * a.rs);
         php[t * ps] = -s;
     }
 }
@@ -133,6 +143,7 @@ __global__ __launch_bounds__(NTH) void lp_angles(Args a) {
 // One block per (b, t), one group at a time: the group's normalised B^ / C^ in LDS, the sin /
 // cos of a tile of its heads' RoPE pairs in LDS, then the rotated rows of those heads, as flat
 // loops over (head, element); then the x terms of every head.
+template <typename T>
 __global__ __launch_bounds__(NTH) void lp_prep(Args a) {
     // B^ [N*R], C^ [N*R], reduction scratch [2*NTH], sin / cos [HT*N/2] each
     extern __shared__ float sm[];
@@ -143,7 +154,7 @@ __global__ __launch_bounds__(NTH) void lp_prep(Args a) {
     float* red = sm + 2 * NR;
     float* sn = red + 2 * NTH;
     float* cn = sn + (int64_t)a.HT * NH;
-    const float* row = a.proj + ((int64_t)b * a.T + t) * a.rs;
+    const T* row = proj_of<T>(a) + ((int64_t)b * a.T + t) * a.rs;
     const int64_t tok0 = ((int64_t)b * a.T + t) * a.H;  // token row of head 0
     const int tid = threadIdx.x;
     const int hpg = a.H / a.G;
@@ -151,7 +162,8 @@ __global__ __launch_bounds__(NTH) void lp_prep(Args a) {
         if (g > 0) __syncthreads();  // the previous group's rows and sin / cos are read
         float sb = 0.f, sc = 0.f;
         for (int e = tid; e < NR; e += NTH) {
-            const float vb = row[a.pl.B + (int64_t)g * NR + e], vc = row[a.pl.C + (int64_t)g * NR + e];
+            const float vb = ld_f32(row + a.pl.B + (int64_t)g * NR + e);
+            const float vc = ld_f32(row + a.pl.C + (int64_t)g * NR + e);
             sb += vb * vb;
             sc += vc * vc;
         }
@@ -168,8 +180,8 @@ __global__ __launch_bounds__(NTH) void lp_prep(Args a) {
         const float rb = rsqrtf(red[0] / NR + a.eps), rc = rsqrtf(red[NTH] / NR + a.eps);
         for (int e = tid; e < NR; e += NTH) {
             const int64_t o = (int64_t)g * NR + e;
-            Bh[e] = row[a.pl.B + o] * rb * a.prm.B_norm_w[e] + a.prm.B_bias[o];
-            Ch[e] = row[a.pl.C + o] * rc * a.prm.C_norm_w[e] + a.prm.C_bias[o];
+            Bh[e] = ld_f32(row + a.pl.B + o) * rb * a.prm.B_norm_w[e] + a.prm.B_bias[o];
+            Ch[e] = ld_f32(row + a.pl.C + o) * rc * a.prm.C_norm_w[e] + a.prm.C_bias[o];
         }
         __syncthreads();
         // the group's heads in tiles of HT, so the sin / cos of a tile fit in LDS whatever
@@ -207,34 +219,35 @@ __global__ __launch_bounds__(NTH) void lp_prep(Args a) {
         const int h = j / PR, e = j % PR, p = e / a.R;
         const int64_t tok = tok0 + h;
         const float mx = a.prm.mimo_x[(int64_t)h * PR + e];
-        const float xr = row[a.pl.x + (int64_t)h * a.P + p] * mx;
+        const float xr = ld_f32(row + a.pl.x + (int64_t)h * a.P + p) * mx;
         float lam = 1.f;
-        if (a.trap) lam = 1.f / (1.f + expf(-row[a.pl.lam + h]));
+        if (a.trap) lam = 1.f / (1.f + expf(-ld_f32(row + a.pl.lam + h)));
         a.xr[tok * PR + e] = xr;
         a.xg[tok * PR + e] = xr * lam;
         if (a.trap) {
             const float sb = (1.f - lam) * expf(a.A[h] * a.dt[tok]);
-            const float xp = t > 0 ? row[a.pl.x + (int64_t)h * a.P + p - a.rs] * mx : 0.f;
+            const float xp = t > 0 ? ld_f32(row + a.pl.x + (int64_t)h * a.P + p - a.rs) * mx : 0.f;
             a.xb[tok * PR + e] = xp * sb;
         }
     }
 }
 
 // out[b,t,h*P+p] = sum_r mimo_down[h,p,r] y[b,t,h,p,r] silu(z[b,t,h*P+p] mimo_z[h,p,r]).
+template <typename T>
 __global__ __launch_bounds__(NTH) void lp_gate(Args a) {
     const int64_t n = (int64_t)a.B * a.T * a.H * a.P;
     const int64_t HP = (int64_t)a.H * a.P;
     for (int64_t e = (int64_t)blockIdx.x * NTH + threadIdx.x; e < n; e += (int64_t)gridDim.x * NTH) {
         const int64_t tok = e / HP;
         const int hp = (int)(e % HP);
-        const float z = a.proj[tok * a.rs + a.pl.z + hp];
+        const float z = ld_f32(proj_of<T>(a) + tok * a.rs + a.pl.z + hp);
         float acc = 0.f;
         for (int r = 0; r < a.R; ++r) {
             const int64_t pr = (int64_t)hp * a.R + r;
             const float zz = z * a.prm.mimo_z[pr];
             acc += a.prm.mimo_down[pr] * a.ys[e * a.R + r] * (zz / (1.f + expf(-zz)));
         }
-        a.y[e] = acc;
+        reinterpret_cast<T*>(a.y)[e] = cvt_out<T>(acc);
     }
 }
 
@@ -348,19 +361,66 @@ void* fp32_layer_scratch(const m3_layer_desc& d, void* ws, size_t* bytes) {
     return ws ? reinterpret_cast<char*>(ws) + pl.chunk_off : nullptr;
 }
 
-bool fp32_layer_supported(const m3_layer_desc& d) {
-    return d.dtype == M3_DTYPE_F32 && prep_heads_per_tile(d) > 0 &&
+static bool staged_shape_ok(const m3_layer_desc& d) {
+    return prep_heads_per_tile(d) > 0 &&
            chunked_fwd_mfma_workspace(d.batch, d.seqlen, d.nheads, d.headdim, d.d_state,
                                       d.mimo_rank, d.use_trapezoidal != 0) > 0;
+}
+
+bool fp32_layer_supported(const m3_layer_desc& d) {
+    return d.dtype == M3_DTYPE_F32 && staged_shape_ok(d);
 }
 
 size_t fp32_layer_workspace(const m3_layer_desc& d) {
     return fp32_layer_supported(d) ? lp::plan(d).total : 0;
 }
 
-int launch_fp32_layer(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
-                      const float* dt_scale, void* y_out, float* h_final, float* angle,
-                      float* prev_bx, void* workspace, hipStream_t stream) {
+// bf16 layers outside the bf16 MFMA kernels: the batch rows are independent, so they run in
+// slices whose staged operands stay within kStagedBf16Cap; a layer of which one row does not
+// fit runs on the generic kernel, and so do short sequences. That kernel walks the sequence on
+// the VALU, one workgroup per (batch, head, column block), at 30-50 us per LDS chunk of its own
+// (64 tokens of a small layer, 16 of d_state 128 rank 3); the ten launches here cost 50-60 us
+// before the tokens count (125 us at d_state 128 rank 3). us per call, generic / staged, bf16,
+// d_state N headdim P rank R:
+//   N 16 P 16 R 2   (16, 500) 431 / 144, (64, 256) 460 / 248, (2, 2000) 1640 / 107, (1, 65) 101 / 55
+//   N 16 P 64 R 1   (1, 65) 61 / 64, (1, 129) 92 / 66, (16, 500) 691 / 332
+//   N 128 P 64 R 3  (1, 16) 48 / 127, (1, 64) 158 / 140, (2, 2000) 4829 / 1054
+//   N 8 P 16 R 1    (1, 129) 86 / 53, (64, 128) 65 / 76, (128, 256) 125 / 152, (64, 1000) 462 / 256
+// so: from the third chunk on, and for the smallest states (N P R < 256, whose tiles here are
+// mostly padding) from the ninth.
+constexpr size_t kStagedBf16Cap = (size_t)4 << 30;
+
+static int staged_bf16_min_chunks(const m3_layer_desc& d) {
+    return d.d_state * d.headdim * d.mimo_rank >= 256 ? 2 : 8;
+}
+
+static int staged_bf16_rows(const m3_layer_desc& d, size_t cap) {
+    m3_layer_desc one = d;
+    one.batch = 1;
+    if (lp::plan(one).total > cap) return 0;
+    int rows = d.batch;
+    for (;;) {  // the plan grows with the rows, up to each part's alignment
+        one.batch = rows;
+        const size_t need = lp::plan(one).total;
+        if (need <= cap) return rows;
+        rows = std::max(1, std::min(rows - 1, (int)((double)rows * cap / need)));
+    }
+}
+
+size_t staged_bf16_workspace(const m3_layer_desc& d, size_t limit) {
+    if (d.dtype != M3_DTYPE_BF16 || (d.flags & M3_FLAG_NO_F16_OPERANDS) || !staged_shape_ok(d)) return 0;
+    if (d.seqlen <= (int64_t)staged_bf16_min_chunks(d) * generic_prefill_chunk(d)) return 0;
+    const int rows = staged_bf16_rows(d, std::min(limit, kStagedBf16Cap));
+    if (rows == 0) return 0;
+    m3_layer_desc part = d;
+    part.batch = rows;
+    return lp::plan(part).total;
+}
+
+template <typename T>
+static int launch_staged(const m3_layer_desc& d, const m3_layer_params& p, const T* proj,
+                         const float* dt_scale, T* y_out, float* h_final, float* angle,
+                         float* prev_bx, void* workspace, hipStream_t stream) {
     using namespace lp;
     const Plan pl = plan(d);
     char* ws = reinterpret_cast<char*>(workspace);
@@ -370,35 +430,62 @@ int launch_fp32_layer(const m3_layer_desc& d, const m3_layer_params& p, const vo
     a.R = d.mimo_rank, a.G = d.ngroups, a.trap = d.use_trapezoidal, a.cplx = d.use_complex;
     a.rs = d.proj_row_stride, a.pl = proj_layout(d), a.eps = d.rms_eps, a.prm = p;
     a.HT = prep_heads_per_tile(d);
-    a.proj = reinterpret_cast<const float*>(proj);
+    a.proj = proj;
     a.dt_scale = dt_scale;
     a.dt = part(0), a.A = part(1), a.phi = part(2), a.xg = part(3);
     a.xb = a.trap ? part(4) : nullptr;
     a.xr = part(5), a.Bt = part(6), a.Bb = a.trap ? part(7) : nullptr, a.Ct = part(8);
     a.ys = part(9), a.phi_sum = part(10);
-    a.y = reinterpret_cast<float*>(y_out), a.h_final = h_final, a.angle = angle;
+    a.y = y_out, a.h_final = h_final, a.angle = angle;
     a.prev_bx = prev_bx;
     const size_t lds = prep_lds(d);
     if (a.HT <= 0 || lds > kPrepLds) return 1;
     const int64_t nbth = (int64_t)d.batch * d.seqlen * d.nheads;
-    hipLaunchKernelGGL(lp_dt, dim3((unsigned)((std::max<int64_t>(nbth, d.nheads) + NTH - 1) / NTH)),
+    hipLaunchKernelGGL(lp_dt<T>, dim3((unsigned)((std::max<int64_t>(nbth, d.nheads) + NTH - 1) / NTH)),
                        dim3(NTH), 0, stream, a);
     if (a.cplx) {
         const int64_t na = (int64_t)d.batch * ((d.seqlen + kAC - 1) / kAC) * d.nheads * (d.d_state / 2);
         const unsigned ga = (unsigned)((na + NTH - 1) / NTH);
-        hipLaunchKernelGGL(lp_angle_sums, dim3(ga), dim3(NTH), 0, stream, a);
-        hipLaunchKernelGGL(lp_angles, dim3(ga), dim3(NTH), 0, stream, a);
+        hipLaunchKernelGGL(lp_angle_sums<T>, dim3(ga), dim3(NTH), 0, stream, a);
+        hipLaunchKernelGGL(lp_angles<T>, dim3(ga), dim3(NTH), 0, stream, a);
     }
-    hipLaunchKernelGGL(lp_prep, dim3(d.batch * d.seqlen), dim3(NTH), lds, stream, a);
+    hipLaunchKernelGGL(lp_prep<T>, dim3(d.batch * d.seqlen), dim3(NTH), lds, stream, a);
     if (launch_chunked_fwd_mfma(a.B, a.T, a.H, a.P, a.N, a.R, a.xg, a.xb, a.Bt, a.Bb, a.Ct, a.dt,
                                 a.A, p.D, a.xr, nullptr, a.ys, h_final, ws + pl.chunk_off,
                                 stream) != 0)
         return 1;
     const int64_t n = (int64_t)d.batch * d.seqlen * d.nheads * d.headdim;
     const unsigned grid = (unsigned)std::min<int64_t>((n + NTH - 1) / NTH, 65536);
-    hipLaunchKernelGGL(lp_gate, dim3(grid), dim3(NTH), 0, stream, a);
+    hipLaunchKernelGGL(lp_gate<T>, dim3(grid), dim3(NTH), 0, stream, a);
     if (angle || prev_bx) hipLaunchKernelGGL(lp_state, dim3(d.batch * d.nheads), dim3(NTH), 0, stream, a);
     return hipGetLastError() == hipSuccess ? 0 : 1;
+}
+
+int launch_fp32_layer(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
+                      const float* dt_scale, void* y_out, float* h_final, float* angle,
+                      float* prev_bx, void* workspace, hipStream_t stream) {
+    return launch_staged(d, p, reinterpret_cast<const float*>(proj), dt_scale,
+                         reinterpret_cast<float*>(y_out), h_final, angle, prev_bx, workspace, stream);
+}
+
+int launch_staged_bf16(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
+                       const float* dt_scale, void* y_out, float* h_final, float* angle,
+                       float* prev_bx, void* workspace, size_t limit, hipStream_t stream) {
+    const int rows = staged_bf16_rows(d, std::min(limit, kStagedBf16Cap));
+    if (rows <= 0) return 1;
+    const int64_t T = d.seqlen, H = d.nheads;
+    for (int b = 0; b < d.batch; b += rows) {
+        m3_layer_desc part = d;
+        part.batch = std::min(rows, d.batch - b);
+        auto at = [&](float* q, int64_t per_row) { return q ? q + b * per_row : nullptr; };
+        if (launch_staged(part, p, reinterpret_cast<const bf16*>(proj) + b * T * d.proj_row_stride,
+                          dt_scale ? dt_scale + b * T * H : nullptr,
+                          reinterpret_cast<bf16*>(y_out) + b * T * H * d.headdim,
+                          at(h_final, H * d.headdim * d.d_state), at(angle, H * (d.d_state / 2)),
+                          at(prev_bx, H * d.headdim * d.d_state), workspace, stream) != 0)
+            return 1;
+    }
+    return 0;
 }
 
 }  // namespace m3

@@ -396,18 +396,21 @@ __global__ __launch_bounds__(64) void bwd_cum(Args a) {
 // ---- K2: chunk-local states (scan input) and the y_inter gradient of each chunk state:
 //   hext[k][p,n] = sum_{s,j} exp(c_end - c_s) Xf[s,p,j] Bf[s,n,j]
 //   gext[k][p,n] = sum_{t,r} exp(c_t) dy[t,p,r] C[t,n,r]
-// plus the extra chunk K: hext = 0, gext = dL/dh_final (or 0). Tiles of 64 p x 128 n.
-template <int R, bool BETA, bool PADR>
+// plus the extra chunk K: hext = 0, gext = dL/dh_final (or 0). Tiles of 64 p x TN n: 128
+// columns, or 64 / 32 where d_state has no more: the wide tile then spent its loads and
+// registers on columns that do not exist (d_state 16, headdim 16, (16, 500) with 8 heads: 78 us
+// with 128 columns, 34 with 32).
+template <int R, bool BETA, bool PADR, int TN>
 __global__ __launch_bounds__(NTH) void bwd_states(Args a) {
     BW_CONSTS
-    __shared__ Lds<TW> l;
+    __shared__ Lds<TN> l;
     __shared__ float cs[64], wx[64], ec[64];
     const Shape& s = a.s;
     int ch, tile;
     if (!chunk_tile(s.B * s.K * s.H, s.nPt * s.nNt, ch, tile)) return;
     const int h = ch % s.H, k = (ch / s.H) % s.K, b = ch / (s.H * s.K);
     const int pt = tile / s.nNt, nt = tile % s.nNt;
-    const int p0 = pt * TT, n0 = nt * TW;
+    const int p0 = pt * TT, n0 = nt * TN;
     const Chunk<R, BETA, PADR> q{&a, b, k, h};
     if (threadIdx.x < QB) cs[threadIdx.x] = a.cum[(int64_t)ch * QB + threadIdx.x];
     __syncthreads();
@@ -418,12 +421,12 @@ __global__ __launch_bounds__(NTH) void bwd_states(Args a) {
     }
     __syncthreads();
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    constexpr int NJ = TW / 16;
+    constexpr int NJ = TN / 16;
     f32x4 acc[NJ];
     const int pmax = s.P - 1, nmax = s.N - 1;
     if (!a.have_hs) {
     zero(acc);
-    gemm_acc<TW, false, false>(acc, QB * R2,
+    gemm_acc<TN, false, false>(acc, QB * R2,
                  [&](int mm, int j) { return q.lx(j / R2, min(p0 + mm, pmax), j % R2); },
                  [&](int mm, int j, float v) {
                      const int t = j / R2;
@@ -444,7 +447,7 @@ __global__ __launch_bounds__(NTH) void bwd_states(Args a) {
     }
     if (!a.fwd) {
     zero(acc);
-    gemm_acc<TW, false, false>(acc, QB * R,
+    gemm_acc<TN, false, false>(acc, QB * R,
                  [&](int mm, int j) { return q.ldy(j / R, min(p0 + mm, pmax), j % R); },
                  [&](int mm, int j, float v) {
                      const int t = j / R;
@@ -1236,17 +1239,19 @@ __global__ __launch_bounds__(NTH) void bwd_reduce(Args a) {
 
 // ---- forward output: y rows (t,r) x columns p of the chunk,
 //   y = (W o G) Xf + exp(c_t) C H_k^T + D x_raw   (M = W o G from bwd_scores in forward mode)
-template <int R, bool BETA, bool PADR>
+// Tiles of 64 rows x TN columns: 64, or 32 / 16 where headdim has no more (d_state 16,
+// headdim 16, (16, 500) with 8 heads: 47 us with 64 columns, 21 with 16).
+template <int R, bool BETA, bool PADR, int TN>
 __global__ __launch_bounds__(NTH, 4) void fwd_out(Args a) {
     BW_CONSTS
-    __shared__ Lds<TT> l;
+    __shared__ Lds<TN> l;
     __shared__ float cs[64], dts[64];
     const Shape& s = a.s;
     int ch, tile;
     if (!chunk_tile(s.B * s.K * s.H, QR / TT * s.nPt, ch, tile)) return;
     const int h = ch % s.H, k = (ch / s.H) % s.K, b = ch / (s.H * s.K);
     const int rt = tile / s.nPt, pt = tile % s.nPt;
-    const int m0 = rt * TT, p0 = pt * TT;
+    const int m0 = rt * TT, p0 = pt * TN;
     const Chunk<R, BETA, PADR> q{&a, b, k, h};
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
     if (tid < QB) {
@@ -1255,18 +1260,19 @@ __global__ __launch_bounds__(NTH, 4) void fwd_out(Args a) {
     }
     __syncthreads();
     const float* Hk = a.Hs + chx(s, b, k, h) * s.PN;
-    f32x4 acc[4];
+    constexpr int NJ = TN / 16;
+    f32x4 acc[NJ];
     zero(acc);
     const int pmax = s.P - 1;
     // x_raw of this thread's outputs, read in one batch ahead of the contractions
-    float xrv[4][4];
+    float xrv[4][NJ];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int m = m0 + 4 * ty + i;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) xrv[i][j] = q.lxr(m / R, min(p0 + tcol(tx, j), pmax), m % R);
+        for (int j = 0; j < NJ; ++j) xrv[i][j] = q.lxr(m / R, min(p0 + tcol(tx, j), pmax), m % R);
     }
-    gemm_acc<TT, true, true>(acc, s.N,
+    gemm_acc<TN, true, true>(acc, s.N,
                              [&](int mm, int n) { const int m = m0 + mm; return q.lc(m / R, n, m % R); },
                              [&](int mm, int n, float v) { const int m = m0 + mm; return q.ok(m / R, m % R) ? v : 0.f; },
                              [&](int n, int pp) { return Hk[min(p0 + pp, pmax) * s.N + n]; },
@@ -1276,10 +1282,10 @@ __global__ __launch_bounds__(NTH, 4) void fwd_out(Args a) {
     for (int i = 0; i < 4; ++i) {
         const float e = __expf(cs[(m0 + 4 * ty + i) / R]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j][i] *= e;
+        for (int j = 0; j < NJ; ++j) acc[j][i] *= e;
     }
     const float* Mi = a.M + (int64_t)ch * QR * QR2;
-    gemm_acc<TT, true, false>(acc, QR2,
+    gemm_acc<TN, true, false>(acc, QR2,
                               [&](int mm, int jc) { return Mi[(m0 + mm) * QR2 + jc]; },
                               [&](int mm, int jc, float v) { return v; },
                               [&](int jc, int pp) { return q.lx(jc / R2, min(p0 + pp, pmax), jc % R2); },
@@ -1296,7 +1302,7 @@ __global__ __launch_bounds__(NTH, 4) void fwd_out(Args a) {
         if (!q.real(t) || !q.has(r)) continue;
         const int64_t base = row(s, b, k * QB + t, h) * s.P * q.rk() + r;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < NJ; ++j) {
             const int p = p0 + tcol(tx, j);
             if (p < s.P) a.y[base + (int64_t)p * q.rk()] = acc[j][i] + Dh * xrv[i][j];
         }
@@ -1367,13 +1373,22 @@ Plan make_plan(const Shape& s, bool hs_given) {
 }
 
 template <int R, bool BETA, bool PADR>
+void launch_states(const Args& a, unsigned nch, hipStream_t stream) {
+    const Shape& s = a.s;
+    const dim3 grid(tile_grid(nch, s.nPt * s.nNt));
+    if (s.N <= 32) hipLaunchKernelGGL((bwd_states<R, BETA, PADR, 32>), grid, dim3(NTH), 0, stream, a);
+    else if (s.N <= 64) hipLaunchKernelGGL((bwd_states<R, BETA, PADR, 64>), grid, dim3(NTH), 0, stream, a);
+    else hipLaunchKernelGGL((bwd_states<R, BETA, PADR, TW>), grid, dim3(NTH), 0, stream, a);
+}
+
+template <int R, bool BETA, bool PADR>
 int launch(const Args& a, const float* h_init, float* dh_init, float* scan_ws, hipStream_t stream) {
     BW_CONSTS
     const Shape& s = a.s;
     const unsigned nch = (unsigned)((int64_t)s.B * s.K * s.H);
     constexpr int nRt = QR / TT, nRt2 = QR2 / TT;
     hipLaunchKernelGGL((bwd_cum<R, BETA, PADR>), dim3(nch), dim3(64), 0, stream, a);
-    hipLaunchKernelGGL((bwd_states<R, BETA, PADR>), dim3(tile_grid(nch, s.nPt * s.nNt)), dim3(NTH), 0, stream, a);
+    launch_states<R, BETA, PADR>(a, nch, stream);
     if (!a.have_hs &&
         launch_scan_fwd(a.dec, a.hext, h_init, a.Hs, s.B, s.K + 1, s.H, s.PN, stream) != 0)
         return 1;
@@ -1416,10 +1431,13 @@ int launch_fwd(const Args& a, const float* h_init, hipStream_t stream) {
     const unsigned nch = (unsigned)((int64_t)s.B * s.K * s.H);
     constexpr int nRt = QR / TT;
     hipLaunchKernelGGL((bwd_cum<R, BETA, PADR>), dim3(nch), dim3(64), 0, stream, a);
-    hipLaunchKernelGGL((bwd_states<R, BETA, PADR>), dim3(tile_grid(nch, s.nPt * s.nNt)), dim3(NTH), 0, stream, a);
+    launch_states<R, BETA, PADR>(a, nch, stream);
     if (launch_scan_fwd(a.dec, a.hext, h_init, a.Hs, s.B, s.K + 1, s.H, s.PN, stream) != 0) return 1;
     hipLaunchKernelGGL((bwd_scores<R, BETA, PADR>), dim3(nch), dim3(NTH), 0, stream, a);
-    hipLaunchKernelGGL((fwd_out<R, BETA, PADR>), dim3(tile_grid(nch, nRt * s.nPt)), dim3(NTH), 0, stream, a);
+    const dim3 og(tile_grid(nch, nRt * s.nPt));
+    if (s.P <= 16) hipLaunchKernelGGL((fwd_out<R, BETA, PADR, 16>), og, dim3(NTH), 0, stream, a);
+    else if (s.P <= 32) hipLaunchKernelGGL((fwd_out<R, BETA, PADR, 32>), og, dim3(NTH), 0, stream, a);
+    else hipLaunchKernelGGL((fwd_out<R, BETA, PADR, TT>), og, dim3(NTH), 0, stream, a);
     if (a.hfin) hipLaunchKernelGGL(fwd_final, dim3(s.B * s.H), dim3(NTH), 0, stream, a);
     return hipGetLastError() == hipSuccess ? 0 : 1;
 }

@@ -882,3 +882,47 @@ def test_prefill_of_a_strided_batch_view_equals_its_contiguous_copy(cuda_device)
     assert torch.equal(y1, y2)
     for k in ("h", "prev_BX", "angle"):
         assert torch.equal(s1[k], s2[k]), k
+
+
+@pytest.mark.parametrize("kw,B,T", [
+    (dict(d_model=64, d_state=16, headdim=16, mimo_rank=2), 3, 129),   # its third 64-token chunk's first token
+    (dict(d_model=64, d_state=16, headdim=16, mimo_rank=4, ngroups=2), 5, 200),
+    (dict(d_model=64, d_state=18, headdim=32, mimo_rank=3, use_trapezoidal=False), 2, 150),
+    (dict(d_model=48, d_state=70, headdim=24, mimo_rank=5, use_complex_ssm=False), 3, 131),
+    (dict(d_model=32, d_state=8, headdim=16, mimo_rank=1, expand=1), 2, 513),  # smallest states: ninth chunk
+])
+def test_bf16_staged_prefill_equals_generic_kernel(kw, B, T, cuda_device):
+    """bf16 layers outside the bf16 MFMA kernels on the fp32 layer path against the generic
+    kernel (a call without workspace), proj at an odd row stride, with dt_scale; and in
+    one-row slices (a workspace that holds no more), bit for bit. Both compute in fp32: states
+    within 1e-5 (fp32 sums of T terms), y within one bf16 ulp (2^-7) of its largest entry."""
+    dev = cuda_device
+    torch.manual_seed(21)
+    layer = mamba3_amd.KulaMamba(**kw).to(dev, torch.bfloat16).eval()
+    with torch.no_grad():
+        proj = layer.in_proj(torch.randn(B, T, kw["d_model"], device=dev, dtype=torch.bfloat16))
+    src = torch.zeros(B, T, proj.shape[-1] + 1, device=dev, dtype=torch.bfloat16)
+    src[..., :-1] = proj
+    ds = torch.rand(B, T, layer.nheads, device=dev) + 0.5
+    desc = layer._desc(B, T, src)
+    assert _native.prefill_kernel_name(desc, src) == "fp32_layer"
+    full = _native.prefill_workspace_bytes(desc)
+    one = layer._desc(1, T, src)
+    row = _native.prefill_workspace_bytes(one)
+    assert 0 < row < full
+
+    def call(nbytes):
+        outs = (torch.empty(B, T, layer.d_inner, device=dev, dtype=torch.bfloat16),
+                *(torch.empty(B, layer.nheads, *s, device=dev) for s in
+                  ((layer.headdim, layer.d_state), (layer.d_state // 2,),
+                   (layer.headdim, layer.d_state))))
+        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8) if nbytes else None
+        _native.prefill_fwd(desc, layer._param_pack(), src, ds, *outs, ws, nbytes)
+        return outs
+
+    staged, sliced, generic = call(full), call(row), call(0)
+    for a, b in zip(staged, sliced):
+        assert torch.equal(a, b)
+    assert max_rel(staged[0].float(), generic[0].float()) < 2.0 ** -7
+    for name, a, b in zip(("h", "angle", "prev_BX"), staged[1:], generic[1:]):
+        assert max_rel(a, b) < 1e-5, name
