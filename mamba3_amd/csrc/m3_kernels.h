@@ -70,11 +70,13 @@ int launch_mfma_prefill(const m3_layer_desc& d, const m3_layer_params& p, const 
                         float* prev_bx, void* workspace, hipStream_t stream);
 
 // bf16 MFMA fused prefill for d_state 64/128/256, mimo_rank 1/2/4, headdim % 32 == 0.
+// Workspace within `limit` bytes where the segments' states fit it, else that of one walk per
+// (batch, head); the launcher takes the same limit.
 bool wide_prefill_supported(const m3_layer_desc& d);
-size_t wide_prefill_workspace(const m3_layer_desc& d);
+size_t wide_prefill_workspace(const m3_layer_desc& d, size_t limit);
 int launch_wide_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                         const float* dt_scale, void* y_out, float* h_final, float* angle,
-                        float* prev_bx, void* workspace, hipStream_t stream);
+                        float* prev_bx, void* workspace, size_t limit, hipStream_t stream);
 
 // Backward of the chunked SSD (fp32): shape support, workspace bytes and launcher.
 bool chunked_bwd_shape_ok(int B, int T, int H, int P, int N, int R, bool beta);

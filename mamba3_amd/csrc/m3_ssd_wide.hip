@@ -5,36 +5,58 @@
 //
 // Same algorithm as the other prefill kernels: the quadratic form inside a chunk and the
 // state carried across chunks (mamba3/ssd.py:118-244), with the layer's preparation fused
-// (mamba3/mamba3.py:197-256). It is organised for shapes whose (batch, head) pairs alone
-// do not fill the GPU:
-//   * a workgroup owns (batch, head, 32 headdim columns), so B*H*P/32 workgroups share
-//     the work (256 for the d_model 2048 layer at batch 2); the scores and the RoPE
-//     rotation are recomputed by each column block;
-//   * a chunk has 64 (t, r) rows, i.e. Q = 64 / R tokens;
-//   * sixteen waves (four per SIMD) share both phases of a chunk: contract (waves 0-7 the
-//     inter-chunk output of their tile, waves 8-15 the score tiles, all the state update;
-//     two score waves compute the next chunk's token scalars and RoPE angles instead of a
-//     tile, and output waves 0-1 take their tiles), then output (waves 0-7 the intra-chunk
-//     output, gate and store; all the next chunk's B~ / C~ tiles, the score waves its X
-//     rows).
+// (mamba3/mamba3.py:197-256).
+//
+// Work decomposition. A workgroup owns (batch, head, PC = 32 NCG headdim columns, segment of
+// the sequence) and walks its chunks of 64 (t, r) rows, Q = 64 / R tokens. PC is the whole
+// headdim (128 or 64) where enough workgroups remain, so the RoPE rotation and the scores,
+// which every column block of a head repeats, are done once per head. Shapes whose (batch,
+// head) pairs do not fill the GPU are cut along the sequence (make_plan): a state-only pass
+// walks every segment but the last from a zero state in its own RoPE frame and leaves its end
+// state, log-decay and angle increment, and seg_combine turns those into the state entering
+// each segment.
+//
+// Roles. Column waves 2c and 2c + 1 own the 32 columns of group c: each keeps half of the
+// state rows, H^T [n][p], in MFMA accumulators (N/32 x 2 tiles), contracts that half for all
+// 64 output rows, swaps the partial sums of half the rows with the other wave through LDS and
+// finishes its own rows. Helper waves (8; 4 for d_state 64) compute the scores and prepare the
+// next chunk's operand tiles. Sixteen waves, four per SIMD: one wave alone issues a VALU
+// instruction only every ~9 cycles, so eight waves of 256 registers (whole state rows per
+// wave, no swap) left the VALU and the matrix cores idle (2.6 ms against 2.2 for both passes
+// of the (2, 16384) d_model 2048 call).
+//
+// Bound: VALU issue and LDS bandwidth together. Per chunk of that call 10.5K cycles, in which
+// the SIMDs issue 5.7K cycles of VALU and 2.6K of MFMA and the LDS is busy 6.5K. The call (both
+// passes, seg_combine and the B / C normalisation) takes 2.30 ms, 0.29 of the bf16 MFMA peak;
+// in blocks of 32 columns without segments (256 workgroups, every block repeating the rotation
+// and the scores) it took 2.84 ms.
 //
 // Per chunk, in LDS (f16 unless noted):
 //   C [(t,r)][n], B [(u,r')][n]       C~ / B~: normalised B^ / C^ (bc_norm_wide) rotated
 //                                     by the RoPE angle; row (t,r) = t*R + r
 //   XT [p][(u,r')], XwT [p][(u,r')]   x * mimo_x, and the same times the chunk weight w_u
 //   S [(t,r)][(u,r')]                 masked scores (fp32 accumulated)
-//   H [p][n]                          copy of the incoming state times kHScale
-//   tok, phi (fp32)                   token scalars and RoPE angles of the chunk
-// The fp32 state H^T lives in MFMA accumulators (wave w owns N/64 tiles of 16 x 16).
+//   tok, part (fp32)                  token scalars; sums of dt theta of token groups
 // Contractions (v_mfma_f32_16x16x32_f16, fp32 accumulation):
+//   G3  Y   = diag(e^{c_t}) C~ H^T    H^T straight from the accumulators: contraction slot
+//             (g, j) of lane group g is n = 4g + j of one 16-row tile for j < 4 and of the
+//             next for j >= 4, which are the rows the lane's accumulators hold, so the state
+//             is converted to f16 in registers and never goes through LDS
 //   G4  H^T = e^{c_end} H^T + B~^T Xw    (A operand by LDS transpose reads of B~)
-//   G3  Y   = diag(e^{c_t}) C~ H^T
 //   G1  S^T = B~ C~^T per causal 16x16 tile, masked by
 //             Lc[t][u] = [u<=t] e^{c_t - c_u} (a_u + [u<t] b_u), plus D on the diagonal
 //   G2  Y  += S X
 // Output: out[t][p] = sum_r mimo_down[p,r] silu(z[t,p] mimo_z[p,r]) Y[(t,r)][p]
 // (mamba3/mamba3.py:233-238). The trapezoid is folded into a_u = lambda_u dt_u and
 // b_u = (1 - lambda_{u+1}) dt_{u+1}, as in the other kernels.
+//
+// Two phases per chunk k, a barrier after each:
+//   contract  column waves G3, G4; helpers G1, chunk k+1's rotation and X rows in registers,
+//             chunk k+2's token scalars
+//   output    column waves G2, gate, store; helpers write chunk k+1's tiles, form chunk k+2's
+//             angle sums and issue its reads
+#include <algorithm>
+
 #include "m3_common.h"
 #include "m3_kernels.h"
 #include "m3_mfma.h"
@@ -42,20 +64,15 @@
 namespace m3 {
 namespace wd {
 
-constexpr int ROWS = 64;              // (t, r) rows per chunk
-constexpr int PB = 32;                // headdim columns per workgroup
-constexpr int THREADS = 1024;         // 16 waves: 0-7 own output tiles, 8-15 score tiles
-constexpr int PAD = 8;                // f16 row padding of the S and H tiles
-// f16 row padding of the X^T / Xw^T tiles: a row stride of 40 32-bit words (their G2 / G4
-// operand reads, 16 rows x 64 bytes per wave, run 1.4-1.8% faster over the whole call than
-// at 36; 44, 48 and 52 were no better). The 256 x 1 instantiation has no LDS to spare.
-template <int N, int R>
-constexpr int padx() { return (N == 256 && R == 1) ? 8 : 16; }
+constexpr int ROWS = 64;   // (t, r) rows per chunk
+constexpr int PW = 32;     // headdim columns per column group (two waves)
+constexpr int PADS = 8;    // f16 row padding of the S tile
+// f16 row padding of the X^T / Xw^T tiles: a row stride of 36 32-bit words.
+constexpr int PADX = 8;
 // f16 row padding of the C~ / B~ tiles: a row stride of 8 (mod 16) 32-bit words keeps the
-// operand and transpose reads of those tiles free of most bank conflicts (a stride of
-// 4 (mod 16) words, padding 8, measured 5% slower at d_state 256).
+// operand and transpose reads of those tiles free of most bank conflicts.
 constexpr int PADCB = 16;
-constexpr float kHScale = 1.f / 256.f;  // the f16 state copy holds h * kHScale
+constexpr float kHScale = 1.f / 256.f;  // the f16 state operand holds h * kHScale
 
 struct Tok {
     float c2[ROWS];  // inclusive prefix of A dt over the chunk, log2 units
@@ -63,28 +80,43 @@ struct Tok {
     float bv[ROWS];  // b_u = (1 - lambda_{u+1}) dt_{u+1}
     float ec[ROWS];  // exp2(c2_t) / kHScale: inter-chunk output scale
     float w[ROWS];   // exp2(c2_end - c2_u) (a_u + b_u): chunk-state weight
+    float dt[ROWS];  // dt_t
     float dec;       // exp2(c2_end): chunk decay of the state
 };
 
-// The R ranks of one token's X row, stored together.
-template <int R>
-struct __align__(2 * R) XRow {
-    f16 v[R];
+// Column groups per workgroup: headdim in blocks of 128, 64 or 32 columns (128 columns of
+// d_state 256 at rank 1, whose helper threads each prepare 16 tokens, would spill).
+template <int N, int R>
+constexpr int kMaxGroups = N == 256 && R == 1 ? 2 : 4;
+inline int column_groups(int P, int N, int R) {
+    const int most = N == 256 && R == 1 ? 2 : 4;
+    return std::min(most, P % 128 == 0 ? 4 : P % 64 == 0 ? 2 : 1);
+}
+
+// Helper thread layout: N/4 lanes (one 4-column group, two RoPE pairs, each) share a token
+// group; GR groups of TPT tokens cover the chunk.
+template <int N, int R>
+struct Layout {
+    static constexpr int HELPERS = N == 64 ? 4 : 8;  // helper waves
+    static constexpr int Q = ROWS / R;               // tokens per chunk
+    static constexpr int LPT = N / 4;                // lanes per token group
+    static constexpr int GR = 64 * HELPERS / LPT;
+    static constexpr int TPT = Q / GR;
+    static_assert(TPT >= 1 && TPT * GR == Q, "token groups cover the chunk");
 };
 
-template <int N, int R>
+template <int N, int R, int NCG, bool FULL>
 struct __align__(16) Smem {
-    static constexpr int Q = ROWS / R;
-    f16 C[ROWS][N + PADCB];
+    static constexpr int PC = PW * NCG;
     f16 B[ROWS][N + PADCB];
-    f16 XT[2][PB][ROWS + padx<N, R>()];  // by chunk parity: G2 of chunk k reads while chunk k+1's is written
-    f16 XwT[PB][ROWS + padx<N, R>()];
-    f16 S[ROWS][ROWS + PAD];
-    f16 H[PB][N + PAD];
-    Tok tok[2];           // by chunk parity
-    alignas(16) float phi[Q][N / 2];  // RoPE angle of each (token, pair) of the chunk being prepared
-    u32x4 th[Q][N / 16];  // theta of that chunk, bf16, 8 pairs per entry
-    float mz[PB][R], md[PB][R], mx[PB][R];  // mimo_z, mimo_down * sB sC sX, mimo_x / sX of the block's columns
+    f16 C[FULL ? ROWS : 1][N + PADCB];
+    f16 XT[FULL ? PC : 1][ROWS + PADX];
+    f16 XwT[PC][ROWS + PADX];
+    f16 S[FULL ? ROWS : 1][ROWS + PADS];
+    f32x4 ex[FULL ? NCG : 1][2][2][2][64];  // partial outputs for the group's other wave: [from][row tile % 2][p tile]
+    Tok tok[3];                             // by chunk mod 3
+    alignas(16) float part[Layout<N, R>::GR][N / 2];     // sum of dt theta per token group
+    alignas(16) float gate[FULL ? PC : 1][2][R];         // mimo_z, mimo_down * sB sC sX of the columns
     F16Scales scl;                          // operand scales of the (group, head)
 };
 
@@ -102,7 +134,19 @@ struct Args {
     float* h_final;
     float* angle;
     float* prev_bx;
+    // segments of the sequence (segs = 1: none); per segment but the last and pair, the state
+    // pass's end state, which seg_combine turns into the state entering the next segment
+    int segs, seg0;
+    f32x4* hseg;  // [seg][pair block][column group][n half][tile][lane]
+    float* lseg;  // log2 of the segment's decay, [seg][b h]
+    float* aseg;  // its RoPE angle increment, [seg][b h][pair]
 };
+
+// First token of segment i: four segments each of seg0, 2 seg0 and 4 seg0 tokens, then 16 seg0.
+__host__ __device__ inline int64_t seg_start(int i, int seg0) {
+    const int u = i <= 4 ? i : i <= 8 ? 4 + 2 * (i - 4) : i <= 12 ? 12 + 4 * (i - 8) : 28 + 16 * (i - 12);
+    return (int64_t)u * seg0;
+}
 
 // Keeps the LDS reads issued above ahead of the LDS writes that follow.
 #define M3_LDS_ORDER() asm volatile("" ::: "memory")
@@ -268,20 +312,6 @@ __global__ __launch_bounds__(256) void bc_norm_wide(const bf16* __restrict__ pro
     }
 }
 
-// R consecutive 32-bit words (one RoPE pair, all ranks).
-template <int R>
-__device__ __forceinline__ void load_pair_words(const f16* p, unsigned (&w)[R]) {
-    if constexpr (R == 4) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-        w[0] = v[0]; w[1] = v[1]; w[2] = v[2]; w[3] = v[3];
-    } else if constexpr (R == 2) {
-        const u32x2 v = *reinterpret_cast<const u32x2*>(p);
-        w[0] = v[0]; w[1] = v[1];
-    } else {
-        w[0] = *reinterpret_cast<const unsigned*>(p);
-    }
-}
-
 // (e, o) rotated by the angle whose (cos, sin) is kA: (e cos - o sin, e sin + o cos).
 __device__ __forceinline__ unsigned rotate_pair(unsigned word, f16x2 kA, f16x2 kS) {
     const f16x2 v = as_f16x2(word);
@@ -289,166 +319,141 @@ __device__ __forceinline__ unsigned rotate_pair(unsigned word, f16x2 kA, f16x2 k
     return bits(f16x2{v[0], v[0]} * kA + f16x2{-u[0], u[1]});
 }
 
-// 8 consecutive bf16 (raw bits): one 128-bit load when the address is 16-byte aligned.
-__device__ __forceinline__ u32x4 load8(const bf16* p, bool vec) {
-    if (vec) return *reinterpret_cast<const u32x4*>(p);
-    const unsigned short* q = reinterpret_cast<const unsigned short*>(p);
-    u32x4 v;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = (unsigned)q[2 * j] | ((unsigned)q[2 * j + 1] << 16);
-    return v;
-}
+__device__ __forceinline__ float bf(unsigned u) { return __builtin_bit_cast(float, u << 16); }
 
-template <int N, int R>
-__global__ __launch_bounds__(THREADS) void ssd_wide(Args a) {
-    constexpr int Q = ROWS / R;    // tokens per chunk
-    constexpr int NH = N / 2;      // RoPE pairs
+template <int N, int R, int NCG, bool FULL>
+__global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
+                             N == 256 ? (2 * NCG + Layout<N, R>::HELPERS + 3) / 4 : 4) void ssd_wide(Args a) {
+    using L = Layout<N, R>;
+    constexpr int Q = L::Q, LPT = L::LPT, GR = L::GR, TPT = L::TPT, HELPERS = L::HELPERS;
+    constexpr int CW = 2 * NCG;     // column waves
+    constexpr int NH = N / 2;       // RoPE pairs
     constexpr int NR = N * R;
-    constexpr int TPW = N >= 128 ? N / 128 : 1;  // state tiles per wave (N/8 tiles in all)
-    constexpr int KN = N / 32;     // k-steps over n
-    constexpr int TPL = 4 / R;     // tokens per lane in an output tile
-    __shared__ Smem<N, R> sm;
+    constexpr int NT = N / 32;      // state row tiles of a wave (half of n)
+    constexpr int KN = N / 32;      // k-steps over n
+    constexpr int PC = PW * NCG;
+    constexpr int HT = 64 * HELPERS;
+    constexpr int XTH = FULL ? HT : 64 * CW;  // threads with X jobs
+    constexpr int TPL = 4 / R;      // tokens per lane in an output tile
+    constexpr int XT = Q * PC / XTH; // X elements per thread: consecutive tokens of one column
+    __shared__ Smem<N, R, NCG, FULL> sm;
 
     // wave index in an SGPR, so the role branches below are scalar branches
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g16 = lane >> 4, l16 = lane & 15;
-    // Workgroups go to the 8 XCDs round-robin; renumber them so that consecutive logical
-    // workgroups -- the column blocks and heads of one batch row, which read the same
-    // normalised B^ / C^ rows -- share an XCD and its L2.
-    const int nblk = gridDim.x;
-    const int blk = (nblk % 8 == 0) ? (blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8 : blockIdx.x;
-    const int pblk = blk % a.PS;
-    const int bh = blk / a.PS;
+    const int npairs = a.B * a.H * a.PS;
+    // Workgroups go to the 8 XCDs round-robin. Segments come longest first; within a segment the
+    // (batch, head, column block) pairs are renumbered so that consecutive ones, which read the
+    // same normalised B^ / C^ rows, share an XCD and its L2.
+    const int so = blockIdx.x / npairs, j0 = blockIdx.x % npairs;
+    const int seg = (FULL ? a.segs : a.segs - 1) - 1 - so;  // the state pass leaves the last segment out
+    const int pair = (npairs % 8 == 0) ? (j0 % 8) * (npairs / 8) + j0 / 8 : j0;
+    const int pblk = pair % a.PS;
+    const int bh = pair / a.PS;
     const int b = bh / a.H, h = bh % a.H;
     const int grp = h / (a.H / a.G);
-    const int p0 = pblk * PB;
+    const int p0 = pblk * PC;
     const int T = a.T;
+    const int tbeg = (int)seg_start(seg, a.seg0);
+    const int tend = seg + 1 < a.segs ? (int)seg_start(seg + 1, a.seg0) : T;
+    const int nchunks = (tend - tbeg + Q - 1) / Q;
     const int64_t rs = a.rs;
     const bf16* proj = a.proj + (int64_t)b * T * rs;
     const int64_t nrs = (int64_t)a.G * NR;  // B^ / C^ token stride
-    const f16* Bn = a.Bn + (int64_t)b * T * nrs + (int64_t)grp * NR;
-    const f16* Cn = a.Cn + (int64_t)b * T * nrs + (int64_t)grp * NR;
-    const int nchunks = (T + Q - 1) / Q;
     const float Ah = -expf(a.prm.A_log[h]);
     const float dtb = a.prm.dt_bias[h];
     if (wave == 0) {
         const F16Scales sc = layer_f16_scales<N, R>(a.prm, grp, h, a.P, lane);
         if (lane == 0) sm.scl = sc;
     }
+    if constexpr (FULL) {
+        // G2 reads 32 score columns per step: the tiles right of the diagonal in row blocks 0
+        // and 2 stay zero.
+        if (wave < 2) *reinterpret_cast<f16x4*>(&sm.S[32 * wave + l16][32 * wave + 16 + 4 * g16]) = f16x4{0, 0, 0, 0};
+    }
     __syncthreads();
     const F16Scales scl = sm.scl.in_sgprs();
-    // the skip term D enters the masked scores, which carry 1 / (sB sC)
-    const float Dh = a.prm.D[h] * scl.inv_bc;
-    const int hp = h * a.P;  // first column of this head in x, z and y
-
-    // Waves 0-7: output tile rows 16 tt .. 16 tt + 15, columns 16 pt .. 16 pt + 15 (G3, G2,
-    // gate, store). Waves 8-15: score tiles (G1 and its mask). All waves: state tiles (G4)
-    // while there are tiles left, and the next chunk's tiles.
-    const bool out_wave = wave < 8;
-    const bool g4_wave = wave * TPW < N / 8;
-    const int tt = (wave & 7) >> 1, pt = wave & 1;
-    const int pe = p0 + 16 * pt + l16;  // this lane's output column
-    // X preparation jobs: column xp of tokens xt0 + m * (THREADS / PB) below Q, m < XJ.
-    constexpr int XJ = (Q * PB + THREADS - 1) / THREADS;
-    // (on the score waves first: the output waves also run G2, the gate and the store in
-    // the phase that prepares X)
-    const int xtid = Q * PB <= THREADS / 2 ? tid ^ (THREADS / 2) : tid;
-    const int xp = xtid % PB, xt0 = xtid / PB;
-    if (tid < PB * R) {
-        const int c = tid / R, r = tid % R;
-        const int64_t e = (int64_t)(hp + p0 + c) * R + r;
-        sm.mz[c][r] = a.prm.mimo_z[e];
-        sm.md[c][r] = a.prm.mimo_down[e] * scl.out;
-        sm.mx[c][r] = a.prm.mimo_x[e] * scl.inv_x;
+    const int hp = h * a.P + p0;  // first column of this block in x, z and y
+    if constexpr (FULL) {
+        for (int e = tid; e < PC * R; e += 64 * (CW + HELPERS)) {
+            sm.gate[e / R][0][e % R] = a.prm.mimo_z[(int64_t)hp * R + e];
+            sm.gate[e / R][1][e % R] = a.prm.mimo_down[(int64_t)hp * R + e] * scl.out;
+        }
     }
-    // theta staging jobs: units of 8 pairs of one token.
-    constexpr int THU = Q * NH / 8;
-    constexpr int THJ = (THU + THREADS - 1) / THREADS;
-    const bool thvec = a.rs % 8 == 0 && a.pl.theta % 8 == 0 &&
-                       reinterpret_cast<uintptr_t>(a.proj) % 16 == 0;
+    const int64_t sbase = (int64_t)a.B * a.H;  // (batch, head) pairs: stride of lseg / aseg
 
-    // ---- per-chunk inputs, read into registers at least a phase before they are used ----
-    // Rotation jobs: this thread's two adjacent RoPE pairs 2 ri, 2 ri + 1 at tokens
-    // rt0 + m * TSTEP (m < J), so each C~ / B~ row segment goes out as one 64-bit store.
-    constexpr int NP2 = NH / 2;
-    constexpr int J = (Q * NP2 + THREADS - 1) / THREADS;  // jobs at tokens below Q
-    constexpr int TSTEP = THREADS / NP2;
-    const int ri = tid % NP2, rt0 = tid / NP2;
-    unsigned pwb[J][2][R], pwc[J][2][R];
-    auto load_bc = [&](int kk) {
-#pragma unroll
-        for (int m = 0; m < J; ++m) {
-            const int st = kk * Q + rt0 + m * TSTEP;
-            const int64_t off = (int64_t)min(st, T - 1) * nrs + 4 * ri * R;  // in range; zeroed when used
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                load_pair_words<R>(Bn + off + 2 * e * R, pwb[m][e]);
-                load_pair_words<R>(Cn + off + 2 * e * R, pwc[m][e]);
-            }
-        }
+    // ---- jobs that either role runs
+    // Reads of one chunk go through buffer resources that start at its first token and end at
+    // the sequence's last: tokens past the end read as zero, and a lane's offset within the
+    // chunk is the same for every chunk.
+    auto chunk_rsrc = [&](const void* base, int kk, int64_t row_bytes) {
+        const int64_t s0 = tbeg + (int64_t)kk * Q;
+        return make_rsrc(reinterpret_cast<const char*>(base) + (s0 < T ? s0 * row_bytes : 0),
+                         s0 < T ? (T - s0) * row_bytes : 0);
     };
-    // x of the X job (8 columns, raw bf16) and theta of the staging jobs.
-    unsigned pxv[XJ];
-    u32x4 pth[THJ];
+    const int rb = (int)rs * 2, nb = (int)nrs * 2;  // bytes of a proj row, of a B^ / C^ token
+    // X jobs: column xp, tokens xt0 .. xt0 + XT - 1
+    const int xtid = FULL ? tid - 64 * CW : tid;  // helpers; column waves in the state pass
+    const int xp = xtid & (PC - 1), xt0 = (xtid / PC) * XT;
+    float mx[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) mx[r] = a.prm.mimo_x[(int64_t)(hp + xp) * R + r] * scl.inv_x;
+    unsigned pxv[XT];
+    const int xoff = xt0 * rb + ((int)a.pl.x + hp + xp) * 2;
     auto load_xv = [&](int kk) {
+        const __amdgpu_buffer_rsrc_t r = chunk_rsrc(proj, kk, rb);
 #pragma unroll
-        for (int m = 0; m < XJ; ++m) {
-            const int st = min(kk * Q + xt0 + m * (THREADS / PB), T - 1);
-            pxv[m] = __builtin_nontemporal_load(
-                reinterpret_cast<const unsigned short*>(proj + (int64_t)st * rs + a.pl.x + hp + p0 + xp));
-        }
+        for (int m = 0; m < XT; ++m) pxv[m] = __builtin_amdgcn_raw_buffer_load_b16(r, xoff, m * rb, kStream);
     };
-    auto load_theta = [&](int kk) {
-        if (a.cplx) {
+    // X rows (t, r) = x_t * mimo_x[p, r] (mamba3/mamba3.py:210), and times w_t, chunk kk
+    constexpr int XP = XT * R < 8 ? XT * R : 8;  // elements per stored piece
+    constexpr int XV = XT * R / XP;              // pieces per thread
+    static_assert(XT >= 1 && XV * XP == XT * R, "whole X pieces");
+    typedef f16 xpiece __attribute__((ext_vector_type(XP)));
+    xpiece xo[FULL ? XV : 1], xw[XV];
+    auto form_x = [&](int kk) {
+        const Tok& tk = sm.tok[kk % 3];
 #pragma unroll
-            for (int m = 0; m < THJ; ++m) {
-                const int u = tid + m * THREADS;
-                if (u < THU) {
-                    const int st = min(kk * Q + u / (NH / 8), T - 1);
-                    pth[m] = load8(proj + (int64_t)st * rs + a.pl.theta + 8 * (u % (NH / 8)), thvec);
-                }
+        for (int m = 0; m < XT; ++m) {
+            const float xval = bf(pxv[m]);
+            const float w = tk.w[xt0 + m];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float v = xval * mx[r];
+                if constexpr (FULL) xo[(m * R + r) / XP][(m * R + r) % XP] = (f16)v;
+                xw[(m * R + r) / XP][(m * R + r) % XP] = (f16)(v * w);
             }
         }
     };
-    auto store_theta = [&]() {
-        if (a.cplx) {
+    auto write_xw = [&]() {
 #pragma unroll
-            for (int m = 0; m < THJ; ++m) {
-                const int u = tid + m * THREADS;
-                if (u < THU) sm.th[u / (NH / 8)][u % (NH / 8)] = pth[m];
-            }
-        }
+        for (int v = 0; v < XV; ++v) *reinterpret_cast<xpiece*>(&sm.XwT[xp][xt0 * R + XP * v]) = xw[v];
     };
-    // Token scalars and RoPE angles (waves 10 .. 10+NWA-1, score waves with one tile each):
-    // lane t = token t of the chunk for the scalars, pair ai for the angles.
-    constexpr int NWA = (NH + 63) / 64;
-    constexpr int kAngleWave0 = 10;
-    const bool angle_wave = wave >= kAngleWave0 && wave < kAngleWave0 + NWA;
-    const int ai = 64 * (wave - kAngleWave0) + lane;
-    float phi_run = 0.f;
+    // token scalars: lane t = token t of the chunk (helper 3)
     unsigned rdt0 = 0, rlam0 = 0, rdt1 = 0, rlam1 = 0;
     float sc0 = 1.f, sc1 = 1.f;
     auto load_tokens = [&](int kk) {
-        if (lane > Q) return;
-        const int s0 = kk * Q;
-        const int st0 = min(s0 + lane, T - 1), st1 = min(s0 + lane + 1, T - 1);
-        const bf16* row0 = proj + (int64_t)st0 * rs;
-        const bf16* row1 = proj + (int64_t)st1 * rs;
-        rdt0 = *reinterpret_cast<const unsigned short*>(row0 + a.pl.dt + h);
-        rdt1 = *reinterpret_cast<const unsigned short*>(row1 + a.pl.dt + h);
-        rlam0 = a.trap ? *reinterpret_cast<const unsigned short*>(row0 + a.pl.lam + h) : 0u;
-        rlam1 = a.trap ? *reinterpret_cast<const unsigned short*>(row1 + a.pl.lam + h) : 0u;
-        sc0 = a.dt_scale ? a.dt_scale[((int64_t)b * T + st0) * a.H + h] : 1.f;
-        sc1 = a.dt_scale ? a.dt_scale[((int64_t)b * T + st1) * a.H + h] : 1.f;
+        const __amdgpu_buffer_rsrc_t r = chunk_rsrc(proj, kk, rb);
+        const int off = (int)opaque(lane) * rb + h * 2;
+        rdt0 = __builtin_amdgcn_raw_buffer_load_b16(r, off, (int)a.pl.dt * 2, 0);
+        rdt1 = __builtin_amdgcn_raw_buffer_load_b16(r, off + rb, (int)a.pl.dt * 2, 0);
+        if (a.trap) {
+            rlam0 = __builtin_amdgcn_raw_buffer_load_b16(r, off, (int)a.pl.lam * 2, 0);
+            rlam1 = __builtin_amdgcn_raw_buffer_load_b16(r, off + rb, (int)a.pl.lam * 2, 0);
+        }
+        if (a.dt_scale) {
+            const __amdgpu_buffer_rsrc_t rd = chunk_rsrc(a.dt_scale + (int64_t)b * T * a.H, kk, (int64_t)a.H * 4);
+            const int od = ((int)opaque(lane) * a.H + h) * 4;
+            sc0 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, od, 0, 0));
+            sc1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, od + a.H * 4, 0, 0));
+        }
     };
-    auto bf = [](unsigned u) { return __builtin_bit_cast(float, u << 16); };
-    // Token scalars of chunk kk into tok[kk & 1], its RoPE angles into phi.
     auto prep_tokens = [&](int kk) {
-        const int s0 = kk * Q;
+        const int s0 = tbeg + kk * Q;
         const int t = lane;
         const bool v0 = t < Q && s0 + t < T, v1 = t < Q && s0 + t + 1 < T;
         // mamba3/mamba3.py:200-204, 212-216
-        // computed for every lane (the clamped reads are finite), then selected
+        // computed for every lane (reads past the end are zero), then selected
         const float sp_t = fast_softplus_hw(bf(rdt0) + dtb) * sc0;
         const float sp_n = fast_softplus_hw(bf(rdt1) + dtb) * sc1;
         const float sg_t = __builtin_amdgcn_rcpf(1.f + fast_exp(-bf(rlam0)));
@@ -459,309 +464,550 @@ __global__ __launch_bounds__(THREADS) void ssd_wide(Args a) {
         const float lam_n = v1 && a.trap ? sg_n : 1.f;
         const float c2 = wave_incl_scan(Ah * dt_t * kLog2e);
         const float c2_end = readlane(c2, Q - 1);
-        if (wave == kAngleWave0 + NWA - 1) {
-            const float av = a.trap ? lam_t * dt_t : dt_t;
-            const float bv = a.trap ? (1.f - lam_n) * dt_n : 0.f;
-            Tok& tk = sm.tok[kk & 1];
-            if (t < Q) {
-                tk.c2[t] = c2;
-                tk.av[t] = av;
-                tk.bv[t] = bv;
-                tk.ec[t] = __builtin_amdgcn_exp2f(c2) * (1.f / kHScale);
-                tk.w[t] = __builtin_amdgcn_exp2f(c2_end - c2) * (av + bv);
-            }
-            if (t == 0) tk.dec = __builtin_amdgcn_exp2f(c2_end);
+        const float av = a.trap ? lam_t * dt_t : dt_t;
+        const float bv = a.trap ? (1.f - lam_n) * dt_n : 0.f;
+        Tok& tk = sm.tok[kk % 3];
+        if (t < Q) {
+            tk.dt[t] = dt_t;
+            tk.c2[t] = c2;
+            tk.av[t] = av;
+            tk.bv[t] = bv;
+            tk.ec[t] = __builtin_amdgcn_exp2f(c2) * (1.f / kHScale);
+            tk.w[t] = __builtin_amdgcn_exp2f(c2_end - c2) * (av + bv);
         }
-        if (a.cplx && ai < NH) {
-            // phi_t[i] = phi_{t-1}[i] - dt_t theta_t[i] (mamba3/mamba3.py:160-162)
-            // 16 theta reads ahead of each group's angle stores (which the reads may not be
-            // ordered after)
-            const unsigned short* thq = reinterpret_cast<const unsigned short*>(&sm.th[0][0]) + ai;
-            float ph = phi_run;
-#pragma unroll
-            for (int q0 = 0; q0 < Q; q0 += 16) {
-                unsigned thv[16];
-#pragma unroll
-                for (int j = 0; j < 16; ++j) thv[j] = thq[(q0 + j) * NH];
-                M3_LDS_ORDER();
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    ph -= readlane(dt_t, q0 + j) * bf(thv[j]);
-                    sm.phi[q0 + j][ai] = ph;
-                }
-            }
-            phi_run = ph;
-        }
-    };
-    // Tiles of chunk kk: rotated C~ / B~ rows, X rows into XT[kk & 1] and XwT.
-    auto prep_chunk = [&](int kk) {
-        const int s0 = kk * Q;
-        const Tok& tk = sm.tok[kk & 1];
-#pragma unroll
-        for (int m = 0; m < J; ++m) {
-            const int t = rt0 + m * TSTEP;
-            if (Q * NP2 % THREADS != 0 && t >= Q) break;  // threads past the chunk's jobs (small d_state)
-            // Tokens past the end get a zero factor, which zeroes their rows (the clamped
-            // words they rotate are finite).
-            const bool valid = s0 + t < T;
-            f16x2 kA[2], kS[2];
-            const f32x2 ph = a.cplx ? *reinterpret_cast<const f32x2*>(&sm.phi[t][2 * ri]) : f32x2{0.f, 0.f};
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                f16x2 k = f16x2{(f16)1.f, (f16)0.f};
-                if (a.cplx) {
-                    float sn, cs;
-                    fast_sincos(ph[e], sn, cs);
-                    k = f16x2{(f16)cs, (f16)sn};
-                }
-                kA[e] = as_f16x2(valid ? bits(k) : 0u);
-                kS[e] = __builtin_shufflevector(kA[e], kA[e], 1, 0);
-            }
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                *reinterpret_cast<u32x2*>(&sm.B[t * R + r][4 * ri]) =
-                    u32x2{rotate_pair(pwb[m][0][r], kA[0], kS[0]), rotate_pair(pwb[m][1][r], kA[1], kS[1])};
-                *reinterpret_cast<u32x2*>(&sm.C[t * R + r][4 * ri]) =
-                    u32x2{rotate_pair(pwc[m][0][r], kA[0], kS[0]), rotate_pair(pwc[m][1][r], kA[1], kS[1])};
-            }
-        }
-        // X rows (t, r) = x_t * mimo_x[p, r] (mamba3/mamba3.py:210), and times w_t.
-#pragma unroll
-        for (int m = 0; m < XJ; ++m) {
-            const int t = xt0 + m * (THREADS / PB);
-            if (t >= Q) break;
-            const float xval = s0 + t < T ? bf(pxv[m]) : 0.f;
-            const float w = tk.w[t];
-            XRow<R> xv, xw;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const float mxr = sm.mx[xp][r];
-                xv.v[r] = (f16)(xval * mxr);
-                xw.v[r] = (f16)(xval * mxr * w);
-            }
-            *reinterpret_cast<XRow<R>*>(&sm.XT[kk & 1][xp][t * R]) = xv;
-            *reinterpret_cast<XRow<R>*>(&sm.XwT[xp][t * R]) = xw;
-        }
+        if (t == 0) tk.dec = __builtin_amdgcn_exp2f(c2_end);
     };
 
-    // State tiles of this wave: j -> (n tile, p tile) = ((wave*TPW + j) / 2, (wave*TPW + j) % 2).
-    f32x4 hacc[TPW];
+    if (wave < CW) {
+        // =============================== column waves ===============================
+        const int cg = wave >> 1, nh = wave & 1;
+        const int pw = PW * cg;      // first column of the group in the block
+        const int n0 = nh * (N / 2); // first state row of the wave
+        f32x4 hacc[NT][2];
 #pragma unroll
-    for (int j = 0; j < TPW; ++j) hacc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int idx = tid; idx < PB * (N + PAD) / 2; idx += THREADS)
-        reinterpret_cast<unsigned*>(&sm.H[0][0])[idx] = 0u;
-    // Prologue: chunk 0's token scalars and tiles; chunk 1's reads and theta.
-    load_bc(0);
-    load_xv(0);
-    load_theta(0);
-    if (angle_wave) load_tokens(0);
-    store_theta();
-    __syncthreads();
-    if (angle_wave) {
-        prep_tokens(0);
-        if (nchunks > 1) load_tokens(1);
-    }
-    if (nchunks > 1) load_theta(1);
-    __syncthreads();
-    prep_chunk(0);
-    if (nchunks > 1) {
-        load_bc(1);
-        load_xv(1);
-        store_theta();
-    }
-    __syncthreads();
-
-    // Per chunk k, two phases:
-    //   contract: G4, G3, G1 of chunk k; token scalars and RoPE angles of chunk k+1
-    //   output:   G2, gate, store of chunk k, its state copy; tiles of chunk k+1
-    for (int k = 0; k < nchunks; ++k) {
-        const int s0 = k * Q;
-        const Tok& tk = sm.tok[k & 1];
-
-        // ---- contract ----
-        unsigned zr_bits[TPL];
-        if (out_wave) {
+        for (int t = 0; t < NT; ++t) hacc[t][0] = hacc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (FULL && seg > 0) {
+            // state entering the segment (seg_combine)
+            const f32x4* hs = a.hseg + (((int64_t)(seg - 1) * npairs + pair) * CW + wave) * (NT * 2 * 64) + lane;
 #pragma unroll
-            for (int q = 0; q < TPL; ++q) {
-                const int st = min(s0 + (16 * tt + 4 * g16) / R + q, T - 1);
-                zr_bits[q] = __builtin_nontemporal_load(
-                    reinterpret_cast<const unsigned short*>(proj + (int64_t)st * rs + a.pl.z + hp + pe));
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int pt = 0; pt < 2; ++pt) hacc[t][pt] = hs[(2 * t + pt) * 64];
+        }
+        float ldec = 0.f;  // log2 of the segment's decay (state pass)
+        // Prologue, beside the helpers' below: in the state pass the column waves form X.
+        if constexpr (!FULL) load_xv(0);
+        __syncthreads();  // token scalars of chunk 0 and 1
+        if constexpr (!FULL) {
+            form_x(0);
+            write_xw();
+            load_xv(1);
+        }
+        __syncthreads();  // angle sums of chunk 0
+        __syncthreads();  // angles of chunk 0
+        __syncthreads();  // tiles of chunk 0, angle sums of chunk 1
+
+        for (int k = 0; k < nchunks; ++k) {
+            const int s0 = tbeg + k * Q;
+            const Tok& tk = sm.tok[k % 3];
+            // ---- contract ----
+            const __amdgpu_buffer_rsrc_t rp = make_rsrc(proj + (int64_t)s0 * rs, (int64_t)(T - s0) * rs * 2);
+            const int zoff = ((4 * g16 / R) * (int)rs + (int)a.pl.z + hp + pw + l16) * 2;
+            // The wave's half of the contraction over n for all 64 rows; row tiles 2 nh, 2 nh + 1
+            // are its own to finish, the others' partial sums go to the group's other wave.
+            unsigned zr_bits[FULL ? 2 : 1][2][TPL];
+            f32x4 yacc[2][2];
+            if constexpr (FULL) {
+                f32x4 ysum[4][2];
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) ysum[tt][0] = ysum[tt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < KN / 2; ++s) {
+                    f16x8 Bo[2];
+#pragma unroll
+                    for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            Bo[pt][v] = (f16)(hacc[2 * s][pt][v] * kHScale);
+                            Bo[pt][4 + v] = (f16)(hacc[2 * s + 1][pt][v] * kHScale);
+                        }
+                    // row tile order: the other wave's two, then the own two; two operand rows in
+                    // flight at a time (four spill the accumulators at d_state 256)
+#pragma unroll
+                    for (int i2 = 0; i2 < 2; ++i2) {
+                        f16x8 A[2];
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+                            A[i] = *reinterpret_cast<const f16x8*>(&sm.C[16 * i + 32 * (i2 == 0 ? 1 - nh : nh) + l16][n0 + 32 * s + 8 * g16]);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i)
+#pragma unroll
+                            for (int pt = 0; pt < 2; ++pt) ysum[2 * i2 + i][pt] = mfma16(A[i], Bo[pt], ysum[2 * i2 + i][pt]);
+                        if constexpr (N == 256) M3_FENCE();
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int pt = 0; pt < 2; ++pt) {
+                        sm.ex[cg][nh][i][pt][lane] = ysum[i][pt];
+                        yacc[i][pt] = ysum[2 + i][pt];
+                    }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int q = 0; q < TPL; ++q) {
+                        const int so = ((32 * nh + 16 * i) / R + q) * (int)rs * 2;
+                        zr_bits[i][0][q] = __builtin_amdgcn_raw_buffer_load_b16(rp, zoff, so, kStream);
+                        zr_bits[i][1][q] = __builtin_amdgcn_raw_buffer_load_b16(rp, zoff + 32, so, kStream);
+                    }
             }
-        }
-        if (k + 2 < nchunks) load_theta(k + 2);
-        if (angle_wave && k + 1 < nchunks) {
-            prep_tokens(k + 1);
-            if (k + 2 < nchunks) load_tokens(k + 2);
-        }
-        if (g4_wave) {
-            const float dec = tk.dec;
+            {
+                const float dec = tk.dec;
+                if constexpr (!FULL) ldec += tk.c2[Q - 1];
+                f16x8 Xo[2][2];
 #pragma unroll
-            for (int j = 0; j < TPW; ++j) hacc[j] *= dec;
+                for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
+                    for (int pt = 0; pt < 2; ++pt)
+                        Xo[s][pt] = *reinterpret_cast<const f16x8*>(&sm.XwT[pw + 16 * pt + l16][32 * s + 8 * g16]);
 #pragma unroll
-                for (int j = 0; j < TPW; ++j) {
-                    const int jt = wave * TPW + j;
-                    const int nt = jt >> 1, ptj = jt & 1;
-                    const f16* bp = &sm.B[32 * s + 8 * g16 + (l16 >> 2)][16 * nt + 4 * (l16 & 3)];
-                    const f16x4 lo = ld_tr(bp);
-                    const f16x4 hi = ld_tr(bp + 4 * (N + PADCB));
-                    const f16x8 A = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-                    const f16x8 Bo = *reinterpret_cast<const f16x8*>(&sm.XwT[16 * ptj + l16][32 * s + 8 * g16]);
-                    hacc[j] = mfma16(A, Bo, hacc[j]);
+                for (int t = 0; t < NT; ++t) {
+                    hacc[t][0] *= dec;
+                    hacc[t][1] *= dec;
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        const f16* bp = &sm.B[32 * s + 8 * g16 + (l16 >> 2)][n0 + 32 * (t >> 1) + 4 * (t & 1) + 8 * (l16 & 3)];
+                        const f16x4 lo = ld_tr(bp);
+                        const f16x4 hi = ld_tr(bp + 4 * (N + PADCB));
+                        const f16x8 A = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                        hacc[t][0] = mfma16(A, Xo[s][0], hacc[t][0]);
+                        hacc[t][1] = mfma16(A, Xo[s][1], hacc[t][1]);
+                    }
                 }
             }
-        }
-        f32x4 yacc = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (out_wave) {
+            __syncthreads();
+            // ---- output ----
+            if constexpr (FULL) {
+                // y rows of this chunk; stores past the last token fall outside and are dropped
+                const __amdgpu_buffer_rsrc_t ry =
+                    make_rsrc(a.y_out + ((int64_t)b * T + s0) * a.H * a.P, (int64_t)(T - s0) * a.H * a.P * 2);
+                f16x8 Xo[2][2];
 #pragma unroll
-            for (int s = 0; s < KN; ++s) {
-                const f16x8 A = *reinterpret_cast<const f16x8*>(&sm.C[16 * tt + l16][32 * s + 8 * g16]);
-                const f16x8 Bo = *reinterpret_cast<const f16x8*>(&sm.H[16 * pt + l16][32 * s + 8 * g16]);
-                yacc = mfma16(A, Bo, yacc);
-            }
+                for (int s = 0; s < 2; ++s)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) yacc[v] *= tk.ec[(16 * tt + 4 * g16 + v) / R];
-        }
-
-        // Causal score tiles (ti, ui), ui <= ti, listed row by row as 0..9: waves 8..15 take
-        // tile wave-8, waves 8 and 9 also tiles 8 and 9, except the angle waves, whose tiles
-        // go to output waves 0.. (which then run a tile and G3, as much as the waves with
-        // two tiles). A lane's four u-rows 16 ui + 4 g16 + v cover NU tokens; their mask
-        // factors are read (unconditionally: every index is below Q) and formed before the
-        // contraction.
-        const int tile0 = wave >= 8 ? (angle_wave ? -1 : wave - 8) : (wave < NWA ? kAngleWave0 - 8 + wave : -1);
-        const int tile1 = wave == 8 || wave == 9 ? wave : -1;
-        for (int c = 0; c < 2; ++c) {
-            const int idx = c == 0 ? tile0 : tile1;
-            if (idx < 0) break;
-            const int ti = idx < 1 ? 0 : idx < 3 ? 1 : idx < 6 ? 2 : 3;
-            const int ui = idx - ti * (ti + 1) / 2;
-            constexpr int NU = R >= 4 ? 1 : 4 / R;
-            const unsigned trow = 16 * ti + l16, t = trow / R;
-            const unsigned ub = (unsigned)(16 * ui + 4 * g16) / R;
-            // operands one k-step ahead of the MFMA that takes them
-            const f16* pa = &sm.B[16 * ui + l16][8 * g16];
-            const f16* pb = &sm.C[16 * ti + l16][8 * g16];
-            f16x8 A = *reinterpret_cast<const f16x8*>(pa);
-            f16x8 Bo = *reinterpret_cast<const f16x8*>(pb);
-            const float ct = tk.c2[t];
-            float fu[NU];
+                    for (int pt = 0; pt < 2; ++pt)
+                        Xo[s][pt] = *reinterpret_cast<const f16x8*>(&sm.XT[pw + 16 * pt + l16][32 * s + 8 * g16]);
 #pragma unroll
-            for (int j = 0; j < NU; ++j) {
-                const unsigned u = ub + j;
-                const float e = __builtin_amdgcn_exp2f(ct - tk.c2[u]);
-                const float ab = fmaf(tk.bv[u], u < t ? 1.f : 0.f, tk.av[u]);
-                fu[j] = u <= t ? e * ab : 0.f;
-            }
-            f32x4 sacc = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int i = 0; i < 2; ++i) {
+                    const int tt = 2 * nh + i;  // scalar
 #pragma unroll
-            for (int s = 0; s < KN; ++s) {
-                f16x8 An = A, Bn = Bo;
-                if (s + 1 < KN) {
-                    An = *reinterpret_cast<const f16x8*>(pa + 32 * (s + 1));
-                    Bn = *reinterpret_cast<const f16x8*>(pb + 32 * (s + 1));
+                    for (int pt = 0; pt < 2; ++pt) yacc[i][pt] += sm.ex[cg][1 - nh][i][pt][lane];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float e = tk.ec[(16 * tt + 4 * g16 + v) / R];
+                        yacc[i][0][v] *= e;
+                        yacc[i][1][v] *= e;
+                    }
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        if (s > nh) break;  // columns past the row block
+                        const f16x8 A = *reinterpret_cast<const f16x8*>(&sm.S[16 * tt + l16][32 * s + 8 * g16]);
+                        yacc[i][0] = mfma16(A, Xo[s][0], yacc[i][0]);
+                        yacc[i][1] = mfma16(A, Xo[s][1], yacc[i][1]);
+                    }
+#pragma unroll
+                    for (int q = 0; q < TPL; ++q) {
+                        const int st = (16 * tt + 4 * g16) / R + q;  // chunk token
+#pragma unroll
+                        for (int pt = 0; pt < 2; ++pt) {
+                            const float z = bf(zr_bits[i][pt][q]);
+                            float o = 0.f;
+#pragma unroll
+                            for (int r = 0; r < R; ++r) {
+                                const float zr = z * sm.gate[pw + 16 * pt + l16][0][r];
+                                o += sm.gate[pw + 16 * pt + l16][1][r] * zr * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-zr * kLog2e)) * yacc[i][pt][q * R + r];
+                            }
+                            __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, (bf16)o), ry,
+                                                                  (st * a.H * a.P + hp + pw + 16 * pt + l16) * 2, 0, kStream);
+                        }
+                    }
                 }
-                sacc = mfma16(A, Bo, sacc);
-                A = An;
-                Bo = Bn;
             }
-            // lane: u-row 16 ui + 4 g16 + v, t-row 16 ti + l16
-            f16x4 sv;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const float val = sacc[v] * fu[v * NU / 4];
-                sv[v] = (f16)(16 * ui + 4 * g16 + v == (int)trow ? val + Dh : val);
-            }
-            *reinterpret_cast<f16x4*>(&sm.S[trow][16 * ui + 4 * g16]) = sv;
-        }
-        if (wave == 15) {
-            // G2 reads 32 score columns per step: the tiles right of the diagonal in row
-            // blocks 0 and 2 are zero.
-#pragma unroll
-            for (int ti = 0; ti < 4; ti += 2)
-                *reinterpret_cast<f16x4*>(&sm.S[16 * ti + l16][16 * (ti + 1) + 4 * g16]) = f16x4{0, 0, 0, 0};
-        }
-        __syncthreads();
-
-        // ---- output ----
-        if (out_wave) {
-            // y rows of this chunk; stores past the last token fall outside and are dropped
-            const __amdgpu_buffer_rsrc_t ry =
-                make_rsrc(a.y_out + ((int64_t)b * T + s0) * a.H * a.P, (int64_t)(T - s0) * a.H * a.P * 2);
-            for (int s = 0; s <= tt / 2; ++s) {
-                const f16x8 A = *reinterpret_cast<const f16x8*>(&sm.S[16 * tt + l16][32 * s + 8 * g16]);
-                const f16x8 Bo = *reinterpret_cast<const f16x8*>(&sm.XT[k & 1][16 * pt + l16][32 * s + 8 * g16]);
-                yacc = mfma16(A, Bo, yacc);
-            }
-#pragma unroll
-            for (int q = 0; q < TPL; ++q) {
-            const int st = s0 + (16 * tt + 4 * g16) / R + q;
-            const float z = bf(zr_bits[q]);
-            float o = 0.f;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const float zr = z * sm.mz[16 * pt + l16][r];
-                o += sm.md[16 * pt + l16][r] * zr * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-zr * kLog2e)) * yacc[q * R + r];
-            }
-            __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, (bf16)o), ry,
-                                                  ((st - s0) * a.H * a.P + hp + pe) * 2, 0, kStream);
-            }
-        }
-        if (g4_wave) {
-#pragma unroll
-            for (int j = 0; j < TPW; ++j) {
-                const int jt = wave * TPW + j;
-                const int nt = jt >> 1, ptj = jt & 1;
-                const f16x4 hv = f16x4{(f16)(hacc[j][0] * kHScale), (f16)(hacc[j][1] * kHScale),
-                                       (f16)(hacc[j][2] * kHScale), (f16)(hacc[j][3] * kHScale)};
-                *reinterpret_cast<f16x4*>(&sm.H[16 * ptj + l16][16 * nt + 4 * g16]) = hv;
-            }
-        }
-        if (k + 1 < nchunks) {
-            prep_chunk(k + 1);
-            if (k + 2 < nchunks) {
-                load_bc(k + 2);
+            if constexpr (!FULL) {
+                form_x(k + 1);
+                write_xw();
                 load_xv(k + 2);
-                store_theta();
             }
+            __syncthreads();
+        }
+        if constexpr (FULL) {
+            // Final state h[p][n] (fp32) from the accumulators.
+            if (a.h_final && tend == T) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int pt = 0; pt < 2; ++pt)
+                        *reinterpret_cast<f32x4*>(a.h_final + ((int64_t)bh * a.P + p0 + pw + 16 * pt + l16) * N + n0 + 32 * (t >> 1) + 8 * g16 + 4 * (t & 1)) = hacc[t][pt] * scl.state;
+            }
+        } else {
+            f32x4* hs = a.hseg + (((int64_t)seg * npairs + pair) * CW + wave) * (NT * 2 * 64) + lane;
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int pt = 0; pt < 2; ++pt) hs[(2 * t + pt) * 64] = hacc[t][pt];
+            if (wave == 0 && lane == 0 && pblk == 0) a.lseg[(int64_t)seg * sbase + bh] = ldec;
+        }
+    } else {
+        // =============================== helper waves ===============================
+        __builtin_amdgcn_s_setprio(3);  // the helpers' chains end both phases; the column waves have slack
+        const int hw = wave - CW, htid = tid - 64 * CW;
+        // the skip term D enters the masked scores, which carry 1 / (sB sC)
+        const float Dh = a.prm.D[h] * scl.inv_bc;
+        const f16* Bn = a.Bn + (int64_t)b * T * nrs + (int64_t)grp * NR;
+        const f16* Cn = a.Cn + (int64_t)b * T * nrs + (int64_t)grp * NR;
+        // rotation jobs: RoPE pairs 2 hl, 2 hl + 1 (columns 4 hl ..) of tokens tg TPT + m
+        const int hl = lane % LPT, tg = htid / LPT;
+        unsigned pwb[TPT][2][R], pwc[FULL ? TPT : 1][2][R];  // raw words, loaded a chunk ahead
+        const int bcoff = tg * TPT * nb + 8 * hl * R;
+        auto load_words = [&](const __amdgpu_buffer_rsrc_t& r, int so, unsigned (&w)[2][R]) {
+            if constexpr (R == 4) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, bcoff + 16 * e, so, 0);
+                    w[e][0] = v[0]; w[e][1] = v[1]; w[e][2] = v[2]; w[e][3] = v[3];
+                }
+            } else if constexpr (R == 2) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, bcoff, so, 0);
+                w[0][0] = v[0]; w[0][1] = v[1]; w[1][0] = v[2]; w[1][1] = v[3];
+            } else {
+                const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, bcoff, so, 0);
+                w[0][0] = v[0]; w[1][0] = v[1];
+            }
+        };
+        auto load_bc = [&](int kk) {
+            const __amdgpu_buffer_rsrc_t r = chunk_rsrc(Bn, kk, nb);
+#pragma unroll
+            for (int m = 0; m < TPT; ++m) load_words(r, m * nb, pwb[m]);
+            if constexpr (FULL) {
+                const __amdgpu_buffer_rsrc_t rc = chunk_rsrc(Cn, kk, nb);
+#pragma unroll
+                for (int m = 0; m < TPT; ++m) load_words(rc, m * nb, pwc[m]);
+            }
+        };
+        // theta of the rotation jobs' two pairs, raw bf16 x 2: [0] of the chunk to rotate next,
+        // [1] of the one after it
+        unsigned pth[2][TPT] = {};
+        const bool thvec = a.rs % 2 == 0 && a.pl.theta % 2 == 0 && reinterpret_cast<uintptr_t>(a.proj) % 4 == 0;
+        const int thoff = tg * TPT * rb + ((int)a.pl.theta + 2 * hl) * 2;
+        auto load_theta = [&](int kk) {
+            if (!a.cplx) return;  // no theta columns
+            const __amdgpu_buffer_rsrc_t r = chunk_rsrc(proj, kk, rb);
+            if (thvec) {
+#pragma unroll
+                for (int m = 0; m < TPT; ++m) pth[1][m] = __builtin_amdgcn_raw_buffer_load_b32(r, thoff, m * rb, 0);
+            } else {
+#pragma unroll
+                for (int m = 0; m < TPT; ++m)
+                    pth[1][m] = (unsigned)__builtin_amdgcn_raw_buffer_load_b16(r, thoff, m * rb, 0) |
+                                ((unsigned)__builtin_amdgcn_raw_buffer_load_b16(r, thoff + 2, m * rb, 0) << 16);
+            }
+        };
+        // this thread's sums of dt theta over its token group, chunk kk (theta in pth[1])
+        auto angle_sums = [&](int kk) {
+            if (!a.cplx) return;
+            const Tok& tk = sm.tok[kk % 3];
+            f32x2 ps = f32x2{0.f, 0.f};
+#pragma unroll
+            for (int m = 0; m < TPT; ++m) {
+                const float dt = tk.dt[tg * TPT + m];
+                ps[0] += dt * bf(pth[1][m]);
+                ps[1] += dt * __builtin_bit_cast(float, pth[1][m] & 0xffff0000u);
+            }
+            *reinterpret_cast<f32x2*>(&sm.part[tg][2 * hl]) = ps;
+        };
+        f32x2 phi_run = f32x2{0.f, 0.f};  // pair angles at the start of the chunk to rotate next
+        if (FULL && a.cplx)
+#pragma unroll 4
+            for (int j = 0; j < seg; ++j)
+                phi_run += *reinterpret_cast<const f32x2*>(a.aseg + ((int64_t)j * sbase + bh) * NH + 2 * hl);
+        // (cos, sin) of chunk kk's pairs: phi_t[i] = phi_{t-1}[i] - dt_t theta_t[i]
+        // (mamba3/mamba3.py:160-162), theta in pth[0]
+        f16x2 kA[TPT][2];
+        auto angles = [&](int kk) {
+            const Tok& tk = sm.tok[kk % 3];
+            f32x2 ph = phi_run;
+            if (a.cplx) {
+                f32x2 run = phi_run;
+#pragma unroll
+                for (int g = 0; g < GR; ++g) {
+                    if (g == tg) ph = run;
+                    run -= *reinterpret_cast<const f32x2*>(&sm.part[g][2 * hl]);
+                }
+                phi_run = run;
+            }
+#pragma unroll
+            for (int m = 0; m < TPT; ++m) {
+                kA[m][0] = kA[m][1] = f16x2{(f16)1.f, (f16)0.f};
+                if (a.cplx) {
+                    const float dt = tk.dt[tg * TPT + m];
+                    ph[0] -= dt * bf(pth[0][m]);
+                    ph[1] -= dt * __builtin_bit_cast(float, pth[0][m] & 0xffff0000u);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        float sn, cs;
+                        fast_sincos(ph[e], sn, cs);
+                        kA[m][e] = f16x2{(f16)cs, (f16)sn};
+                    }
+                }
+            }
+        };
+        // C~ / B~ rows of the words in hand (words of tokens past the end are zero), and Xw^T
+        auto write_tiles = [&]() {
+#pragma unroll
+            for (int m = 0; m < TPT; ++m) {
+                const int t = tg * TPT + m;
+                const f16x2 k0 = kA[m][0], k1 = kA[m][1];
+                const f16x2 s0 = __builtin_shufflevector(k0, k0, 1, 0), s1 = __builtin_shufflevector(k1, k1, 1, 0);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    *reinterpret_cast<u32x2*>(&sm.B[t * R + r][4 * hl]) =
+                        u32x2{rotate_pair(pwb[m][0][r], k0, s0), rotate_pair(pwb[m][1][r], k1, s1)};
+                    if constexpr (FULL)
+                        *reinterpret_cast<u32x2*>(&sm.C[t * R + r][4 * hl]) =
+                            u32x2{rotate_pair(pwc[m][0][r], k0, s0), rotate_pair(pwc[m][1][r], k1, s1)};
+                }
+            }
+            if constexpr (FULL) write_xw();
+        };
+        auto next_theta = [&]() {
+#pragma unroll
+            for (int m = 0; m < TPT; ++m) pth[0][m] = pth[1][m];
+        };
+        const bool token_wave = hw == 3;
+
+        // Prologue: chunks 0 and 1's token scalars, chunk 0's tiles, chunk 1's angle sums and
+        // reads (chunks past the end read as zero).
+        load_bc(0);
+        if constexpr (FULL) load_xv(0);
+        load_theta(0);
+        if (token_wave) {
+            load_tokens(0);
+            prep_tokens(0);
+            load_tokens(1);
+            prep_tokens(1);
+            load_tokens(2);
         }
         __syncthreads();
-    }
+        angle_sums(0);
+        next_theta();
+        load_theta(1);
+        __syncthreads();
+        angles(0);
+        if constexpr (FULL) {
+            form_x(0);
+            load_xv(1);
+        }
+        __syncthreads();
+        write_tiles();
+        load_bc(1);
+        angle_sums(1);
+        next_theta();
+        load_theta(2);
+        __syncthreads();
 
-    // Final state h[p][n] (fp32) from the accumulators: lane holds n = 16 nt + 4 g16 + v.
-    if (a.h_final && g4_wave) {
+        for (int k = 0; k < nchunks; ++k) {
+            const bool more = k + 1 < nchunks;
+            // ---- contract ----
+            if constexpr (FULL) {  // G2 of the previous chunk has read its X^T
 #pragma unroll
-        for (int j = 0; j < TPW; ++j) {
-            const int jt = wave * TPW + j;
-            const int nt = jt >> 1, ptj = jt & 1;
-            const int p = p0 + 16 * ptj + l16;
-            *reinterpret_cast<f32x4*>(a.h_final + ((int64_t)bh * a.P + p) * N + 16 * nt + 4 * g16) = hacc[j] * scl.state;
+                for (int v = 0; v < XV; ++v) *reinterpret_cast<xpiece*>(&sm.XT[xp][xt0 * R + XP * v]) = xo[v];
+            }
+            // the next chunk's angles and X first: their reads were issued a chunk ago
+            if (more) {
+                angles(k + 1);
+                if constexpr (FULL) {
+                    form_x(k + 1);
+                    load_xv(k + 2);
+                }
+            }
+            if (token_wave) {
+                prep_tokens(k + 2);
+                load_tokens(k + 3);
+            }
+            if constexpr (FULL) {
+                // Causal score tiles (ti, ui), ui <= ti, listed row by row as 0..9, dealt to the
+                // helpers in turn. A lane's four u-rows 16 ui + 4 g16 + v cover NU tokens; their
+                // mask factors are read (unconditionally: every index is below Q) and formed
+                // before the contraction.
+                const Tok& tk = sm.tok[k % 3];
+#pragma unroll 1
+                for (int idx = hw; idx < 10; idx += HELPERS) {
+                    const int ti = idx < 1 ? 0 : idx < 3 ? 1 : idx < 6 ? 2 : 3;
+                    const int ui = idx - ti * (ti + 1) / 2;
+                    constexpr int NU = R >= 4 ? 1 : 4 / R;
+                    const unsigned trow = 16 * ti + l16, t = trow / R;
+                    const unsigned ub = (unsigned)(16 * ui + 4 * g16) / R;
+                    const f16* pa = &sm.B[16 * ui + l16][8 * g16];
+                    const f16* pb = &sm.C[16 * ti + l16][8 * g16];
+                    const float ct = tk.c2[t];
+                    float fu[NU];
+#pragma unroll
+                    for (int j = 0; j < NU; ++j) {
+                        const unsigned u = ub + j;
+                        const float e = __builtin_amdgcn_exp2f(ct - tk.c2[u]);
+                        const float ab = fmaf(tk.bv[u], u < t ? 1.f : 0.f, tk.av[u]);
+                        fu[j] = u <= t ? e * ab : 0.f;
+                    }
+                    f32x4 sacc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int s = 0; s < KN; ++s) {
+                        const f16x8 A = *reinterpret_cast<const f16x8*>(pa + 32 * s);
+                        const f16x8 Bo = *reinterpret_cast<const f16x8*>(pb + 32 * s);
+                        sacc = mfma16(A, Bo, sacc);
+                    }
+                    // lane: u-row 16 ui + 4 g16 + v, t-row 16 ti + l16
+                    f16x4 sv;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float val = sacc[v] * fu[v * NU / 4];
+                        sv[v] = (f16)(16 * ui + 4 * g16 + v == (int)trow ? val + Dh : val);
+                    }
+                    *reinterpret_cast<f16x4*>(&sm.S[trow][16 * ui + 4 * g16]) = sv;
+                }
+            }
+            __syncthreads();
+            // ---- output ----
+            if (more) {
+                write_tiles();
+                load_bc(k + 2);
+                angle_sums(k + 2);
+                next_theta();
+                load_theta(k + 3);
+            }
+            __syncthreads();
+        }
+        // phi_run is the angle after the last chunk (rotated by the last pass)
+        if constexpr (FULL) {
+            if (a.angle && tend == T && pblk == 0 && htid < LPT)
+                *reinterpret_cast<f32x2*>(a.angle + (int64_t)bh * NH + 2 * hl) = phi_run;
+            // prev_BX = sum_r B~_{T-1}[n][r] X_{T-1}[p][r] (mamba3/mamba3.py:247-250) from the
+            // last chunk's tiles.
+            if (a.prev_bx && tend == T) {
+                const int tl = T - 1 - tbeg - (nchunks - 1) * Q;
+                for (int idx = htid; idx < PC * N; idx += HT) {
+                    const int p = idx / N, n = idx % N;
+                    float v = 0.f;
+#pragma unroll
+                    for (int r = 0; r < R; ++r) v += (float)sm.B[tl * R + r][n] * (float)sm.XT[p][tl * R + r];
+                    a.prev_bx[((int64_t)bh * a.P + p0 + p) * N + n] = v * scl.state;
+                }
+            }
+        } else {
+            if (pblk == 0 && htid < LPT)
+                *reinterpret_cast<f32x2*>(a.aseg + ((int64_t)seg * sbase + bh) * NH + 2 * hl) = phi_run;
         }
     }
-    if (a.angle && pblk == 0 && angle_wave && ai < NH)
-        a.angle[(int64_t)bh * NH + ai] = a.cplx ? phi_run : 0.f;
-    // prev_BX = sum_r B~_{T-1}[n][r] X_{T-1}[p][r] (mamba3/mamba3.py:247-250) from the last
-    // chunk's tiles.
-    if (a.prev_bx) {
-        const int tl = T - 1 - (nchunks - 1) * Q;
-        for (int idx = tid; idx < PB * N; idx += THREADS) {
-            const int p = idx / N, n = idx % N;
-            float v = 0.f;
-#pragma unroll
-            for (int r = 0; r < R; ++r) v += (float)sm.B[tl * R + r][n] * (float)sm.XT[(nchunks - 1) & 1][p][tl * R + r];
-            a.prev_bx[((int64_t)bh * a.P + p0 + p) * N + n] = v * scl.state;
+}
+
+// Turns the segments' end states (from a zero start, each in its own RoPE frame, whose zero is
+// its first token's incoming angle) into the states entering the next segments, in place: one
+// thread per four state rows of a column, walking the segments in order. HBM-bound (two passes
+// over the states); the full pass would otherwise read every earlier segment's.
+template <int N, int NCG>
+__global__ __launch_bounds__(256) void seg_combine(Args a) {
+    constexpr int NT = N / 32, CW = 2 * NCG;
+    constexpr int PER = CW * NT * 2 * 64;  // entries per pair block
+    const int npairs = a.B * a.H * a.PS;
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (int64_t)npairs * PER) return;
+    const int bh = (int)(e / PER) / a.PS;
+    const int w = (int)(e % PER) / (NT * 2 * 64), t = (int)(e % (NT * 2 * 64)) / 128, g16 = (int)(e % 64) / 16;
+    const int i = ((w & 1) * (N / 2) + 32 * (t >> 1) + 8 * g16 + 4 * (t & 1)) / 2;  // first RoPE pair
+    const int64_t sbase = (int64_t)a.B * a.H;
+    f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x2 phi = f32x2{0.f, 0.f};
+#pragma unroll 2
+    for (int j = 0; j < a.segs - 1; ++j) {
+        f32x4* hj = a.hseg + (int64_t)j * npairs * PER + e;
+        const f32x4 v = *hj;
+        const f32x2 inc = *reinterpret_cast<const f32x2*>(a.aseg + ((int64_t)j * sbase + bh) * (N / 2) + i);
+        const float dec = __builtin_amdgcn_exp2f(a.lseg[(int64_t)j * sbase + bh]);
+        float s0, c0, s1, c1;
+        fast_sincos(phi[0], s0, c0);
+        fast_sincos(phi[1], s1, c1);
+        h = h * dec + f32x4{v[0] * c0 - v[1] * s0, v[0] * s0 + v[1] * c0,
+                            v[2] * c1 - v[3] * s1, v[2] * s1 + v[3] * c1};
+        *hj = h;
+        phi += inc;
+    }
+}
+
+template <int N, int R, int NCG>
+void launch_ssd(const Args& a, hipStream_t stream) {
+    const unsigned npairs = (unsigned)(a.B * a.H * a.PS);
+    const dim3 threads(64 * (2 * NCG + Layout<N, R>::HELPERS));
+    if (a.segs > 1) {
+        hipLaunchKernelGGL((ssd_wide<N, R, NCG, false>), dim3(npairs * (a.segs - 1)), threads, 0, stream, a);
+        hipLaunchKernelGGL((seg_combine<N, NCG>), dim3((unsigned)(((int64_t)npairs * PW * NCG * N / 4 + 255) / 256)),
+                           dim3(256), 0, stream, a);
+    }
+    hipLaunchKernelGGL((ssd_wide<N, R, NCG, true>), dim3(npairs * a.segs), threads, 0, stream, a);
+}
+
+inline size_t al256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+// Workspace: B^ and C^ rows, then the segments' states, log-decays and angle increments.
+struct Plan {
+    int segs, seg0;
+    int ncg;  // column groups per workgroup
+    size_t rows, hseg, lseg, total;  // bytes of B^ (and of C^); offsets; bytes in all
+};
+
+// Segments of a call. The pairs alone fill the 256 CUs from about 192 on (a segmented walk
+// does 1.5x the work: its state pass). The cuts lie at fixed tokens, closer at the start, so
+// that a short prompt splits finely and a long one into few states, and no segment is much
+// longer than the mean of its sequence's share per CU; as they depend on neither the length
+// nor, below that pair count, the batch, a prefix or a sub-batch reproduces the same bits.
+Plan make_plan(const m3_layer_desc& d, size_t limit) {
+    const size_t BH = (size_t)d.batch * d.nheads;
+    Plan p;
+    p.ncg = column_groups(d.headdim, d.d_state, d.mimo_rank);
+    p.rows = (size_t)d.batch * d.seqlen * d.ngroups * d.d_state * d.mimo_rank * sizeof(f16);
+    p.seg0 = std::max(256, d.headdim * d.d_state / 64);
+    p.segs = 1;
+    p.hseg = al256(2 * p.rows);
+    p.lseg = p.hseg;
+    p.total = 2 * p.rows + 256;
+    if (BH * (d.headdim / (PW * p.ncg)) < 192 && d.seqlen > p.seg0) {
+        int segs = 1;
+        while (seg_start(segs, p.seg0) < d.seqlen) ++segs;
+        const size_t n = segs - 1;
+        const size_t lseg = p.hseg + al256(n * BH * d.headdim * d.d_state * sizeof(float));
+        const size_t total = lseg + al256(n * BH * sizeof(float)) + n * BH * (d.d_state / 2) * sizeof(float) + 256;
+        if (total <= limit) {  // else a caller's workspace without room for the states: one walk
+            p.segs = segs;
+            p.lseg = lseg;
+            p.total = total;
         }
     }
+    // Narrower blocks where the workgroups would leave CUs idle: they repeat the rotation and
+    // the scores, but each walks its chunks faster (same bits: a column's arithmetic does not
+    // depend on its block).
+    while (p.ncg > 1 && BH * (d.headdim / (PW * p.ncg)) * p.segs < 192) p.ncg /= 2;
+    return p;
 }
 
 template <int N, int R>
 int launch(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
            const float* dt_scale, void* y_out, float* h_final, float* angle, float* prev_bx,
-           void* workspace, hipStream_t stream) {
+           void* workspace, size_t limit, hipStream_t stream) {
+    const Plan plan = make_plan(d, limit);
+    const int ncg = plan.ncg;
+    char* ws = reinterpret_cast<char*>(workspace);
     Args a;
     a.B = d.batch; a.T = d.seqlen; a.H = d.nheads; a.G = d.ngroups; a.P = d.headdim;
-    a.PS = d.headdim / PB;
+    a.PS = d.headdim / (PW * ncg);
     a.trap = d.use_trapezoidal; a.cplx = d.use_complex;
     a.rs = d.proj_row_stride;
     a.pl = proj_layout(d);
@@ -769,14 +1015,19 @@ int launch(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
     a.proj = reinterpret_cast<const bf16*>(proj);
     a.dt_scale = dt_scale;
     const int64_t nrows = (int64_t)d.batch * d.seqlen * d.ngroups;
-    f16* bn = reinterpret_cast<f16*>(workspace);
-    f16* cn = bn + nrows * N * R;
+    f16* bn = reinterpret_cast<f16*>(ws);
+    f16* cn = reinterpret_cast<f16*>(ws + plan.rows);
     a.Bn = bn;
     a.Cn = cn;
     a.y_out = reinterpret_cast<bf16*>(y_out);
     a.h_final = h_final;
     a.angle = angle;
     a.prev_bx = prev_bx;
+    a.segs = plan.segs;
+    a.seg0 = plan.seg0;
+    a.hseg = reinterpret_cast<f32x4*>(ws + plan.hseg);
+    a.lseg = reinterpret_cast<float*>(ws + plan.lseg);
+    a.aseg = reinterpret_cast<float*>(ws + plan.lseg + al256((size_t)(plan.segs - 1) * d.batch * d.nheads * sizeof(float)));
     // vector loads of a pair's 2R raw values when every row offset keeps them aligned
     const int vec = a.rs % (2 * R) == 0 && a.pl.B % (2 * R) == 0 && a.pl.C % (2 * R) == 0 &&
                     reinterpret_cast<uintptr_t>(proj) % (4 * R) == 0;
@@ -784,8 +1035,14 @@ int launch(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
     hipLaunchKernelGGL((bc_norm_wide<N, R>), dim3((unsigned)((nrows + rows_per_block - 1) / rows_per_block)),
                        dim3(256), 0, stream, a.proj, a.rs, a.pl.B, a.pl.C, a.G, nrows, d.rms_eps, vec,
                        p.B_norm_w, p.B_bias, p.C_norm_w, p.C_bias, bn, cn);
-    hipLaunchKernelGGL((ssd_wide<N, R>), dim3((unsigned)(d.batch * d.nheads * a.PS)), dim3(THREADS), 0,
-                       stream, a);
+    if constexpr (kMaxGroups<N, R> == 4) {
+        if (ncg == 4) {
+            launch_ssd<N, R, 4>(a, stream);
+            return hipGetLastError() == hipSuccess ? M3_OK : M3_ERR_LAUNCH;
+        }
+    }
+    if (ncg == 2) launch_ssd<N, R, 2>(a, stream);
+    else launch_ssd<N, R, 1>(a, stream);
     return hipGetLastError() == hipSuccess ? M3_OK : M3_ERR_LAUNCH;
 }
 
@@ -793,25 +1050,26 @@ int launch(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
 
 bool wide_prefill_supported(const m3_layer_desc& d) {
     if (d.dtype != M3_DTYPE_BF16) return false;
-    if (d.headdim % wd::PB != 0) return false;
+    if (d.headdim % wd::PW != 0) return false;
     const int N = d.d_state, R = d.mimo_rank;
     if (N != 64 && N != 128 && N != 256) return false;
     if (R != 1 && R != 2 && R != 4) return false;
-    return true;
+    // a chunk's rows (up to 64 tokens) are addressed with 32-bit byte offsets
+    const int64_t lim = (int64_t)1 << 23;
+    return d.proj_row_stride < lim && (int64_t)d.ngroups * N * R < lim && (int64_t)d.nheads * d.headdim < lim;
 }
 
-size_t wide_prefill_workspace(const m3_layer_desc& d) {
-    const size_t nrows = (size_t)d.batch * d.seqlen * d.ngroups;
-    return 2 * nrows * d.d_state * d.mimo_rank * sizeof(f16) + 256;
+size_t wide_prefill_workspace(const m3_layer_desc& d, size_t limit) {
+    return wd::make_plan(d, limit).total;
 }
 
 int launch_wide_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                         const float* dt_scale, void* y_out, float* h_final, float* angle,
-                        float* prev_bx, void* workspace, hipStream_t stream) {
+                        float* prev_bx, void* workspace, size_t limit, hipStream_t stream) {
 #define M3_WIDE_CASE(n, r)                                                                      \
     if (d.d_state == n && d.mimo_rank == r)                                                     \
         return wd::launch<n, r>(d, p, proj, dt_scale, y_out, h_final, angle, prev_bx, workspace, \
-                                stream);
+                                limit, stream);
     M3_WIDE_CASE(64, 1) M3_WIDE_CASE(64, 2) M3_WIDE_CASE(64, 4)
     M3_WIDE_CASE(128, 1) M3_WIDE_CASE(128, 2) M3_WIDE_CASE(128, 4)
     M3_WIDE_CASE(256, 1) M3_WIDE_CASE(256, 2) M3_WIDE_CASE(256, 4)

@@ -926,3 +926,66 @@ def test_bf16_staged_prefill_equals_generic_kernel(kw, B, T, cuda_device):
     assert max_rel(staged[0].float(), generic[0].float()) < 2.0 ** -7
     for name, a, b in zip(("h", "angle", "prev_BX"), staged[1:], generic[1:]):
         assert max_rel(a, b) < 1e-5, name
+
+
+@pytest.mark.parametrize("N", [64, 128, 256])
+@pytest.mark.parametrize("R", [1, 2, 4])
+@pytest.mark.parametrize("P", [64, 128])
+def test_general_kernel_column_blocks_agree(N, R, P, cuda_device):
+    """A batch of 192 (batch, head) pairs runs the general MFMA kernel in blocks of the whole
+    headdim (64 or 128 columns), one row alone in blocks of 32: a column's arithmetic does not
+    depend on its block, so rows agree bit for bit (T ends mid-chunk)."""
+    print(f"column blocks N {N} R {R} P {P}", flush=True)
+    kw = dict(d_model=256, d_state=N, headdim=P, mimo_rank=R, ngroups=2)
+    torch.manual_seed(31)
+    layer = mamba3_amd.KulaMamba(**kw).to(cuda_device, torch.bfloat16).eval()
+    if N == 128 and P == 64 and R == 2:
+        pytest.skip("the d_state 128 / headdim 64 / rank 2 kernel's shape")
+    B, T = 192 // layer.nheads, 67
+    with torch.no_grad():
+        proj = layer.in_proj(torch.randn(B, T, 256, device=cuda_device, dtype=torch.bfloat16))
+        assert _native.prefill_kernel_name(layer._desc(B, T, proj), proj) == "mfma_general"
+        y, st = layer.ssd_from_proj(proj, return_state=True)
+        for b in (0, B - 1):
+            y1, st1 = layer.ssd_from_proj(proj[b:b + 1].contiguous(), return_state=True)
+            assert torch.equal(y1, y[b:b + 1])
+            for k in ("h", "prev_BX", "angle"):
+                assert torch.equal(st1[k], st[k][b:b + 1]), k
+
+
+@pytest.mark.parametrize("kw,T", [
+    (dict(d_model=64, d_state=64, headdim=64, mimo_rank=2), 257),     # second segment of one token
+    (dict(d_model=64, d_state=64, headdim=32, mimo_rank=1, ngroups=2), 1100),  # into the 512-token segments
+    (dict(d_model=64, d_state=128, headdim=64, mimo_rank=4, use_trapezoidal=False), 600),
+    (dict(d_model=64, d_state=256, headdim=128, mimo_rank=4, use_complex_ssm=False), 520),
+    (dict(d_model=128, d_state=256, headdim=128, mimo_rank=1), 513),
+])
+def test_general_kernel_segments_match_fp32_oracle(kw, T, cuda_device):
+    """Sequences cut into segments (state pass, combine, full pass) with dt_scale against the
+    fp32 oracle, and as one walk in a workspace without room for the segments' states; a
+    prefix that ends inside the segmented run reproduces it bit for bit."""
+    print(f"segments {kw} T {T}", flush=True)
+    dev = cuda_device
+    layer, cfg, p = _bf16_pair(kw, dev, seed=17)
+    torch.manual_seed(T)
+    x = torch.randn(2, T, kw["d_model"]).to(torch.bfloat16)
+    ds = torch.rand(2, T, layer.nheads) * 1.5 + 0.5
+    with torch.no_grad():
+        y_ref, st_ref = ref.layer_forward(cfg, p, x.float(), dt_scale=ds, return_state=True)
+        proj = layer.in_proj(x.to(dev)).contiguous()
+        dsd = ds.to(dev)
+        y, st = layer.ssd_from_proj(proj, dt_scale=dsd, return_state=True)
+        cut = T - 60
+        yp, _ = layer.ssd_from_proj(proj[:, :cut].contiguous(), dt_scale=dsd[:, :cut])
+        assert torch.equal(yp, y[:, :cut])
+        desc = layer._desc(2, T, proj)
+        rows = 2 * 2 * T * layer.ngroups * layer.d_state * layer.mimo_rank * 2 + 256
+        assert rows < _native.prefill_workspace_bytes(desc)
+        y1, h1, a1, b1 = (torch.empty_like(t) for t in (y, st["h"], st["angle"], st["prev_BX"]))
+        ws = torch.empty(rows, device=dev, dtype=torch.uint8)
+        _native.prefill_fwd(desc, layer._param_pack(), proj, dsd, y1, h1, a1, b1, ws, rows)
+        for out in (y, y1):
+            assert max_rel(layer.out_proj(out).float(), y_ref) < BF16_TOL
+    for k, one in (("h", h1), ("prev_BX", b1), ("angle", a1)):
+        assert max_rel(st[k], st_ref[k]) < BF16_TOL, k
+        assert max_rel(one, st_ref[k]) < BF16_TOL, k
