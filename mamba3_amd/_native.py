@@ -203,8 +203,15 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# The current stream's handle by device index, without the Stream object that
+# torch.cuda.current_stream builds (4 us a call; a decode step makes three).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.get_device())
 
 
 def scan_fwd(decay: torch.Tensor, h_chunk: torch.Tensor, h_init: torch.Tensor | None,
@@ -244,10 +251,11 @@ def prefill_kernel_name(desc: LayerDesc, proj=None, y_out=None, h_final=None, pr
 
 def prefill_fwd(desc: LayerDesc, params: LayerParams, proj, dt_scale, y_out, h_final, angle,
                 prev_bx, workspace, workspace_bytes: int) -> None:
-    check(lib().m3_prefill_fwd(ctypes.byref(desc), ctypes.byref(params), ptr(proj),
-                               ptr(dt_scale), ptr(y_out), ptr(h_final), ptr(angle),
-                               ptr(prev_bx), ptr(workspace), workspace_bytes,
-                               stream_of(proj)), "m3_prefill_fwd")
+    st = lib().m3_prefill_fwd(ctypes.byref(desc), ctypes.byref(params), proj.data_ptr(),
+                              ptr(dt_scale), y_out.data_ptr(), ptr(h_final), ptr(angle),
+                              ptr(prev_bx), ptr(workspace), workspace_bytes, stream_of(proj))
+    if st:
+        check(st, "m3_prefill_fwd")
 
 
 def prefill_fwd_noalloc(desc: LayerDesc, params: LayerParams, proj, dt_scale, y_out, h_final,
@@ -260,10 +268,12 @@ def prefill_fwd_noalloc(desc: LayerDesc, params: LayerParams, proj, dt_scale, y_
 
 def step_fwd(desc: LayerDesc, params: LayerParams, proj, dt_scale, h_in, prev_in, angle_in,
              y_out, h_out, prev_out, angle_out) -> None:
-    check(lib().m3_step_fwd(ctypes.byref(desc), ctypes.byref(params), ptr(proj),
-                            ptr(dt_scale), ptr(h_in), ptr(prev_in), ptr(angle_in),
-                            dtype_code(angle_in.dtype), ptr(y_out), ptr(h_out), ptr(prev_out),
-                            ptr(angle_out), stream_of(proj)), "m3_step_fwd")
+    st = lib().m3_step_fwd(ctypes.byref(desc), ctypes.byref(params), proj.data_ptr(),
+                           ptr(dt_scale), h_in.data_ptr(), prev_in.data_ptr(), angle_in.data_ptr(),
+                           dtype_code(angle_in.dtype), y_out.data_ptr(), h_out.data_ptr(),
+                           prev_out.data_ptr(), angle_out.data_ptr(), stream_of(proj))
+    if st:
+        check(st, "m3_step_fwd")
 
 
 def chunked_fwd_mfma_applies(B, T, H, P, N, R, has_beta: bool) -> bool:
@@ -365,9 +375,11 @@ def step_bwd(desc: LayerDesc, params: LayerParams, proj, dt_scale, h_in, prev_in
 def rmsnorm_fwd(x, weight, y, rstd, eps: float) -> None:
     """m3_rmsnorm_fwd on contiguous x (rows, d)."""
     rows, d = x.shape
-    check(lib().m3_rmsnorm_fwd(ptr(x), dtype_code(x.dtype), ptr(weight), dtype_code(weight.dtype),
-                               ptr(y), dtype_code(y.dtype), ptr(rstd), rows, d, eps,
-                               stream_of(x)), "m3_rmsnorm_fwd")
+    st = lib().m3_rmsnorm_fwd(x.data_ptr(), dtype_code(x.dtype), weight.data_ptr(),
+                              dtype_code(weight.dtype), y.data_ptr(), dtype_code(y.dtype),
+                              ptr(rstd), rows, d, eps, stream_of(x))
+    if st:
+        check(st, "m3_rmsnorm_fwd")
 
 
 SMALL_PROJ_MAX_ROWS = 8
@@ -385,15 +397,19 @@ def small_proj_ok(m: int, k: int, norm: bool = False) -> bool:
 def small_linear(x, norm_w, eps, weight, residual, scale, out) -> None:
     """m3_small_linear on contiguous bf16 x (m, k), weight (n, k), out (m, n)."""
     m, k = x.shape
-    check(lib().m3_small_linear(ptr(x), ptr(norm_w), eps, ptr(weight), ptr(residual), scale,
-                                ptr(out), m, weight.shape[0], k, stream_of(x)), "m3_small_linear")
+    st = lib().m3_small_linear(x.data_ptr(), ptr(norm_w), eps, weight.data_ptr(), ptr(residual),
+                               scale, out.data_ptr(), m, weight.shape[0], k, stream_of(x))
+    if st:
+        check(st, "m3_small_linear")
 
 
 def small_swiglu(x, norm_w, eps, w_gate, w_up, out) -> None:
     """m3_small_swiglu on contiguous bf16 x (m, k), weights (n, k), out (m, n)."""
     m, k = x.shape
-    check(lib().m3_small_swiglu(ptr(x), ptr(norm_w), eps, ptr(w_gate), ptr(w_up), ptr(out), m,
-                                w_gate.shape[0], k, stream_of(x)), "m3_small_swiglu")
+    st = lib().m3_small_swiglu(x.data_ptr(), ptr(norm_w), eps, w_gate.data_ptr(), w_up.data_ptr(),
+                               out.data_ptr(), m, w_gate.shape[0], k, stream_of(x))
+    if st:
+        check(st, "m3_small_swiglu")
 
 
 def silu_mul(gate_up, d_ff, out) -> None:

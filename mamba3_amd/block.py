@@ -154,20 +154,23 @@ class KulaMambaBlock(nn.Module):
         """The decode step runs on the small-batch projection kernels (norm + in_proj,
         out_proj + residual, norm + SwiGLU, w_down + residual): bf16, at most 8 rows, no
         biases, last-dimension norms, nothing to differentiate."""
-        ssm = self.ssm
-        ws = [self.ssm_norm.weight, ssm.in_proj.weight, ssm.out_proj.weight]
-        lins = [ssm.in_proj, ssm.out_proj]
-        if self.use_mlp:
-            ws += [self.mlp_norm.weight, self.mlp.w_gate.weight, self.mlp.w_up.weight,
-                   self.mlp.w_down.weight]
-            lins += [self.mlp.w_gate, self.mlp.w_up, self.mlp.w_down]
-        norms = [self.ssm_norm] + ([self.mlp_norm] if self.use_mlp else [])
         m = x.shape[0]
+        if m > _native.SMALL_PROJ_MAX_ROWS or x.dtype != torch.bfloat16:
+            return False
+        ssm, norm = self.ssm, self.ssm_norm
+        ip, op = ssm.in_proj, ssm.out_proj
         # every projection's K: d_model (with a norm), d_inner, d_ff
-        ks_ok = _native.small_proj_ok(m, ssm.out_proj.in_features) and (
-            not self.use_mlp or _native.small_proj_ok(m, self.mlp.w_down.in_features))
-        return (ks_ok and all(l.bias is None for l in lins) and all(n.dim in (-1, 1) for n in norms)
-                and ops.small_proj_usable(x, *ws, norm=True))
+        if not (_native.small_proj_ok(m, op.in_features) and ip.bias is None and op.bias is None
+                and norm.dim in (-1, 1)):
+            return False
+        if not self.use_mlp:
+            return ops.small_proj_usable(x, norm.weight, ip.weight, op.weight, norm=True)
+        mlp, norm2 = self.mlp, self.mlp_norm
+        gate, up, down = mlp.w_gate, mlp.w_up, mlp.w_down
+        return (_native.small_proj_ok(m, down.in_features) and gate.bias is None
+                and up.bias is None and down.bias is None and norm2.dim in (-1, 1)
+                and ops.small_proj_usable(x, norm.weight, ip.weight, op.weight, norm2.weight,
+                                          gate.weight, up.weight, down.weight, norm=True))
 
     def _small_step_tail(self, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
         """x + s out_proj(y), then the MLP residual, on the small-batch kernels."""

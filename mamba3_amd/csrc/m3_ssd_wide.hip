@@ -38,10 +38,10 @@
 //   S [(t,r)][(u,r')]                 masked scores (fp32 accumulated)
 //   tok, part (fp32)                  token scalars; sums of dt theta of token groups
 // Contractions (v_mfma_f32_16x16x32_f16, fp32 accumulation):
-//   G3  Y   = diag(e^{c_t}) C~ H^T    H^T straight from the accumulators: contraction slot
-//             (g, j) of lane group g is n = 4g + j of one 16-row tile for j < 4 and of the
-//             next for j >= 4, which are the rows the lane's accumulators hold, so the state
-//             is converted to f16 in registers and never goes through LDS
+//   G3  Y   = diag(e^{c_t}) C~ H^T    H^T straight from the accumulators, converted to f16 in
+//             registers: state tile 2s + i holds the rows n = 32 s + 8 g + 4 i + v (lane group
+//             g, accumulator v), so tiles 2s and 2s + 1 give a lane the eight contraction slots
+//             that its 128-bit read of a C~ row covers (the transpose reads of G4 pick the rows)
 //   G4  H^T = e^{c_end} H^T + B~^T Xw    (A operand by LDS transpose reads of B~)
 //   G1  S^T = B~ C~^T per causal 16x16 tile, masked by
 //             Lc[t][u] = [u<=t] e^{c_t - c_u} (a_u + [u<t] b_u), plus D on the diagonal

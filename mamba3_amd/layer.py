@@ -40,10 +40,8 @@ class RMSNorm(nn.Module):
         _native.require_gpu(x)
         d = self.dim % x.ndim
         if d != x.ndim - 1:
-            y, _ = ops.rmsnorm(x.movedim(d, -1), self.weight, float(self.eps))
-            return y.movedim(-1, d)
-        y, _ = ops.rmsnorm(x, self.weight, float(self.eps))
-        return y
+            return ops.rmsnorm_fast(x.movedim(d, -1), self.weight, float(self.eps)).movedim(-1, d)
+        return ops.rmsnorm_fast(x, self.weight, float(self.eps))
 
 
 class KulaMamba(nn.Module):
@@ -122,8 +120,15 @@ class KulaMamba(nn.Module):
 
     # ------------------------------------------------------------------ native glue
     def _small_params(self):
-        return (self.A_log, self.D, self.dt_bias, self.B_norm.weight, self.C_norm.weight,
-                self.B_bias, self.C_bias, self.mimo_x, self.mimo_z, self.mimo_down)
+        # straight from the registries: Module.__getattr__ ten times over is 3 us of a step
+        p, m = self._parameters, self._modules
+        try:
+            return (p["A_log"], p["D"], p["dt_bias"], m["B_norm"]._parameters["weight"],
+                    m["C_norm"]._parameters["weight"], p["B_bias"], p["C_bias"], p["mimo_x"],
+                    p["mimo_z"], p["mimo_down"])
+        except KeyError:  # a parametrized or otherwise replaced parameter
+            return (self.A_log, self.D, self.dt_bias, self.B_norm.weight, self.C_norm.weight,
+                    self.B_bias, self.C_bias, self.mimo_x, self.mimo_z, self.mimo_down)
 
     def _param_pack(self) -> _native.LayerParams:
         """fp32 copies of the small parameters as the C-ABI struct (cached per version)."""
@@ -213,7 +218,7 @@ class KulaMamba(nn.Module):
                                         any(p.requires_grad for p in params)):
             y, h, angle, prev, _ = ops.prefill_train(proj, *params, scale, *args)
         else:
-            y, h, angle, prev = ops.prefill(proj, *params, scale, *args, return_state)
+            y, h, angle, prev = ops.prefill_fast(proj, *params, scale, *args, return_state)
         state = {"h": h, "angle": angle, "prev_BX": prev} if return_state else None
         return y, state
 

@@ -21,6 +21,8 @@ from collections import OrderedDict
 from typing import Optional
 
 import torch
+from torch import _C
+from torch.autograd import forward_ad as _forward_ad
 
 from . import _native
 
@@ -33,11 +35,17 @@ _F32_CACHE_MAX = 256
 def _cache_entry(params) -> list:
     """[LayerParams, fp32 tensors, weak refs] for the ten layer parameters. An entry is
     used only while every source tensor is the same live object at the same version."""
-    key = tuple((t.data_ptr(), t._version, t.dtype, t.device) for t in params)
+    # (an address names its device)
+    key = (*[t.data_ptr() for t in params], *[t._version for t in params],
+           *[t.dtype for t in params])
     hit = _F32_CACHE.get(key)
-    if hit is not None and all(r() is t for r, t in zip(hit[2], params)):
-        _F32_CACHE.move_to_end(key)
-        return hit
+    if hit is not None:
+        for r, t in zip(hit[2], params):
+            if r() is not t:
+                break
+        else:
+            _F32_CACHE.move_to_end(key)
+            return hit
     with torch.no_grad():
         f32 = [t.detach().float().contiguous() for t in params]
     entry = [_native.LayerParams(*[t.data_ptr() for t in f32]), f32,
@@ -56,10 +64,9 @@ def _f32_params(params) -> tuple:
 
 def _desc(batch, seqlen, nheads, headdim, d_state, mimo_rank, ngroups, trap, cplx, eps,
           dtype, row_stride) -> _native.LayerDesc:
-    return _native.LayerDesc(
-        batch=batch, seqlen=seqlen, nheads=nheads, headdim=headdim, d_state=d_state,
-        mimo_rank=mimo_rank, ngroups=ngroups, use_trapezoidal=int(trap), use_complex=int(cplx),
-        dtype=_native.dtype_code(dtype), proj_row_stride=row_stride, rms_eps=float(eps))
+    return _native.LayerDesc(batch, seqlen, nheads, headdim, d_state, mimo_rank, ngroups,
+                             int(trap), int(cplx), _native.dtype_code(dtype), row_stride,
+                             float(eps), 0)
 
 
 def _state_shapes(B, nheads, headdim, d_state):
@@ -67,16 +74,11 @@ def _state_shapes(B, nheads, headdim, d_state):
 
 
 # ---------------------------------------------------------------------------- prefill
-@torch.library.custom_op(f"{NS}::prefill", mutates_args=())
-def prefill(proj: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor, dt_bias: torch.Tensor,
-            B_norm_w: torch.Tensor, C_norm_w: torch.Tensor, B_bias: torch.Tensor,
-            C_bias: torch.Tensor, mimo_x: torch.Tensor, mimo_z: torch.Tensor,
-            mimo_down: torch.Tensor, dt_scale: Optional[torch.Tensor], nheads: int,
-            headdim: int, d_state: int, mimo_rank: int, ngroups: int, trap: bool, cplx: bool,
-            eps: float, return_state: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor,
-                                                     torch.Tensor]:
+def _prefill_eager(proj, A_log, D, dt_bias, B_norm_w, C_norm_w, B_bias, C_bias, mimo_x, mimo_z,
+                   mimo_down, dt_scale, nheads, headdim, d_state, mimo_rank, ngroups, trap, cplx,
+                   eps, return_state):
     """m3_prefill_fwd: in_proj output (B,T,W) -> (y (B,T,H*P) in proj.dtype, h, angle,
-    prev_BX). Without return_state the three state tensors are empty."""
+    prev_BX), the states None without return_state."""
     _native.require_gpu(proj)
     proj = proj.contiguous()
     Bat, T, _ = proj.shape
@@ -96,9 +98,25 @@ def prefill(proj: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor, dt_bias: t
     ws_bytes = _native.prefill_workspace_bytes(desc)
     ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
     _native.prefill_fwd(desc, pack, proj, dt_scale, y, h, angle, prev, ws, ws_bytes)
-    if not return_state:  # three distinct empty tensors: outputs of an op may not alias
-        h, angle, prev = (torch.empty(0, device=dev, dtype=torch.float32) for _ in range(3))
     return y, h, angle, prev
+
+
+@torch.library.custom_op(f"{NS}::prefill", mutates_args=())
+def prefill(proj: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor, dt_bias: torch.Tensor,
+            B_norm_w: torch.Tensor, C_norm_w: torch.Tensor, B_bias: torch.Tensor,
+            C_bias: torch.Tensor, mimo_x: torch.Tensor, mimo_z: torch.Tensor,
+            mimo_down: torch.Tensor, dt_scale: Optional[torch.Tensor], nheads: int,
+            headdim: int, d_state: int, mimo_rank: int, ngroups: int, trap: bool, cplx: bool,
+            eps: float, return_state: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor,
+                                                     torch.Tensor]:
+    """_prefill_eager as an op. Without return_state the three state tensors are empty."""
+    out = _prefill_eager(proj, A_log, D, dt_bias, B_norm_w, C_norm_w, B_bias, C_bias, mimo_x,
+                         mimo_z, mimo_down, dt_scale, nheads, headdim, d_state, mimo_rank, ngroups,
+                         trap, cplx, eps, return_state)
+    if return_state:
+        return out
+    # three distinct empty tensors: outputs of an op may not alias
+    return (out[0], *(torch.empty(0, device=proj.device, dtype=torch.float32) for _ in range(3)))
 
 
 @prefill.register_fake
@@ -529,18 +547,24 @@ def layer_args(layer) -> tuple:
 
 
 # ---------------------------------------------------------------------------- RMSNorm
+def _rmsnorm_eager(x: torch.Tensor, weight: torch.Tensor, eps: float, keep: bool = False):
+    """m3_rmsnorm_fwd over the last dimension of x: y in the promotion of x's and the weight's
+    dtypes, and with `keep` rstd (rows,) fp32 (else None)."""
+    _native.require_gpu(x, weight)
+    x2 = x.reshape(-1, x.shape[-1]).contiguous()
+    y = torch.empty(x2.shape, device=x.device,
+                    dtype=x.dtype if x.dtype == weight.dtype
+                    else torch.promote_types(x.dtype, weight.dtype))
+    rstd = torch.empty(x2.shape[0], device=x.device, dtype=torch.float32) if keep else None
+    _native.rmsnorm_fwd(x2, weight.contiguous(), y, rstd, eps)
+    return y.view(x.shape), rstd
+
+
 @torch.library.custom_op(f"{NS}::rmsnorm", mutates_args=())
 def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """m3_rmsnorm_fwd over the last dimension of x: (y in the promotion of x's and the
     weight's dtypes, rstd (rows,) fp32)."""
-    _native.require_gpu(x, weight)
-    d = x.shape[-1]
-    x2 = x.reshape(-1, d).contiguous()
-    wc = weight.contiguous()
-    y = torch.empty(x2.shape, device=x.device, dtype=torch.promote_types(x.dtype, weight.dtype))
-    rstd = torch.empty(x2.shape[0], device=x.device, dtype=torch.float32)
-    _native.rmsnorm_fwd(x2, wc, y, rstd, eps)
-    return y.reshape(x.shape), rstd
+    return _rmsnorm_eager(x, weight, eps, True)
 
 
 @rmsnorm.register_fake
@@ -658,25 +682,45 @@ def _(gate_up, d_ff):
     return gate_up.new_empty(*gate_up.shape[:-1], d_ff)
 
 
-# ---------------------------------------------------------------- eager decode calls
-def _direct() -> bool:
-    """Eager calls with autograd off bypass the dispatcher: its per-call host time is what a
-    per-token decode loop waits on. Traced calls and calls under autograd go through the
-    registered ops and their autograd formulas."""
-    return not torch.is_grad_enabled() and not torch.compiler.is_compiling()
+# ---------------------------------------------------------------- eager calls
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _direct(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Eager calls with autograd off bypass the dispatcher: its per-call host time (16 us for
+    the prefill op) is what a per-token decode loop and a short prompt wait on. Traced calls,
+    calls under autograd, a dispatch or function mode, a functorch transform or forward-mode
+    AD, and calls on tensor subclasses go through the registered ops and their formulas. `a`
+    and `b` stand for the activations and the parameters."""
+    return not (torch.is_grad_enabled() or torch.compiler.is_compiling()
+                or _C._len_torch_dispatch_stack() or _C._len_torch_function_stack()
+                or _C._get_tracing_state() is not None
+                or _C._functorch.peek_interpreter_stack() is not None
+                or _forward_ad._current_level >= 0
+                or type(a) not in _PLAIN or type(b) not in _PLAIN)
+
+
+def prefill_fast(*args):
+    return (_prefill_eager if _direct(args[0], args[1]) else prefill)(*args)
 
 
 def step_fast(*args):
-    return (_step_eager if _direct() else step)(*args)
+    return (_step_eager if _direct(args[0], args[1]) else step)(*args)
 
 
-def small_linear_fast(*args):
-    return (_small_linear_eager if _direct() else small_linear)(*args)
+def small_linear_fast(x, norm_w, eps, weight, residual, scale):
+    fn = _small_linear_eager if _direct(x, weight) else small_linear
+    return fn(x, norm_w, eps, weight, residual, scale)
 
 
-def small_swiglu_fast(*args):
-    return (_small_swiglu_eager if _direct() else small_swiglu)(*args)
+def small_swiglu_fast(x, norm_w, eps, w_gate, w_up):
+    fn = _small_swiglu_eager if _direct(x, w_gate) else small_swiglu
+    return fn(x, norm_w, eps, w_gate, w_up)
 
 
-def silu_mul_fast(*args):
-    return (_silu_mul_eager if _direct() else silu_mul)(*args)
+def silu_mul_fast(gate_up, d_ff):
+    return (_silu_mul_eager if _direct(gate_up, gate_up) else silu_mul)(gate_up, d_ff)
+
+
+def rmsnorm_fast(x, weight, eps):
+    return (_rmsnorm_eager if _direct(x, weight) else rmsnorm)(x, weight, eps)[0]

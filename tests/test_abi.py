@@ -264,6 +264,37 @@ def test_custom_op_fake_kernels_give_output_shapes():
         assert out.shape == (2, 3, 4, 10)
 
 
+def test_module_calls_under_a_dispatch_mode_go_through_the_ops():
+    """Eager calls without autograd skip the dispatcher only for plain tensors outside any mode
+    or transform: under FakeTensorMode the modules still give shapes (no kernel, no GPU), and
+    the predicate is false in vmap, forward-mode AD, function modes, autograd, and for
+    subclasses."""
+    import torch
+    import mamba3_amd
+    from mamba3_amd import ops
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    with FakeTensorMode(), torch.no_grad():
+        with torch.device("cuda"):
+            layer = mamba3_amd.KulaMamba(d_model=64, d_state=16, headdim=16, mimo_rank=2)
+            norm, x = mamba3_amd.RMSNorm(64), torch.empty(2, 5, 64)
+        y, st = layer.prefill(norm(x))
+        assert y.shape == x.shape and st["h"].shape == (2, layer.nheads, 16, 16)
+        out, st = layer.step(x[:, 0], st)
+        assert out.shape == (2, 64) and st["angle"].shape == (2, layer.nheads, 8)
+    t = torch.ones(3)
+    assert not ops._direct(t, t)
+    with torch.no_grad():
+        assert ops._direct(t, torch.nn.Parameter(t))
+        assert not ops._direct(t.as_subclass(type("Sub", (torch.Tensor,), {})), t)
+        seen = []
+        torch.func.vmap(lambda v: seen.append(ops._direct(t, t)) or v)(t)
+        with torch.autograd.forward_ad.dual_level():
+            seen.append(ops._direct(t, t))
+        with torch.device("cpu"):
+            seen.append(ops._direct(t, t))
+        assert seen == [False] * 3
+
+
 def test_noalloc_prefill_refuses_workspace_beyond_scratch_before_any_launch():
     """m3_prefill_fwd_noalloc rejects a workload whose workspace exceeds the static scratch
     on the host, before touching the device (so this runs without a GPU); the pointers
