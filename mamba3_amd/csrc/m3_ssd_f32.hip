@@ -8,29 +8,43 @@
 // Every operand stays fp32: the contractions run on v_mfma_f32_16x16x4_f32 (lane l supplies
 // A[l%16][l/16] and B[l/16][l%16]; it holds D[4(l/16)+v][l%16]).
 //
-// Two launches:
+// Launches:
 //   1. bc_norm_f32: per (token, group), B^ = RMSNorm(B) * w + bias and C^ likewise, fp32, in
 //      the reference's (n, r) order (mamba3/mamba3.py:19-35, 147-157).
-//   2. ssd_f32<PB>: one 512-thread workgroup (8 waves) per (batch, head, block of PB of the 64
-//      headdim columns) walks the sequence in chunks of Q = 32 tokens (rows (t, r) = 2t + r,
-//      64 rows), carrying its columns of the fp32 state H^T [n][p] in MFMA accumulators (wave
-//      w owns rows n = 16w .. 16w+15). PB = 32 when the (batch, head) pairs alone leave CUs
-//      idle: two workgroups per pair then repeat the scores and the rotation. Per chunk:
-//        prep   token scalars; X rows x_u mimo_x[r] and z into LDS; the state copy H;
-//               the RoPE angles (a prefix over 8 groups of 4 tokens per pair) and the
-//               rotated C~ / B~ tiles (mamba3/mamba3.py:38-45, 160-166)
-//        G1     S = (C~ B~^T) * Lc on the 10 causal 16 x 16 blocks, into LDS, with
-//               Lc[t][u] = [u<=t] exp(c_t - c_u) (a_u + [u<t] b_u) and D on the diagonal
-//        G3+G2  Y = diag(e^{c_t}) C~ H^T + S X (waves: 16-row block w/2, PB/2 columns)
-//        G4     H^T = e^{c_end} H^T + (B~ diag(w))^T X, w_u = e^{c_end - c_u} (a_u + b_u)
-//        gate   out = sum_r mimo_down_r silu(z mimo_z_r) y_r (mamba3/mamba3.py:233-239)
-//      The angles stay absolute (the walk starts at t = 0), so the final state, angle and
-//      prev_BX = B~_{T-1} x_r,{T-1}^T need no frame change (mamba3/mamba3.py:241-256).
-//      For the training forward (M3_FLAG_FOR_BACKWARD) the walk also stores, from the
-//      values it holds, the per-token operands the layer backward reads, in the staged
-//      fp32 layer path's layouts (m3_layer_fp32.hip), instead of that path's five launches.
-// LDS rows have odd strides (in 32-bit words), so the column reads of the MFMA operands (16
-// lanes on 16 rows) hit distinct banks.
+//   2. with few (batch, head) pairs (seg_plan), ssd_f32<false>: a state-only walk of every
+//      segment of the sequence but the last, from a zero state in its own RoPE frame, and
+//      seg_combine_f32, which turns the end states into the states entering each segment;
+//   3. ssd_f32<true>: one 768-thread workgroup per (batch, head, segment) walks its chunks of
+//      Q = 32 tokens (64 rows (t, r) = 2t + r).
+//
+// Waves 0-3 are column waves: each carries its 16 headdim columns of the fp32 state H^T [n][p]
+// in MFMA accumulators and computes their outputs. Waves 4-11 are helpers: they compute the
+// scores and prepare the next chunk's tiles. Per chunk, two phases with a barrier after each:
+//   scores    column waves  G3  Y = diag(e^{c_t}) C~ H^T (H^T straight from the accumulators:
+//                               accumulator v of lane group g is row n = 16 t + 4 g + v, the
+//                               contraction slot of MFMA step v, whose C~ operands are one
+//                               128-bit read for four steps)
+//             helpers       X^T; G1  S = (C~ B~^T) * Lc on the 10 causal 16 x 16 blocks,
+//                               Lc[t][u] = [u<=t] exp(c_t - c_u) (a_u + [u<t] b_u), D on the diagonal;
+//                           the next chunk's angle sums, the token scalars of the one after it
+//   update    column waves  G2  Y += S X, out = sum_r mimo_down_r silu(z mimo_z_r) y_r
+//                               (mamba3/mamba3.py:233-239)
+//                           G4  H^T = e^{c_end} H^T + B~^T (diag(w) X), w_u = e^{c_end - c_u} (a_u + b_u)
+//             helpers       angles and rotated C~ / B~ tiles (mamba3/mamba3.py:38-45, 160-166) of
+//                           the next chunk
+// B~ is kept twice (G4 reads it while the helpers write the next chunk's), which balances the
+// phases: 208-224 MFMAs per SIMD in the first, 168 in the second.
+// For the training forward (M3_FLAG_FOR_BACKWARD) the walk also stores, from the values it
+// holds, the per-token operands the layer backward reads, in the staged fp32 layer path's
+// layouts (m3_layer_fp32.hip), and its chunk-start states.
+//
+// Bound by SIMD issue: 1,500 v_mfma_f32_16x16x4_f32 of 32 cycles per chunk are 12K cycles on
+// four SIMDs, and the helpers' VALU work (about 4K) and the phase tails do not hide under them:
+// 19.7K measured, 8.2 us per chunk and workgroup. d_model 768 over 4 x 1024 tokens (96 (batch,
+// head) pairs): 300 us with two workgroups of 32 columns per pair, state and operands through
+// LDS, all eight waves in step; 212 us with this split (135 + 70 state pass + 7).
+#include <algorithm>
+
 #include "m3_common.h"
 #include "m3_kernels.h"
 #include "m3_mfma.h"
@@ -45,22 +59,37 @@ constexpr int R = 2;
 constexpr int NR = N * R;
 constexpr int NH = N / 2;
 constexpr int ROWS = Q * R;
-constexpr int THREADS = 512;
-constexpr int CST = N + 1;
-constexpr int SST = ROWS + 1;
+constexpr int CW = 4, HW = 8;         // column and helper waves
+constexpr int HT = 64 * HW;
+constexpr int THREADS = 64 * (CW + HW);
+constexpr int LPT = N / 4;            // helper lanes per token: two RoPE pairs each
+constexpr int GR = HT / LPT;          // token groups of a chunk
+constexpr int TPT = Q / GR;           // tokens per group
+constexpr int XTOK = Q * P / HT;      // X elements per helper thread: consecutive tokens of one column
+constexpr int NT = N / 16;            // state row tiles
+// LDS row strides of 4 (mod 64) words: the 128-bit operand reads of 16 rows and the 32-bit
+// reads of 16 columns in rows 4 apart (G4) each touch every bank once.
+constexpr int CST = N + 4;
+constexpr int SST = ROWS + 4;
 
-template <int PB>
-struct Smem {
-    float C[ROWS][CST];      // C~ rows (t, r)
-    float B[ROWS][CST];      // B~ rows (u, r)
-    float X[ROWS][PB + 1];   // x_u mimo_x[p, r], rows (u, r), this block's columns
-    float S[ROWS][SST];      // masked scores, rows (t, r), columns (u, r')
-    float H[N][PB + 1];      // state H^T at the chunk start, this block's columns
-    float Z[Q][PB];          // z
-    float part[8][NH];       // per 4-token group: sum of dt theta, per pair
-    float phi_run[2][NH];    // pair angles at the end of the previous chunk (by chunk parity)
-    float dtv[Q + 1], lamv[Q + 1];  // dt and lambda of the chunk's tokens and the next one
-    float c[Q], ec[Q], av[Q], bv[Q], w[Q];
+struct Tok {
+    float c[Q];   // inclusive prefix of A dt over the chunk
+    float ec[Q];  // exp(c_t)
+    float av[Q], bv[Q];  // a_u = lambda_u dt_u, b_u = (1 - lambda_{u+1}) dt_{u+1}
+    float w[Q];   // exp(c_end - c_u) (a_u + b_u)
+    float dt[Q], lam[Q];
+    float sb[Q];  // (1 - lambda_{u+1}) exp(A dt_{u+1}): x_b of the next token over x_r of this one
+    float cend;
+};
+
+template <bool FULL>
+struct __align__(16) Smem {
+    float B[2][ROWS][CST];             // B~ rows (u, r), by chunk parity
+    float C[FULL ? ROWS : 1][CST];     // C~ rows (t, r)
+    float XT[P][SST];                  // x_u mimo_x[p, r], [p][(u, r)]
+    float S[FULL ? ROWS : 1][SST];     // masked scores, rows (t, r), columns (u, r')
+    float part[GR][NH];                // sum of dt theta per token group, per pair
+    Tok tok[3];                        // by chunk mod 3
 };
 
 struct Args {
@@ -86,7 +115,21 @@ struct Args {
     // backward's chunking: the state entering every hs_every-th chunk k at entry k / hs_every
     // of (B, hs_K + 1, H, P, N) (the zero start at entry 0), and the final state at entry hs_K.
     int hs_every, hs_K;
+    // segments of the sequence (segs = 1: none) and the state pass's results, per segment but
+    // the last and (batch, head): end state [wave][tile][lane] (seg_combine_f32 turns it into
+    // the state entering the next segment), log-decay, RoPE angle increments
+    int segs;
+    f32x4* hseg;
+    float* lseg;
+    float* aseg;
 };
+
+// First token of segment i: four segments each of kSeg0, 2 kSeg0 and 4 kSeg0 tokens, then 16 kSeg0.
+constexpr int kSeg0 = 128;
+__host__ __device__ inline int64_t seg_start(int i) {
+    const int u = i <= 4 ? i : i <= 8 ? 4 + 2 * (i - 4) : i <= 12 ? 12 + 4 * (i - 8) : 28 + 16 * (i - 12);
+    return (int64_t)u * kSeg0;
+}
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -137,345 +180,648 @@ __global__ __launch_bounds__(256) void bc_norm_f32(const float* __restrict__ pro
     *reinterpret_cast<f32x4*>(Cn + tg * NR + e) = oc;
 }
 
-template <int PB>
-__global__ __launch_bounds__(THREADS, 1) void ssd_f32(Args a) {
-    constexpr int NPT = PB / 16;          // column tiles of the block
-    constexpr int TPW = NPT / 2;          // output tiles per wave (row block wave / 2)
-    constexpr int XE = PB * Q / THREADS;  // X / Z elements per thread
-    constexpr int NPE = PB * N / THREADS; // prev_BX elements per thread
-    __shared__ Smem<PB> sm;
-    const int tid = threadIdx.x;
-    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63;
-    const int l16 = lane & 15, g4 = lane >> 4;
+__device__ __forceinline__ float ld_b32(const __amdgpu_buffer_rsrc_t& r, int off, int so) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, so, 0));
+}
+__device__ __forceinline__ f32x4 ld_b128(const __amdgpu_buffer_rsrc_t& r, int off, int so) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, so, 0));
+}
 
-    // XCD-aware order: consecutive workgroups of one batch row land on one XCD.
-    const int nblk = gridDim.x;
-    const int blk = (nblk % 8 == 0) ? (blockIdx.x % 8) * (nblk / 8) + blockIdx.x / 8 : blockIdx.x;
-    const int bh = blk / (P / PB);
-    const int pc = (blk % (P / PB)) * PB;  // first headdim column of the block
+// sin and cos of |x| <= kSincosMax: x minus the nearest multiple of pi/2, in three steps of a
+// split pi/2 (Cody and Waite), then the Cephes library's minimax polynomials on [-pi/4, pi/4].
+// Straight-line, so that a thread's angles interleave; sincosf spends about four times the
+// cycles on its range branches. Largest error over the range 7.1e-8, rms 1.7e-8 (float rounding
+// of the exact value: 6e-8, 1.5e-8).
+constexpr float kSincosMax = 1e5f;
+__device__ __forceinline__ void sincos_small(float x, float& s, float& c) {
+    const float k = rintf(x * 0.636619772f);
+    float r = fmaf(-k, 1.57079637e+00f, x);
+    r = fmaf(-k, -4.37113883e-08f, r);
+    r = fmaf(-k, -1.71512451e-15f, r);
+    const float r2 = r * r;
+    float p = fmaf(r2, -1.9515295891e-4f, 8.3321608736e-3f);
+    p = fmaf(p, r2, -1.6666654611e-1f);
+    const float sr = fmaf(p * r2, r, r);
+    float q = fmaf(r2, 2.443315711809948e-5f, -1.388731625493765e-3f);
+    q = fmaf(q, r2, 4.166664568298827e-2f);
+    q = fmaf(q, r2, -0.5f);
+    const float cr = fmaf(q, r2, 1.f);
+    const int n = (int)k;
+    const unsigned ss = n & 1 ? __builtin_bit_cast(unsigned, cr) : __builtin_bit_cast(unsigned, sr);
+    const unsigned cc = n & 1 ? __builtin_bit_cast(unsigned, sr) : __builtin_bit_cast(unsigned, cr);
+    s = __builtin_bit_cast(float, ss ^ ((unsigned)(n & 2) << 30));
+    c = __builtin_bit_cast(float, cc ^ ((unsigned)((n + 1) & 2) << 30));
+}
+
+template <bool FULL>
+__global__ __launch_bounds__(THREADS, 3) void ssd_f32(Args a) {
+    __shared__ Smem<FULL> sm;
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int l16 = lane & 15, g16 = lane >> 4;
+    const int npairs = a.B * a.H;
+    // Segments longest first; within one, consecutive (batch, head) pairs share an XCD.
+    const int j0 = blockIdx.x % npairs;
+    const int seg = (FULL ? a.segs : a.segs - 1) - 1 - (int)(blockIdx.x / npairs);
+    const int bh = (npairs % 8 == 0) ? (j0 % 8) * (npairs / 8) + j0 / 8 : j0;
     const int b = bh / a.H, h = bh % a.H;
     const int grp = h / (a.H / a.G);
     const int T = a.T;
-    const int K = (T + Q - 1) / Q;
-    const int HP = a.H * P;
-
+    const int tbeg = (int)seg_start(seg);
+    const int tend = seg + 1 < a.segs ? (int)seg_start(seg + 1) : T;
+    const int K = (tend - tbeg + Q - 1) / Q;
+    const int k0 = tbeg / Q;              // the segment's first chunk in the sequence
+    const int KT = (T + Q - 1) / Q;
     const float Ah = -expf(a.prm.A_log[h]);
-    const float Dh = a.prm.D[h];
-    const float dtb = a.prm.dt_bias[h];
-    const float* prow = a.proj + (int64_t)b * T * a.rs;
+    const float* proj = a.proj + (int64_t)b * T * a.rs;
+    const int rb = (int)a.rs * 4;         // bytes of a proj row
+    // Reads of a chunk go through buffer resources that start at its first token and end at the
+    // sequence's last: tokens past the end read as zero.
+    auto chunk_rsrc = [&](const void* base, int kk, int64_t row_bytes) {
+        const int64_t s0 = tbeg + (int64_t)kk * Q;
+        return make_rsrc(reinterpret_cast<const char*>(base) + (s0 < T ? s0 * row_bytes : 0),
+                         s0 < T ? (T - s0) * row_bytes : 0);
+    };
 
-    // prep roles: X / Z element block (token xu, block columns xp .. xp + XE - 1), and the
-    // rotation job (tokens 4 wv .. 4 wv + 3 of pair lane)
-    const int xu = tid >> 4, xp = XE * (tid & 15);
-    float mx0[XE], mx1[XE];
+    if (wave < CW) {
+        // =============================== column waves ===============================
+        const int p = 16 * wave + l16;
+        f32x4 hacc[NT];
 #pragma unroll
-    for (int j = 0; j < XE; ++j) {
-        mx0[j] = a.prm.mimo_x[(h * P + pc + xp + j) * R];
-        mx1[j] = a.prm.mimo_x[(h * P + pc + xp + j) * R + 1];
-    }
-    // output roles: row block I, block column tiles ptb .. ptb + TPW - 1
-    const int I = wv >> 1;
-    const int ptb = TPW * (wv & 1);
-    float mz[TPW][2], md[TPW][2];
+        for (int t = 0; t < NT; ++t) hacc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (FULL && seg > 0) {
+            const f32x4* hs = a.hseg + (((int64_t)(seg - 1) * npairs + bh) * CW + wave) * (NT * 64) + lane;
 #pragma unroll
-    for (int q = 0; q < TPW; ++q)
+            for (int t = 0; t < NT; ++t) hacc[t] = hs[t * 64];
+        }
+        float mz[R], md[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const int p = pc + 16 * (ptb + q) + l16;
-            mz[q][r] = a.prm.mimo_z[(h * P + p) * R + r];
-            md[q][r] = a.prm.mimo_down[(h * P + p) * R + r];
+            mz[r] = a.prm.mimo_z[(h * P + p) * R + r];
+            md[r] = a.prm.mimo_down[(h * P + p) * R + r];
         }
-    if (tid < NH) sm.phi_run[0][tid] = 0.f;
-    const bool st_head = a.stage && pc == 0;  // per-(token, head) operands: one block writes them
-    if (st_head && tid == 0) a.st.A[h] = Ah;
+        // chunk-start states for the layer backward: entry e of (B, hs_K + 1, H, P, N), this
+        // lane's column
+        auto hs_entry = [&](int e) {
+            return a.st.Hs + (((int64_t)b * (a.hs_K + 1) + e) * a.H + h) * (P * N) + (int64_t)p * N + 4 * g16;
+        };
+        if (FULL && a.hs_every > 0 && seg == 0) {  // the zero start state
+            float* hk = hs_entry(0);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(hk + 16 * t) = hacc[t];
+        }
+        float ldec = 0.f;  // log of the segment's decay (state pass)
+        __syncthreads();  // token scalars of chunks 0 and 1
+        __syncthreads();  // angle sums of chunk 0
+        __syncthreads();  // tiles of chunk 0
 
-    f32x4 hacc[NPT];
+        for (int k = 0; k < K; ++k) {
+            const int s0 = tbeg + k * Q;
+            const Tok& tk = sm.tok[k % 3];
+            const float (&sB)[ROWS][CST] = sm.B[k & 1];
+            // ---- scores ----
+            float zv[FULL ? 4 : 1][2];
+            f32x4 y[FULL ? 4 : 1], gz[FULL ? 4 : 1];
+            if constexpr (FULL) {
+                const __amdgpu_buffer_rsrc_t rp = chunk_rsrc(proj, k, rb);
+                const int zoff = 2 * g16 * rb + ((int)a.pl.z + h * P + p) * 4;
 #pragma unroll
-    for (int pt = 0; pt < NPT; ++pt) hacc[pt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // Raw reads of one chunk (tokens past T read nothing and keep zeros): dt / lambda /
-    // dt_scale of token tid (tid <= Q, one past the chunk for b_u), x and z of token xu, and
-    // the B^ / C^ rows and theta of tokens 4 wv .. 4 wv + 3, pair lane. Issued a chunk ahead.
-    float rdt = 0.f, rlam = 0.f, rsc = 1.f;
-    float xv[XE], zv[XE];
-    f32x4 rb[4], rc[4];
-    float th[4];
-    auto load_chunk = [&](int kk) {
-        const int s0n = kk * Q;
-        if (tid <= Q && s0n + tid < T) {
-            const float* pr = prow + (int64_t)(s0n + tid) * a.rs;
-            rdt = pr[a.pl.dt + h];
-            if (a.trap) rlam = pr[a.pl.lam + h];
-            if (a.dt_scale) rsc = a.dt_scale[((int64_t)b * T + s0n + tid) * a.H + h];
-        }
-#pragma unroll
-        for (int j = 0; j < XE; ++j) xv[j] = zv[j] = 0.f;
-        if (s0n + xu < T) {
-            const float* pr = prow + (int64_t)(s0n + xu) * a.rs + h * P + pc + xp;
-#pragma unroll
-            for (int j = 0; j < XE; ++j) {
-                xv[j] = pr[a.pl.x + j];
-                zv[j] = pr[a.pl.z + j];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int tok = s0n + 4 * wv + j;
-            rb[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            rc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            th[j] = 0.f;
-            if (tok < T) {
-                const int64_t row = (((int64_t)b * T + tok) * a.G + grp) * NR + 4 * lane;
-                rb[j] = *reinterpret_cast<const f32x4*>(a.Bn + row);
-                rc[j] = *reinterpret_cast<const f32x4*>(a.Cn + row);
-                if (a.cplx) th[j] = prow[(int64_t)tok * a.rs + a.pl.theta + lane];
-            }
-        }
-    };
-    load_chunk(0);
-
-    for (int k = 0; k < K; ++k) {
-        const int s0 = k * Q;
-        const int par = k & 1;
-        __syncthreads();  // the previous chunk's tiles are consumed
-        // ---- prep 1: token scalars, X / Z rows and the state copy into LDS, from the raw
-        // reads issued during the previous chunk's contractions
-        if (tid <= Q) {
-            float dt = 0.f, lam = 1.f;
-            if (s0 + tid < T) {
-                dt = softplus_f(rdt + dtb) * rsc;
-                if (a.trap) lam = sigmoid_f(rlam);
-            }
-            sm.dtv[tid] = dt;
-            sm.lamv[tid] = lam;
-            if (st_head && tid < Q && s0 + tid < T) a.st.dt[((int64_t)b * T + s0 + tid) * a.H + h] = dt;
-        }
-#pragma unroll
-        for (int j = 0; j < XE; ++j) {
-            sm.X[2 * xu][xp + j] = xv[j] * mx0[j];
-            sm.X[2 * xu + 1][xp + j] = xv[j] * mx1[j];
-            sm.Z[xu][xp + j] = zv[j];
-        }
-#pragma unroll
-        for (int pt = 0; pt < NPT; ++pt)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) sm.H[16 * wv + 4 * g4 + v][16 * pt + l16] = hacc[pt][v];
-        if (a.hs_every > 0 && k == 0) {  // the zero start state
-            float* hk = a.st.Hs + ((int64_t)b * (a.hs_K + 1) * a.H + h) * (P * N) + (int64_t)pc * N;
-#pragma unroll
-            for (int pt = 0; pt < NPT; ++pt)
-                *reinterpret_cast<f32x4*>(&hk[(16 * pt + l16) * N + 16 * wv + 4 * g4]) = hacc[pt];
-        }
-        __syncthreads();
-        if (a.stage && s0 + xu < T) {
-            // x_r, x_g = lambda_t x_r and x_b of the next token = (1 - lambda_{t+1})
-            // exp(A dt_{t+1}) x_r (mamba3/mamba3.py:210-224), this thread's X elements
-            const int64_t e0 = (((int64_t)b * T + s0 + xu) * a.H + h) * (P * R) + (int64_t)(pc + xp) * R;
-            const float lam = sm.lamv[xu];
-            const float sbn = a.trap ? (1.f - sm.lamv[xu + 1]) * expf(Ah * sm.dtv[xu + 1]) : 0.f;
-#pragma unroll
-            for (int j = 0; j < XE; ++j) {
-                const f32x2 xr = f32x2{xv[j] * mx0[j], xv[j] * mx1[j]};
-                *reinterpret_cast<f32x2*>(a.st.xr + e0 + j * R) = xr;
-                *reinterpret_cast<f32x2*>(a.st.xg + e0 + j * R) = xr * lam;
-                if (a.trap) {
-                    if (s0 + xu + 1 < T) *reinterpret_cast<f32x2*>(a.st.xb + e0 + (int64_t)a.H * P * R + j * R) = xr * sbn;
-                    if (s0 + xu == 0) *reinterpret_cast<f32x2*>(a.st.xb + e0 + j * R) = f32x2{0.f, 0.f};
+                for (int tt = 0; tt < 4; ++tt) {
+                    zv[tt][0] = ld_b32(rp, zoff, 8 * tt * rb);
+                    zv[tt][1] = ld_b32(rp, zoff, (8 * tt + 1) * rb);
+                    y[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
-            }
-        }
-        // ---- prep 2: chunk scalars (wave 0, lane = token: a prefix scan of A dt) and the
-        // angle partial sums
-        if (wv == 0) {
-            const bool in = lane < Q;
-            const float dt = in ? sm.dtv[lane] : 0.f;
-            const float c = wave_incl_scan(Ah * dt);
-            const float cend = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c), Q - 1));
-            if (in) {
-                const float av = a.trap ? sm.lamv[lane] * dt : dt;
-                const float bv = a.trap ? (1.f - sm.lamv[lane + 1]) * sm.dtv[lane + 1] : 0.f;
-                sm.c[lane] = c;
-                sm.ec[lane] = exp_hw(c);
-                sm.av[lane] = av;
-                sm.bv[lane] = bv;
-                sm.w[lane] = exp_hw(cend - c) * (av + bv);
-            }
-        }
-        {
-            float ps = 0.f;
+                f32x4 A[2][4];
+                auto load_c = [&](int t) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) ps += sm.dtv[4 * wv + j] * th[j];
-            sm.part[wv][lane] = ps;
-        }
-        __syncthreads();
-        // ---- prep 3: angles and the rotated C~ / B~ rows of tokens 4 wv .. 4 wv + 3, pair lane
-        {
-            float phi = sm.phi_run[par][lane];
-            for (int g = 0; g < wv; ++g) phi -= sm.part[g][lane];
+                    for (int tt = 0; tt < 4; ++tt) A[t & 1][tt] = *reinterpret_cast<const f32x4*>(&sm.C[16 * tt + l16][16 * t + 4 * g16]);
+                };
+                load_c(0);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int t = 4 * wv + j;
-                phi -= sm.dtv[t] * th[j];
-                float sn, cs;
-                sincosf(phi, &sn, &cs);
-                f32x4 bt, ct;  // (n=2i, r0) (2i, r1) (2i+1, r0) (2i+1, r1)
+                for (int t = 0; t < NT; ++t) {
+                    if (t + 1 < NT) load_c(t + 1);
+                    M3_FENCE();
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    // pair lane holds (n=2i, r0) (2i, r1) (2i+1, r0) (2i+1, r1)
-                    const float be = rb[j][r], bo = rb[j][2 + r];
-                    const float ce = rc[j][r], co = rc[j][2 + r];
-                    bt[r] = be * cs - bo * sn;
-                    bt[2 + r] = be * sn + bo * cs;
-                    ct[r] = ce * cs - co * sn;
-                    ct[2 + r] = ce * sn + co * cs;
-                    sm.B[2 * t + r][2 * lane] = bt[r];
-                    sm.B[2 * t + r][2 * lane + 1] = bt[2 + r];
-                    sm.C[2 * t + r][2 * lane] = ct[r];
-                    sm.C[2 * t + r][2 * lane + 1] = ct[2 + r];
+                    for (int v = 0; v < 4; ++v)
+#pragma unroll
+                        for (int tt = 0; tt < 4; ++tt) y[tt] = mfma4(A[t & 1][tt][v], hacc[t][v], y[tt]);
                 }
-                if (st_head && s0 + t < T) {
-                    const int64_t tk = ((int64_t)b * T + s0 + t) * a.H + h;
-                    *reinterpret_cast<f32x4*>(a.st.Bt + tk * NR + 4 * lane) = bt;
-                    *reinterpret_cast<f32x4*>(a.st.Ct + tk * NR + 4 * lane) = ct;
-                    if (a.trap) {
-                        if (s0 + t + 1 < T) *reinterpret_cast<f32x4*>(a.st.Bb + (tk + a.H) * NR + 4 * lane) = bt;
-                        if (s0 + t == 0) *reinterpret_cast<f32x4*>(a.st.Bb + tk * NR + 4 * lane) = f32x4{0.f, 0.f, 0.f, 0.f};
+                // gate factors of the two ranks
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const float z = zv[tt][q];
+                        gz[tt][2 * q] = md[0] * silu_hw(z * mz[0]);
+                        gz[tt][2 * q + 1] = md[1] * silu_hw(z * mz[1]);
                     }
-                    a.st.phi[tk * NH + lane] = phi;
+#pragma unroll
+                for (int tt = 0; tt < 4; ++tt) {
+                    const f32x2 e = *reinterpret_cast<const f32x2*>(&tk.ec[8 * tt + 2 * g16]);
+                    y[tt][0] *= e[0];
+                    y[tt][1] *= e[0];
+                    y[tt][2] *= e[1];
+                    y[tt][3] *= e[1];
                 }
             }
-            if (wv == 7) sm.phi_run[par ^ 1][lane] = phi;
-        }
-        if (k + 1 < K) load_chunk(k + 1);  // consumed by the next chunk's prep
-        __syncthreads();
-        // ---- G1: masked scores of the causal blocks (I, J), J <= I; wave w takes blocks w
-        // and w + 8 of the list (0,0) (1,0) (1,1) (2,0) (2,1) (2,2) (3,0) (3,1) (3,2) (3,3)
-        for (int blk = wv; blk < 10; blk += 8) {
-            const int bI = blk < 1 ? 0 : blk < 3 ? 1 : blk < 6 ? 2 : 3;
-            const int bJ = blk - (bI * (bI + 1)) / 2;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-            for (int k0 = 0; k0 < N; k0 += 4)
-                acc = mfma4(sm.C[16 * bI + l16][k0 + g4], sm.B[16 * bJ + l16][k0 + g4], acc);
-            const int col = 16 * bJ + l16;
-            const int u = col >> 1, rp = col & 1;
-            const float cu = sm.c[u], au = sm.av[u], bu = sm.bv[u];
+            M3_FENCE();
+            __syncthreads();
+            // ---- update ----
+            f32x4 X[4];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = 16 * bI + 4 * g4 + v;
-                const int t = row >> 1, r = row & 1;
-                float s = 0.f;
-                if (u <= t) {
-                    s = acc[v] * exp_hw(sm.c[t] - cu) * (au + (u < t ? bu : 0.f));
-                    if (u == t && r == rp) s += Dh;
+            for (int s = 0; s < 4; ++s) X[s] = *reinterpret_cast<const f32x4*>(&sm.XT[p][16 * s + 4 * g16]);
+            if constexpr (FULL) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    f32x4 A[4];
+#pragma unroll
+                    for (int tt = s; tt < 4; ++tt) A[tt] = *reinterpret_cast<const f32x4*>(&sm.S[16 * tt + l16][16 * s + 4 * g16]);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+#pragma unroll
+                        for (int tt = s; tt < 4; ++tt) y[tt] = mfma4(A[tt][v], X[s][v], y[tt]);
                 }
-                sm.S[row][col] = s;
-            }
-        }
-        __syncthreads();
-        // ---- G3 + G2: output rows 16 I .. 16 I + 15, block columns 16 (ptb + q) + l16
-        f32x4 yacc[TPW];
+                // gate and MIMO-down: rows 4 g16 + 2 q + r of row block tt are (t, r); stores past
+                // the sequence's end fall outside the resource
+                const __amdgpu_buffer_rsrc_t ro = chunk_rsrc(a.y_out + (int64_t)b * T * a.H * P, k, (int64_t)a.H * P * 4);
+                const int ob = a.H * P * 4, ooff = 2 * g16 * ob + (h * P + p) * 4;
 #pragma unroll
-        for (int q = 0; q < TPW; ++q) yacc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const float o = gz[tt][2 * q] * y[tt][2 * q] + gz[tt][2 * q + 1] * y[tt][2 * q + 1];
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, o), ro, ooff, (8 * tt + q) * ob, 0);
+                    }
+            }
+            {
+                const float dec = tk.ec[Q - 1];
+                if constexpr (!FULL) ldec += tk.cend;
+#pragma unroll
+                for (int t = 0; t < NT; ++t) hacc[t] *= dec;
+                // rows 4 g16 + v of k-step i = 4 s + v
+                float A[2][NT], xw[4][4];
+                auto load_b = [&](int i) {
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) A[i & 1][t] = sB[16 * (i / 4) + 4 * g16 + i % 4][16 * t + l16];
+                };
+                load_b(0);
+#pragma unroll
+                for (int s = 0; s < 4; ++s) {
+                    const f32x2 w = *reinterpret_cast<const f32x2*>(&tk.w[8 * s + 2 * g16]);
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) xw[s][v] = X[s][v] * w[v / 2];
+                }
+#pragma unroll
+                for (int i = 0; i < ROWS / 4; ++i) {
+                    if (i + 1 < ROWS / 4) load_b(i + 1);
+                    M3_FENCE();
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) hacc[t] = mfma4(A[i & 1][t], xw[i / 4][i % 4], hacc[t]);
+                }
+            }
+            if constexpr (FULL) {
+                if (a.stage) {
+#pragma unroll
+                    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q) {
+                            const int st = s0 + 8 * tt + 2 * g16 + q;
+                            if (st < T)
+                                *reinterpret_cast<f32x2*>(a.st.ys + ((((int64_t)b * T + st) * a.H + h) * P + p) * R) =
+                                    f32x2{y[tt][2 * q], y[tt][2 * q + 1]};
+                        }
+                }
+            }
+            // The state entering the next chunk for the layer backward. The walk folds the beta
+            // term of the next chunk's first token into this chunk (b_{Q-1} B~_{Q-1} x_{Q-1}^T); the
+            // chunk kernels count it in the next chunk, so it is taken out of the stored state
+            // (b = 0 without the trapezoid).
+            if (FULL && a.hs_every > 0 && (k0 + k + 1) % a.hs_every == 0 && k0 + k + 1 < KT) {
+                const float bq = tk.bv[Q - 1];
+                const float x0 = bq * sm.XT[p][2 * (Q - 1)], x1 = bq * sm.XT[p][2 * (Q - 1) + 1];
+                float* hk = hs_entry((k0 + k + 1) / a.hs_every);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const f32x4 b0 = *reinterpret_cast<const f32x4*>(&sB[2 * (Q - 1)][16 * t + 4 * g16]);
+                    const f32x4 b1 = *reinterpret_cast<const f32x4*>(&sB[2 * (Q - 1) + 1][16 * t + 4 * g16]);
+                    *reinterpret_cast<f32x4*>(hk + 16 * t) = hacc[t] - (b0 * x0 + b1 * x1);
+                }
+            }
+            __syncthreads();
+        }
+        if constexpr (FULL) {
+            if (tend == T) {
+                if (a.hs_every > 0) {
+                    float* hk = hs_entry(a.hs_K);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(hk + 16 * t) = hacc[t];
+                }
+                if (a.h_final) {
+                    float* hf = a.h_final + (int64_t)bh * P * N + (int64_t)p * N + 4 * g16;
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4*>(hf + 16 * t) = hacc[t];
+                }
+            }
+        } else {
+            f32x4* hs = a.hseg + (((int64_t)seg * npairs + bh) * CW + wave) * (NT * 64) + lane;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) hs[t * 64] = hacc[t];
+            if (wave == 0 && lane == 0) a.lseg[(int64_t)seg * npairs + bh] = ldec;
+        }
+    } else {
+        // =============================== helper waves ===============================
+        const int hw = wave - CW, htid = tid - 64 * CW;
+        const float Dh = a.prm.D[h];
+        const float dtb = a.prm.dt_bias[h];
+        const int64_t nrs = (int64_t)a.G * NR;  // B^ / C^ token stride
+        const int nb = (int)nrs * 4;
+        const float* Bn = a.Bn + (int64_t)b * T * nrs + (int64_t)grp * NR;
+        const float* Cn = a.Cn + (int64_t)b * T * nrs + (int64_t)grp * NR;
+        const bool stage = FULL && a.stage;
+        if (stage && htid == 0) a.st.A[h] = Ah;
+        // rotation jobs: RoPE pairs 2 hl, 2 hl + 1 (columns 4 hl ..) of tokens tg TPT + m; a pair's
+        // words are (n=2i, r0) (2i, r1) (2i+1, r0) (2i+1, r1)
+        const int hl = lane % LPT, tg = htid / LPT;
+        f32x4 pb[TPT][2], pc[FULL ? TPT : 1][2];
+        auto load_bc = [&](int kk) {
+            const int off = tg * TPT * nb + 32 * hl;
+            const __amdgpu_buffer_rsrc_t r = chunk_rsrc(Bn, kk, nb);
+#pragma unroll
+            for (int m = 0; m < TPT; ++m) {
+                pb[m][0] = ld_b128(r, off, m * nb);
+                pb[m][1] = ld_b128(r, off + 16, m * nb);
+            }
+            if constexpr (FULL) {
+                const __amdgpu_buffer_rsrc_t rc = chunk_rsrc(Cn, kk, nb);
+#pragma unroll
+                for (int m = 0; m < TPT; ++m) {
+                    pc[m][0] = ld_b128(rc, off, m * nb);
+                    pc[m][1] = ld_b128(rc, off + 16, m * nb);
+                }
+            }
+        };
+        // X jobs: column xp, tokens xt0 .. xt0 + XTOK - 1
+        const int xp = htid % P, xt0 = (htid / P) * XTOK;
+        const float mx0 = a.prm.mimo_x[(h * P + xp) * R], mx1 = a.prm.mimo_x[(h * P + xp) * R + 1];
+        float pxv[XTOK];
+        auto load_xv = [&](int kk) {
+            const __amdgpu_buffer_rsrc_t r = chunk_rsrc(proj, kk, rb);
+            const int off = xt0 * rb + ((int)a.pl.x + h * P + xp) * 4;
+#pragma unroll
+            for (int m = 0; m < XTOK; ++m) pxv[m] = ld_b32(r, off, m * rb);
+        };
+        f32x2 pth[TPT] = {};  // theta of the rotation jobs' pairs
+        auto load_theta = [&](int kk) {
+            if (!a.cplx) return;  // no theta columns
+            const __amdgpu_buffer_rsrc_t r = chunk_rsrc(proj, kk, rb);
+            const int off = tg * TPT * rb + ((int)a.pl.theta + 2 * hl) * 4;
+#pragma unroll
+            for (int m = 0; m < TPT; ++m) pth[m] = f32x2{ld_b32(r, off, m * rb), ld_b32(r, off + 4, m * rb)};
+        };
+        // token scalars: lane t = token t of the chunk (the last helper)
+        float rdt0 = 0.f, rdt1 = 0.f, rlam0 = 0.f, rlam1 = 0.f, sc0 = 1.f, sc1 = 1.f;
+        auto load_tokens = [&](int kk) {
+            const __amdgpu_buffer_rsrc_t r = chunk_rsrc(proj, kk, rb);
+            const int off = lane * rb + h * 4;
+            rdt0 = ld_b32(r, off, (int)a.pl.dt * 4);
+            rdt1 = ld_b32(r, off + rb, (int)a.pl.dt * 4);
+            if (a.trap) {
+                rlam0 = ld_b32(r, off, (int)a.pl.lam * 4);
+                rlam1 = ld_b32(r, off + rb, (int)a.pl.lam * 4);
+            }
+            if (a.dt_scale) {
+                const __amdgpu_buffer_rsrc_t rd = chunk_rsrc(a.dt_scale + (int64_t)b * T * a.H, kk, (int64_t)a.H * 4);
+                sc0 = ld_b32(rd, (lane * a.H + h) * 4, 0);
+                sc1 = ld_b32(rd, ((lane + 1) * a.H + h) * 4, 0);
+            }
+        };
+        auto prep_tokens = [&](int kk) {
+            const int s0 = tbeg + kk * Q, t = lane;
+            const bool v0 = t < Q && s0 + t < T, v1 = t < Q && s0 + t + 1 < T;
+            const float dt0 = v0 ? softplus_f(rdt0 + dtb) * sc0 : 0.f;
+            const float dt1 = v1 ? softplus_f(rdt1 + dtb) * sc1 : 0.f;
+            const float lam0 = v0 && a.trap ? sigmoid_f(rlam0) : 1.f;
+            const float lam1 = v1 && a.trap ? sigmoid_f(rlam1) : 1.f;
+            const float c = wave_incl_scan(Ah * dt0);
+            const float cend = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c), Q - 1));
+            Tok& tk = sm.tok[kk % 3];
+            if (t < Q) {
+                const float av = a.trap ? lam0 * dt0 : dt0;
+                const float bv = a.trap ? (1.f - lam1) * dt1 : 0.f;
+                tk.c[t] = c;
+                tk.ec[t] = exp_hw(c);
+                tk.av[t] = av;
+                tk.bv[t] = bv;
+                tk.w[t] = exp_hw(cend - c) * (av + bv);
+                tk.dt[t] = dt0;
+                tk.lam[t] = lam0;
+                tk.sb[t] = a.trap ? (1.f - lam1) * expf(Ah * dt1) : 0.f;
+                if (stage && v0 && s0 + t < tend) a.st.dt[((int64_t)b * T + s0 + t) * a.H + h] = dt0;
+            }
+            if (t == 0) tk.cend = cend;
+        };
+        // this thread's sums of dt theta over its token group, chunk kk
+        auto angle_sums = [&](int kk) {
+            if (!a.cplx) return;
+            const Tok& tk = sm.tok[kk % 3];
+            f32x2 ps = f32x2{0.f, 0.f};
+#pragma unroll
+            for (int m = 0; m < TPT; ++m) ps += pth[m] * tk.dt[tg * TPT + m];
+            *reinterpret_cast<f32x2*>(&sm.part[tg][2 * hl]) = ps;
+        };
+        f32x2 phi_run = f32x2{0.f, 0.f};  // pair angles at the start of the chunk to rotate next
+        if (FULL && a.cplx)
 #pragma unroll 4
-        for (int k0 = 0; k0 < N; k0 += 4) {
-            const float av = sm.C[16 * I + l16][k0 + g4];
+            for (int j = 0; j < seg; ++j)
+                phi_run += *reinterpret_cast<const f32x2*>(a.aseg + ((int64_t)j * npairs + bh) * NH + 2 * hl);
+        // sin / cos of chunk kk's pairs: phi_t[i] = phi_{t-1}[i] - dt_t theta_t[i]
+        // (mamba3/mamba3.py:160-162)
+        f32x2 cs[TPT], sn[TPT];
+        auto angles = [&](int kk) {
+            const Tok& tk = sm.tok[kk % 3];
+            f32x2 ph = phi_run;
+            if (a.cplx) {
+                f32x2 pp[GR], run = phi_run;
 #pragma unroll
-            for (int q = 0; q < TPW; ++q) yacc[q] = mfma4(av, sm.H[k0 + g4][16 * (ptb + q) + l16], yacc[q]);
-        }
+                for (int g = 0; g < GR; ++g) pp[g] = *reinterpret_cast<const f32x2*>(&sm.part[g][2 * hl]);
+                M3_FENCE();
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const float e = sm.ec[(16 * I + 4 * g4 + v) >> 1];
-#pragma unroll
-            for (int q = 0; q < TPW; ++q) yacc[q][v] *= e;
-        }
-        for (int k0 = 0; k0 < 16 * (I + 1); k0 += 4) {
-            const float sv = sm.S[16 * I + l16][k0 + g4];
-#pragma unroll
-            for (int q = 0; q < TPW; ++q) yacc[q] = mfma4(sv, sm.X[k0 + g4][16 * (ptb + q) + l16], yacc[q]);
-        }
-        // ---- G4: state update on this wave's rows n = 16 wv .. 16 wv + 15
-        {
-            const float dec = sm.ec[Q - 1];
-#pragma unroll
-            for (int pt = 0; pt < NPT; ++pt) hacc[pt] *= dec;
-#pragma unroll 4
-            for (int k0 = 0; k0 < ROWS; k0 += 4) {
-                const float bw = sm.B[k0 + g4][16 * wv + l16] * sm.w[(k0 + g4) >> 1];
-#pragma unroll
-                for (int pt = 0; pt < NPT; ++pt) hacc[pt] = mfma4(bw, sm.X[k0 + g4][16 * pt + l16], hacc[pt]);
-            }
-        }
-        // ---- the state entering chunk k + 1 for the layer backward. The walk folds the beta
-        // term of the next chunk's first token into this chunk (b_{Q-1} B~_{Q-1} x_{Q-1}^T, the
-        // last row pair of the tiles); the chunk kernels count it in the next chunk, so it is
-        // taken out of the stored state (b = 0 without the trapezoid).
-        if (a.hs_every > 0 && (k + 1) % a.hs_every == 0 && k + 1 < K) {
-            const float bq = sm.bv[Q - 1];
-            float* hk = a.st.Hs + (((int64_t)b * (a.hs_K + 1) + (k + 1) / a.hs_every) * a.H + h) * (P * N) +
-                        (int64_t)pc * N;
-#pragma unroll
-            for (int pt = 0; pt < NPT; ++pt) {
-                const int pl = 16 * pt + l16;
-                const float x0 = sm.X[2 * (Q - 1)][pl], x1 = sm.X[2 * (Q - 1) + 1][pl];
-                f32x4 o;
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int n = 16 * wv + 4 * g4 + v;
-                    o[v] = hacc[pt][v] - bq * (sm.B[2 * (Q - 1)][n] * x0 + sm.B[2 * (Q - 1) + 1][n] * x1);
+                for (int g = 0; g < GR; ++g) {
+                    if (g == tg) ph = run;
+                    run -= pp[g];
                 }
-                *reinterpret_cast<f32x4*>(&hk[pl * N + 16 * wv + 4 * g4]) = o;
+                phi_run = run;
             }
-        }
-        // ---- gate and MIMO-down; rows 4 g4 + 2 tt + r of the block are (t, r)
+            f32x2 pm[TPT];
+            bool small = true;
 #pragma unroll
-        for (int q = 0; q < TPW; ++q) {
-            const int pl = 16 * (ptb + q) + l16;  // block column
+            for (int m = 0; m < TPT; ++m) {
+                const int t = tg * TPT + m, st = tbeg + kk * Q + t;
+                if (a.cplx) ph -= pth[m] * tk.dt[t];
+                pm[m] = ph;
+                small &= fabsf(ph[0]) <= kSincosMax && fabsf(ph[1]) <= kSincosMax;
+                if (stage && st < T)
+                    *reinterpret_cast<f32x2*>(a.st.phi + (((int64_t)b * T + st) * a.H + h) * NH + 2 * hl) = ph;
+            }
+            // (without complex parameters the angles are 0: cos 1, sin 0)
+            if (small) {
 #pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                const int t = 8 * I + 2 * g4 + tt;
-                if (s0 + t < T) {
-                    if (a.stage)
-                        *reinterpret_cast<f32x2*>(a.st.ys + (((int64_t)b * T + s0 + t) * a.H + h) * (P * R) + (int64_t)(pc + pl) * R) =
-                            f32x2{yacc[q][2 * tt], yacc[q][2 * tt + 1]};
-                    const float z = sm.Z[t][pl];
-                    const float o = md[q][0] * yacc[q][2 * tt] * silu_hw(z * mz[q][0]) +
-                                    md[q][1] * yacc[q][2 * tt + 1] * silu_hw(z * mz[q][1]);
-                    a.y_out[((int64_t)b * T + s0 + t) * HP + h * P + pc + pl] = o;
+                for (int m = 0; m < TPT; ++m)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        float s, c;
+                        sincos_small(pm[m][e], s, c);
+                        sn[m][e] = s;
+                        cs[m][e] = c;
+                    }
+            } else {
+#pragma unroll 1
+                for (int m = 0; m < TPT; ++m)
+#pragma unroll 1
+                    for (int e = 0; e < 2; ++e) {
+                        float s, c;
+                        sincosf(pm[m][e], &s, &c);
+                        sn[m][e] = s;
+                        cs[m][e] = c;
+                    }
+            }
+        };
+        // X^T columns (t, r) = x_t * mimo_x[p, r] (mamba3/mamba3.py:210) of chunk kk
+        auto write_x = [&](int kk) {
+            const Tok& tk = sm.tok[kk % 3];
+            f32x4 xo[XTOK / 2];
+#pragma unroll
+            for (int m = 0; m < XTOK; ++m) {
+                const int t = xt0 + m, st = tbeg + kk * Q + t;
+                const f32x2 xr = f32x2{pxv[m] * mx0, pxv[m] * mx1};
+                xo[m / 2][2 * (m % 2)] = xr[0];
+                xo[m / 2][2 * (m % 2) + 1] = xr[1];
+                if (stage && st < T) {
+                    // x_r, x_g = lambda_t x_r and x_b of the next token (mamba3/mamba3.py:210-224)
+                    const int64_t e = ((((int64_t)b * T + st) * a.H + h) * P + xp) * R;
+                    *reinterpret_cast<f32x2*>(a.st.xr + e) = xr;
+                    *reinterpret_cast<f32x2*>(a.st.xg + e) = xr * tk.lam[t];
+                    if (a.trap) {
+                        if (st + 1 < T) *reinterpret_cast<f32x2*>(a.st.xb + e + (int64_t)a.H * P * R) = xr * tk.sb[t];
+                        if (st == 0) *reinterpret_cast<f32x2*>(a.st.xb + e) = f32x2{0.f, 0.f};
+                    }
                 }
             }
+#pragma unroll
+            for (int v = 0; v < XTOK / 2; ++v) *reinterpret_cast<f32x4*>(&sm.XT[xp][xt0 * R + 4 * v]) = xo[v];
+        };
+        // rotated C~ / B~ rows of the words in hand (words of tokens past the end are zero),
+        // chunk kk
+        auto write_tiles = [&](int kk) {
+            float (&sB)[ROWS][CST] = sm.B[kk & 1];
+#pragma unroll
+            for (int m = 0; m < TPT; ++m) {
+                const int t = tg * TPT + m, st = tbeg + kk * Q + t;
+                const f32x2 c = cs[m], s = sn[m];
+                // rank r: words r (n even) and 2 + r (n odd) of each pair
+                auto turn = [&](const f32x4 (&v)[2], int r) {
+                    return f32x4{v[0][r] * c[0] - v[0][2 + r] * s[0], v[0][r] * s[0] + v[0][2 + r] * c[0],
+                                 v[1][r] * c[1] - v[1][2 + r] * s[1], v[1][r] * s[1] + v[1][2 + r] * c[1]};
+                };
+                const f32x4 b0 = turn(pb[m], 0), b1 = turn(pb[m], 1);
+                *reinterpret_cast<f32x4*>(&sB[2 * t][4 * hl]) = b0;
+                *reinterpret_cast<f32x4*>(&sB[2 * t + 1][4 * hl]) = b1;
+                if constexpr (FULL) {
+                    const f32x4 c0 = turn(pc[m], 0), c1 = turn(pc[m], 1);
+                    *reinterpret_cast<f32x4*>(&sm.C[2 * t][4 * hl]) = c0;
+                    *reinterpret_cast<f32x4*>(&sm.C[2 * t + 1][4 * hl]) = c1;
+                    if (stage && st < T) {
+                        const int64_t tk = ((int64_t)b * T + st) * a.H + h;
+                        const f32x4 bl = f32x4{b0[0], b1[0], b0[1], b1[1]}, bu = f32x4{b0[2], b1[2], b0[3], b1[3]};
+                        f32x4* q = reinterpret_cast<f32x4*>(a.st.Bt + tk * NR + 8 * hl);
+                        q[0] = bl;
+                        q[1] = bu;
+                        q = reinterpret_cast<f32x4*>(a.st.Ct + tk * NR + 8 * hl);
+                        q[0] = f32x4{c0[0], c1[0], c0[1], c1[1]};
+                        q[1] = f32x4{c0[2], c1[2], c0[3], c1[3]};
+                        if (a.trap) {  // B_b[t + 1] = B~[t]
+                            if (st + 1 < T) {
+                                q = reinterpret_cast<f32x4*>(a.st.Bb + (tk + a.H) * NR + 8 * hl);
+                                q[0] = bl;
+                                q[1] = bu;
+                            }
+                            if (st == 0) {
+                                q = reinterpret_cast<f32x4*>(a.st.Bb + tk * NR + 8 * hl);
+                                q[0] = q[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+                            }
+                        }
+                    }
+                }
+            }
+        };
+        const bool token_wave = hw == HW - 1;
+
+        // Prologue: chunks 0 and 1's token scalars, chunk 0's tiles, chunk 1's reads (chunks past
+        // the end read as zero).
+        load_bc(0);
+        load_xv(0);
+        load_theta(0);
+        if (hw >= HW - 2) {
+            load_tokens(hw - (HW - 2));
+            prep_tokens(hw - (HW - 2));
+            if (token_wave) load_tokens(2);
+        }
+        __syncthreads();
+        angle_sums(0);
+        __syncthreads();
+        angles(0);
+        write_tiles(0);
+        load_bc(1);
+        load_theta(1);
+        __syncthreads();
+
+        for (int k = 0; k < K; ++k) {
+            const bool more = k + 1 < K;
+            // ---- scores ----
+            if constexpr (FULL) {
+                // causal score tiles (ti, ui), ui <= ti: helpers 0-3 take (3, 0..3), 4-6 (2, 0..2) and
+                // (1, 0), (1, 1), (0, 0); lane: u-rows 16 ui + 4 g16 + v, t-row 16 ti + l16
+                const Tok& tk = sm.tok[k % 3];
+                const float (&sB)[ROWS][CST] = sm.B[k & 1];
+                const int nt = hw < 4 ? 1 : token_wave ? 0 : 2;
+#pragma unroll 1
+                for (int c = 0; c < nt; ++c) {
+                    const int ti = hw < 4 ? 3 : c == 0 ? 2 : hw == 6 ? 0 : 1;
+                    const int ui = hw == 6 && c == 1 ? 0 : hw & 3;
+                    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;  // even and odd k-steps
+                    f32x4 A[2][2], B[2][2];
+                    auto load_s = [&](int s) {
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) {
+                            A[s & 1][j] = *reinterpret_cast<const f32x4*>(&sB[16 * ui + l16][32 * s + 16 * j + 4 * g16]);
+                            B[s & 1][j] = *reinterpret_cast<const f32x4*>(&sm.C[16 * ti + l16][32 * s + 16 * j + 4 * g16]);
+                        }
+                    };
+                    load_s(0);
+#pragma unroll
+                    for (int s = 0; s < N / 32; ++s) {
+                        if (s + 1 < N / 32) load_s(s + 1);
+                        M3_FENCE();
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            s0 = mfma4(A[s & 1][0][v], B[s & 1][0][v], s0);
+                            s1 = mfma4(A[s & 1][1][v], B[s & 1][1][v], s1);
+                        }
+                    }
+                    s0 += s1;
+                    // the lane's rows are two tokens u, u + 1; masked pairs get weight 0 (their
+                    // exponent is capped, so no overflow meets the 0)
+                    const int trow = 16 * ti + l16, t = trow >> 1, u = 8 * ui + 2 * g16;
+                    const float ct = tk.c[t];
+                    const f32x2 cu = *reinterpret_cast<const f32x2*>(&tk.c[u]);
+                    const f32x2 au = *reinterpret_cast<const f32x2*>(&tk.av[u]);
+                    const f32x2 bu = *reinterpret_cast<const f32x2*>(&tk.bv[u]);
+                    float f[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const float wu = u + e < t ? au[e] + bu[e] : u + e == t ? au[e] : 0.f;
+                        f[e] = exp_hw(fminf(ct - cu[e], 0.f)) * wu;
+                    }
+                    f32x4 sv;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        sv[v] = u + v / 2 <= t ? s0[v] * f[v / 2] : 0.f;
+                        if (2 * u + v == trow) sv[v] += Dh;
+                    }
+                    *reinterpret_cast<f32x4*>(&sm.S[trow][16 * ui + 4 * g16]) = sv;
+                }
+            }
+            write_x(k);
+            load_xv(k + 1);
+            if (more) angle_sums(k + 1);
+            if (token_wave) {
+                prep_tokens(k + 2);
+                load_tokens(k + 3);
+            }
+            __syncthreads();
+            // ---- update ----
+            if (more) {
+                angles(k + 1);
+                write_tiles(k + 1);
+                load_bc(k + 2);
+                load_theta(k + 2);
+            }
+            __syncthreads();
+        }
+        // phi_run is the angle after the last chunk
+        if constexpr (FULL) {
+            if (a.angle && tend == T && htid < LPT) {
+                float* ang = a.angle + (int64_t)bh * NH + 2 * hl;
+                ang[0] = phi_run[0];
+                ang[1] = phi_run[1];
+            }
+            if (a.prev_bx && tend == T) {
+                // B~_{T-1} x_r,{T-1}^T from the last chunk's tiles
+                const int ul = T - 1 - tbeg - (K - 1) * Q;
+                for (int i = htid; i < P * N / 4; i += HT) {
+                    const int pp = i / (N / 4), n = 4 * (i % (N / 4));
+                    const f32x4 b0 = *reinterpret_cast<const f32x4*>(&sm.B[(K - 1) & 1][2 * ul][n]);
+                    const f32x4 b1 = *reinterpret_cast<const f32x4*>(&sm.B[(K - 1) & 1][2 * ul + 1][n]);
+                    *reinterpret_cast<f32x4*>(a.prev_bx + ((int64_t)bh * P + pp) * N + n) =
+                        b0 * sm.XT[pp][2 * ul] + b1 * sm.XT[pp][2 * ul + 1];
+                }
+            }
+        } else {
+            if (htid < LPT)
+                *reinterpret_cast<f32x2*>(a.aseg + ((int64_t)seg * npairs + bh) * NH + 2 * hl) = phi_run;
         }
     }
-    __syncthreads();
-    // ---- outputs of the walk
-    if (a.hs_every > 0) {
-        float* hk = a.st.Hs + (((int64_t)b * (a.hs_K + 1) + a.hs_K) * a.H + h) * (P * N) + (int64_t)pc * N;
-#pragma unroll
-        for (int pt = 0; pt < NPT; ++pt)
-            *reinterpret_cast<f32x4*>(&hk[(16 * pt + l16) * N + 16 * wv + 4 * g4]) = hacc[pt];
+}
+
+// Turns the segments' end states (from a zero start, each in its own RoPE frame) into the
+// states entering the next segments, in place: one thread per four state rows of a column.
+__global__ __launch_bounds__(256) void seg_combine_f32(Args a) {
+    constexpr int PER = CW * NT * 64;  // entries per (batch, head)
+    const int npairs = a.B * a.H;
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (int64_t)npairs * PER) return;
+    const int bh = (int)(e / PER), t = (int)(e % (NT * 64)) / 64, g16 = (int)(e % 64) / 16;
+    const int i = (16 * t + 4 * g16) / 2;  // first RoPE pair
+    f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x2 phi = f32x2{0.f, 0.f};
+#pragma unroll 2
+    for (int j = 0; j < a.segs - 1; ++j) {
+        f32x4* hj = a.hseg + (int64_t)j * npairs * PER + e;
+        const f32x4 v = *hj;
+        const f32x2 inc = *reinterpret_cast<const f32x2*>(a.aseg + ((int64_t)j * npairs + bh) * NH + i);
+        const float dec = expf(a.lseg[(int64_t)j * npairs + bh]);
+        float s0, c0, s1, c1;
+        sincosf(phi[0], &s0, &c0);
+        sincosf(phi[1], &s1, &c1);
+        h = h * dec + f32x4{v[0] * c0 - v[1] * s0, v[0] * s0 + v[1] * c0,
+                            v[2] * c1 - v[3] * s1, v[2] * s1 + v[3] * c1};
+        *hj = h;
+        phi += inc;
     }
-    if (a.h_final) {
-        float* hf = a.h_final + (int64_t)bh * P * N + (int64_t)pc * N;
-#pragma unroll
-        for (int pt = 0; pt < NPT; ++pt)
-            *reinterpret_cast<f32x4*>(&hf[(16 * pt + l16) * N + 16 * wv + 4 * g4]) = hacc[pt];
-    }
-    if (a.angle && pc == 0 && tid < NH) a.angle[(int64_t)bh * NH + tid] = a.cplx ? sm.phi_run[K & 1][tid] : 0.f;
-    if (a.prev_bx) {
-        // B~_{T-1} x_r,{T-1}^T from the last chunk's tiles (still in LDS)
-        const int ul = (T - 1) - (K - 1) * Q;
-        const int p = tid / (N / NPE), n0 = NPE * (tid % (N / NPE));  // block column p
-        const float x0 = sm.X[2 * ul][p], x1 = sm.X[2 * ul + 1][p];
-        float* pb = a.prev_bx + (int64_t)bh * P * N + (int64_t)(pc + p) * N + n0;
-#pragma unroll
-        for (int j = 0; j < NPE; j += 4) {
-            f32x4 o;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = sm.B[2 * ul][n0 + j + e] * x0 + sm.B[2 * ul + 1][n0 + j + e] * x1;
-            *reinterpret_cast<f32x4*>(pb + j) = o;
-        }
-    }
+}
+
+// Segments of a call (1: one walk per (batch, head)) and the bytes of their states, log-decays
+// and angle increments. The state pass costs about half a walk, so segments pay only while the
+// pairs leave more than half of the 256 CUs idle and the walk is long: whole d_model 768
+// forward, one walk against segments, 48 pairs x 500 tokens 223 / 159 us, 96 x 1024 551 / 475;
+// but 24 x 129 80 / 98, 96 x 200 139 / 146, 144 x 1024 680 / 697, 192 x 1024 782 / 864.
+struct SegPlan {
+    int segs;
+    size_t lseg, aseg, bytes;  // offsets behind the states
+};
+inline size_t al256(size_t n) { return (n + 255) & ~(size_t)255; }
+SegPlan seg_plan(const m3_layer_desc& d, size_t limit) {
+    SegPlan p = {1, 0, 0, 0};
+    const size_t BH = (size_t)d.batch * d.nheads;
+    if (BH >= 128 || d.seqlen <= 2 * kSeg0) return p;
+    int segs = 1;
+    while (seg_start(segs) < d.seqlen) ++segs;
+    const size_t n = segs - 1;
+    const size_t lseg = n * BH * P * N * sizeof(float);
+    const size_t aseg = lseg + al256(n * BH * sizeof(float));
+    const size_t bytes = aseg + al256(n * BH * NH * sizeof(float));
+    return bytes <= limit ? SegPlan{segs, lseg, aseg, bytes} : p;
 }
 
 }  // namespace f32k
@@ -485,7 +831,10 @@ static bool fused_fp32_shape_ok(const m3_layer_desc& d, const void* proj, const 
     if (d.dtype != M3_DTYPE_F32) return false;
     if (d.d_state != f32k::N || d.headdim != f32k::P || d.mimo_rank != f32k::R) return false;
     const ProjLayout pl = proj_layout(d);
-    // 16-byte reads of the B / C rows and of x / z
+    // a chunk's rows are addressed with 32-bit byte offsets
+    if (d.proj_row_stride >= (1 << 22) || (int64_t)d.ngroups * f32k::NR >= (1 << 22) || d.nheads >= (1 << 18))
+        return false;
+    // 16-byte reads of the B / C rows
     if (d.proj_row_stride % 4 != 0 || pl.x % 4 != 0 || pl.z % 4 != 0 || pl.B % 4 != 0 || pl.C % 4 != 0)
         return false;
     auto al16 = [](const void* ptr) { return reinterpret_cast<uintptr_t>(ptr) % 16 == 0; };
@@ -503,31 +852,43 @@ bool fused_fp32_train_supported(const m3_layer_desc& d, const void* proj, const 
     if (!fused_fp32_shape_ok(d, proj, y_out, h_final, prev_bx) || !fp32_layer_supported(d)) return false;
     size_t bytes = 0;
     fp32_layer_scratch(d, nullptr, &bytes);
-    return bytes >= fused_fp32_prefill_workspace(d);
+    return bytes >= fused_fp32_prefill_workspace(d, 0);
 }
 
-size_t fused_fp32_prefill_workspace(const m3_layer_desc& d) {
-    return 2 * (size_t)d.batch * d.seqlen * d.ngroups * f32k::NR * sizeof(float) + 256;
+// B^ and C^ rows, then the segments' states where `limit` bytes hold them.
+static size_t fused_fp32_rows(const m3_layer_desc& d) {
+    return f32k::al256((size_t)d.batch * d.seqlen * d.ngroups * f32k::NR * sizeof(float));
+}
+size_t fused_fp32_prefill_workspace(const m3_layer_desc& d, size_t limit) {
+    const size_t rows = 2 * fused_fp32_rows(d);
+    return rows + f32k::seg_plan(d, limit > rows ? limit - rows : 0).bytes;
 }
 
 int launch_fused_fp32_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                               const float* dt_scale, void* y_out, float* h_final, float* angle,
-                              float* prev_bx, void* workspace, hipStream_t stream,
+                              float* prev_bx, void* workspace, size_t limit, hipStream_t stream,
                               const Fp32LayerParts* stage) {
     const ProjLayout pl = proj_layout(d);
     const int64_t nrows = (int64_t)d.batch * d.seqlen * d.ngroups;
-    float* bn = reinterpret_cast<float*>(workspace);
-    float* cn = bn + nrows * f32k::NR;
+    const size_t rows = fused_fp32_rows(d);
+    char* ws = reinterpret_cast<char*>(workspace);
+    float* bn = reinterpret_cast<float*>(ws);
+    float* cn = reinterpret_cast<float*>(ws + rows);
+    char* seg = ws + 2 * rows;  // the segments' states, in room bytes
+    size_t room = limit > 2 * rows ? limit - 2 * rows : 0;
     // Training forward with room for the chunk-start states (workspace = the fp32 layer
-    // workspace's chunk-kernel region, whose Hs part is stage->Hs): C^ rows past them.
+    // workspace's chunk-kernel region, whose Hs part is stage->Hs): C^ rows past them, the
+    // segments' states between the B^ rows and them.
     const bool hs = stage && stage->Hs && fp32_layer_hs_ok(d);
     int hs_every = 0, hs_K = 0;
     if (hs) {
         const bool trap = d.use_trapezoidal != 0;
         const size_t off = chunked_fwd_hs_offset(d.batch, d.seqlen, d.nheads, d.headdim, d.d_state,
                                                  d.mimo_rank, trap);
-        const size_t hsb = (fp32_layer_hs_bytes(d) + 255) & ~(size_t)255;
-        cn = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + off + hsb);
+        const size_t hsb = f32k::al256(fp32_layer_hs_bytes(d));
+        cn = reinterpret_cast<float*>(ws + off + hsb);
+        seg = ws + rows;
+        room = off > rows ? off - rows : 0;
         const int qb = chunked_chunk_tokens(d.mimo_rank, trap);
         if (qb % f32k::Q != 0) return M3_ERR_UNSUPPORTED;
         hs_every = qb / f32k::Q;
@@ -554,12 +915,18 @@ int launch_fused_fp32_prefill(const m3_layer_desc& d, const m3_layer_params& p, 
     a.stage = stage != nullptr;
     a.hs_every = hs_every;
     a.hs_K = hs_K;
-    // two 32-column blocks per (batch, head) while the pairs alone leave CUs idle
-    const int64_t bh = (int64_t)d.batch * d.nheads;
-    if (bh < 256)
-        hipLaunchKernelGGL(f32k::ssd_f32<32>, dim3((unsigned)(bh * 2)), dim3(f32k::THREADS), 0, stream, a);
-    else
-        hipLaunchKernelGGL(f32k::ssd_f32<64>, dim3((unsigned)bh), dim3(f32k::THREADS), 0, stream, a);
+    const f32k::SegPlan sp = f32k::seg_plan(d, room);
+    a.segs = sp.segs;
+    a.hseg = reinterpret_cast<f32x4*>(seg);
+    a.lseg = reinterpret_cast<float*>(seg + sp.lseg);
+    a.aseg = reinterpret_cast<float*>(seg + sp.aseg);
+    const unsigned bh = (unsigned)(d.batch * d.nheads);
+    if (sp.segs > 1) {
+        hipLaunchKernelGGL(f32k::ssd_f32<false>, dim3(bh * (sp.segs - 1)), dim3(f32k::THREADS), 0, stream, a);
+        hipLaunchKernelGGL(f32k::seg_combine_f32, dim3((unsigned)(((int64_t)bh * f32k::P * f32k::N / 4 + 255) / 256)),
+                           dim3(256), 0, stream, a);
+    }
+    hipLaunchKernelGGL(f32k::ssd_f32<true>, dim3(bh * sp.segs), dim3(f32k::THREADS), 0, stream, a);
     return hipGetLastError() == hipSuccess ? M3_OK : M3_ERR_LAUNCH;
 }
 

@@ -711,6 +711,83 @@ def test_fp32_fused_prefill_matches_oracle(extra, T, scaled, cuda_device):
     assert max_rel(y_train.detach(), y) < FP32_TOL
 
 
+@pytest.mark.parametrize("extra,B,T", [
+    (dict(), 2, 257),                                     # third segment of one token
+    (dict(ngroups=2), 1, 1100),                           # into the 512-token segments, last chunk of 12
+    (dict(use_trapezoidal=False), 2, 545),                # into the 256-token segments
+    (dict(use_complex_ssm=False, ngroups=2), 1, 384),     # ends with a segment
+])
+def test_fp32_fused_segments_match_oracle(extra, B, T, cuda_device):
+    """Sequences cut into segments (state pass, combine, full pass) with dt_scale against the
+    fp64 oracle, and as one walk in a workspace without room for the segments' states; the
+    training forward, which also stores the backward's operands and chunk-start states, gives
+    the same output and the oracle's input gradient."""
+    kw = dict(d_model=128, d_state=128, headdim=64, mimo_rank=2, **extra)
+    print(f"fp32 segments {extra} B {B} T {T}", flush=True)
+    dev = cuda_device
+    torch.manual_seed(6)
+    layer = mamba3_amd.KulaMamba(**kw).to(dev).eval()
+    p = {k: v.detach().double().cpu() for k, v in layer.state_dict().items()}
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(B, T, 128, generator=g)
+    ds = torch.rand(B, T, layer.nheads, generator=g) + 0.5
+    dsd = ds.to(dev)
+    w, xr = torch.randn(B, T, 128, generator=g), x.double().requires_grad_()
+    y_ref, st_ref = ref.layer_forward(oracle_cfg(kw), p, xr, dt_scale=ds.double(), return_state=True)
+    ((y_ref * w).sum() + st_ref["h"].sum()).backward()
+    y_ref, st_ref = y_ref.detach(), {k: v.detach() for k, v in st_ref.items()}
+    with torch.no_grad():
+        proj = layer.in_proj(x.to(dev)).contiguous()
+        y, st = layer.ssd_from_proj(proj, dt_scale=dsd, return_state=True)
+        desc = layer._desc(B, T, proj)
+        assert _native.prefill_kernel_name(desc, proj) == "fp32_fused"
+        rows = 2 * (B * T * layer.ngroups * 256 * 4 + 256)
+        assert rows < _native.prefill_workspace_bytes(desc)
+        y1, h1, a1, b1 = (torch.empty_like(t) for t in (y, st["h"], st["angle"], st["prev_BX"]))
+        ws = torch.empty(rows, device=dev, dtype=torch.uint8)
+        _native.prefill_fwd(desc, layer._param_pack(), proj, dsd, y1, h1, a1, b1, ws, rows)
+        for out in (y, y1):
+            assert max_rel(layer.out_proj(out), y_ref) < FP32_TOL
+    for k, one in (("h", h1), ("prev_BX", b1), ("angle", a1)):
+        assert max_rel(st[k], st_ref[k]) < FP32_TOL, k
+        assert max_rel(one, st_ref[k]) < FP32_TOL, k
+    xg = x.to(dev).requires_grad_()
+    y, st = layer.prefill(xg, dt_scale=dsd)
+    ((y * w.to(dev)).sum() + st["h"].sum()).backward()
+    assert max_rel(y.detach(), y_ref) < FP32_TOL
+    assert max_rel(xg.grad, xr.grad) < FP32_TOL
+
+
+def test_fp32_fused_rotation_over_the_angle_range(cuda_device):
+    """The rotation's sines and cosines on both sides of the 1e5 bound of the straight-line
+    form: one token with the RoPE rates set to each size against the same token unrotated,
+    turned by the returned angles in fp64. Per rank each sine is off by at most 7.1e-8 and the
+    two products, their sum and the product with x round once (2^-24 each): 2.5e-7 of the
+    pair's length, twice that for the two ranks, and twice again where they cancel."""
+    dev = cuda_device
+    torch.manual_seed(8)
+    layer = mamba3_amd.KulaMamba(d_model=128, d_state=128, headdim=64, mimo_rank=2).to(dev).eval()
+    with torch.no_grad():
+        proj = layer.in_proj(torch.randn(1, 1, 128, device=dev)).contiguous()
+        nh = layer.d_state // 2
+        theta = torch.randn(nh, device=dev)
+        proj[..., -nh:] = 0.0
+        plain = layer.ssd_from_proj(proj, return_state=True)[1]["prev_BX"].double()
+        assert plain.abs().max() > 0
+        for scale in (1.0, 1e3, 1e6, 3e7, 1e9):
+            print(f"theta scale {scale}", flush=True)
+            proj[..., -nh:] = theta * scale
+            st = layer.ssd_from_proj(proj, return_state=True)[1]
+            ang = st["angle"].double()[:, :, None, :]
+            v = plain.unflatten(-1, (nh, 2))
+            want = torch.stack([v[..., 0] * ang.cos() - v[..., 1] * ang.sin(),
+                                v[..., 0] * ang.sin() + v[..., 1] * ang.cos()], -1)
+            err = (st["prev_BX"].double().unflatten(-1, (nh, 2)) - want).abs().amax(-1)
+            # against the head's largest pair
+            size = v.norm(dim=-1).amax(dim=(-1, -2), keepdim=True)
+            assert (err / size).max() < 1e-6, (scale, (err / size).max())
+
+
 # ------------------------------------------------------------------ general MFMA prefill kernel
 # bf16 layers with d_state 64/128/256, rank 1/2/4 and headdim % 32 == 0 (other than
 # d_state 128 / headdim 64 / rank 2) run on the general MFMA kernel: one case per
