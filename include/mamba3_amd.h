@@ -218,8 +218,9 @@ int m3_prefill_fwd(const m3_layer_desc* desc, const m3_layer_params* params,
  * m3_prefill_fwd, but the workspace is a static array of the library on each GPU
  * (M3_NOALLOC_SCRATCH_BYTES, held from the first call on that GPU until the process
  * ends; bf16 layers outside the MFMA kernels take what it holds, see
- * m3_prefill_workspace_size); calls needing more return M3_ERR_SCRATCH_LIMIT and launch nothing. It calls no
- * allocator. M3_FLAG_FOR_BACKWARD is refused (M3_ERR_UNSUPPORTED): the backward's operands
+ * m3_prefill_workspace_size; the general MFMA and the fused fp32 kernel walk each sequence in
+ * one piece where the states of its segments do not fit, which moves results by rounding);
+ * calls needing more return M3_ERR_SCRATCH_LIMIT and launch nothing. It calls no allocator. M3_FLAG_FOR_BACKWARD is refused (M3_ERR_UNSUPPORTED): the backward's operands
  * would be left in the shared scratch, which the next call overwrites. The scratch keeps the last call's contents and needs no clearing (every
  * kernel writes what it later reads). All calls on one GPU share the array: calls that
  * overlap in time on one GPU (other streams or threads) race and must be serialised by
