@@ -77,7 +77,7 @@ PrefillPath prefill_path(const m3_layer_desc& d, const void* proj, const void* y
 size_t prefill_path_workspace(const m3_layer_desc& d, PrefillPath path, size_t limit) {
     switch (path) {
         case PrefillPath::kMfma: return m3::mfma_prefill_workspace(d);
-        case PrefillPath::kWide: return m3::wide_prefill_workspace(d, limit);
+        case PrefillPath::kWide: return m3::wide_prefill_min_workspace(d);
         case PrefillPath::kFp32Fused: return m3::fused_fp32_prefill_workspace(d, limit);
         case PrefillPath::kFp32FusedTrain:
         case PrefillPath::kFp32: return m3::fp32_layer_workspace(d);
@@ -250,7 +250,7 @@ static size_t prefill_workspace(const m3_layer_desc& d) {
     if (m3::fused_fp32_prefill_supported(d, nullptr, nullptr, nullptr, nullptr))
         n = std::max(n, m3::fused_fp32_prefill_workspace(d, SIZE_MAX));
     if (m3::mfma_prefill_supported(d, nullptr, nullptr)) n = std::max(n, m3::mfma_prefill_workspace(d));
-    if (m3::wide_prefill_supported(d)) n = std::max(n, m3::wide_prefill_workspace(d, SIZE_MAX));
+    if (m3::wide_prefill_supported(d)) n = std::max(n, m3::wide_prefill_workspace(d));
     else n = std::max(n, m3::staged_bf16_workspace(d, SIZE_MAX));
     return n;
 }

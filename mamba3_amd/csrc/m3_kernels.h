@@ -70,10 +70,11 @@ int launch_mfma_prefill(const m3_layer_desc& d, const m3_layer_params& p, const 
                         float* prev_bx, void* workspace, hipStream_t stream);
 
 // bf16 MFMA fused prefill for d_state 64/128/256, mimo_rank 1/2/4, headdim % 32 == 0.
-// Workspace within `limit` bytes where the segments' states fit it, else that of one walk per
-// (batch, head); the launcher takes the same limit.
+// Workspace of a call in one piece, and the least one that it runs in; the launcher takes the
+// bytes of its workspace.
 bool wide_prefill_supported(const m3_layer_desc& d);
-size_t wide_prefill_workspace(const m3_layer_desc& d, size_t limit);
+size_t wide_prefill_workspace(const m3_layer_desc& d);
+size_t wide_prefill_min_workspace(const m3_layer_desc& d);
 int launch_wide_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                         const float* dt_scale, void* y_out, float* h_final, float* angle,
                         float* prev_bx, void* workspace, size_t limit, hipStream_t stream);

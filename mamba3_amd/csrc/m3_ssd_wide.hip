@@ -134,10 +134,12 @@ struct Args {
     float* h_final;
     float* angle;
     float* prev_bx;
-    // segments of the sequence (segs = 1: none); per segment but the last and pair, the state
-    // pass's end state, which seg_combine turns into the state entering the next segment
+    // segments of the sequence (segs = 1: none), of which a launch takes lo .. hi - 1; per segment
+    // but the last and pair, the state pass's end state, which seg_combine turns into the state
+    // entering the next segment. The state entering segment e is kept in slot (e - 1) % slots.
     int segs, seg0;
-    f32x4* hseg;  // [seg][pair block][column group][n half][tile][lane]
+    int lo, hi, slots;
+    f32x4* hseg;  // [slot][pair block][column group][n half][tile][lane]
     float* lseg;  // log2 of the segment's decay, [seg][b h]
     float* aseg;  // its RoPE angle increment, [seg][b h][pair]
 };
@@ -346,7 +348,7 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
     // (batch, head, column block) pairs are renumbered so that consecutive ones, which read the
     // same normalised B^ / C^ rows, share an XCD and its L2.
     const int so = blockIdx.x / npairs, j0 = blockIdx.x % npairs;
-    const int seg = (FULL ? a.segs : a.segs - 1) - 1 - so;  // the state pass leaves the last segment out
+    const int seg = (FULL ? a.hi : min(a.hi, a.segs - 1)) - 1 - so;  // the state pass leaves the last segment out
     const int pair = (npairs % 8 == 0) ? (j0 % 8) * (npairs / 8) + j0 / 8 : j0;
     const int pblk = pair % a.PS;
     const int bh = pair / a.PS;
@@ -488,7 +490,7 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
         for (int t = 0; t < NT; ++t) hacc[t][0] = hacc[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (FULL && seg > 0) {
             // state entering the segment (seg_combine)
-            const f32x4* hs = a.hseg + (((int64_t)(seg - 1) * npairs + pair) * CW + wave) * (NT * 2 * 64) + lane;
+            const f32x4* hs = a.hseg + (((int64_t)((seg - 1) % a.slots) * npairs + pair) * CW + wave) * (NT * 2 * 64) + lane;
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -651,7 +653,7 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
                         *reinterpret_cast<f32x4*>(a.h_final + ((int64_t)bh * a.P + p0 + pw + 16 * pt + l16) * N + n0 + 32 * (t >> 1) + 8 * g16 + 4 * (t & 1)) = hacc[t][pt] * scl.state;
             }
         } else {
-            f32x4* hs = a.hseg + (((int64_t)seg * npairs + pair) * CW + wave) * (NT * 2 * 64) + lane;
+            f32x4* hs = a.hseg + (((int64_t)(seg % a.slots) * npairs + pair) * CW + wave) * (NT * 2 * 64) + lane;
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
@@ -925,13 +927,20 @@ __global__ __launch_bounds__(256) void seg_combine(Args a) {
     const int w = (int)(e % PER) / (NT * 2 * 64), t = (int)(e % (NT * 2 * 64)) / 128, g16 = (int)(e % 64) / 16;
     const int i = ((w & 1) * (N / 2) + 32 * (t >> 1) + 8 * g16 + 4 * (t & 1)) / 2;  // first RoPE pair
     const int64_t sbase = (int64_t)a.B * a.H;
+    auto slot = [&](int j) { return a.hseg + (int64_t)(j % a.slots) * npairs * PER + e; };
+    auto angle_inc = [&](int j) {
+        return *reinterpret_cast<const f32x2*>(a.aseg + ((int64_t)j * sbase + bh) * (N / 2) + i);
+    };
     f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f};
     f32x2 phi = f32x2{0.f, 0.f};
+    if (a.lo > 0) h = *slot(a.lo - 1);
+    for (int j = 0; j < a.lo; ++j) phi += angle_inc(j);
+    const int hi = min(a.hi, a.segs - 1);
 #pragma unroll 2
-    for (int j = 0; j < a.segs - 1; ++j) {
-        f32x4* hj = a.hseg + (int64_t)j * npairs * PER + e;
+    for (int j = a.lo; j < hi; ++j) {
+        f32x4* hj = slot(j);
         const f32x4 v = *hj;
-        const f32x2 inc = *reinterpret_cast<const f32x2*>(a.aseg + ((int64_t)j * sbase + bh) * (N / 2) + i);
+        const f32x2 inc = angle_inc(j);
         const float dec = __builtin_amdgcn_exp2f(a.lseg[(int64_t)j * sbase + bh]);
         float s0, c0, s1, c1;
         fast_sincos(phi[0], s0, c0);
@@ -943,66 +952,99 @@ __global__ __launch_bounds__(256) void seg_combine(Args a) {
     }
 }
 
+// The segments in groups of `group` (all of them, unless the workspace holds fewer states).
 template <int N, int R, int NCG>
-void launch_ssd(const Args& a, hipStream_t stream) {
+void launch_ssd(Args a, int group, hipStream_t stream) {
     const unsigned npairs = (unsigned)(a.B * a.H * a.PS);
     const dim3 threads(64 * (2 * NCG + Layout<N, R>::HELPERS));
-    if (a.segs > 1) {
-        hipLaunchKernelGGL((ssd_wide<N, R, NCG, false>), dim3(npairs * (a.segs - 1)), threads, 0, stream, a);
-        hipLaunchKernelGGL((seg_combine<N, NCG>), dim3((unsigned)(((int64_t)npairs * PW * NCG * N / 4 + 255) / 256)),
-                           dim3(256), 0, stream, a);
+    for (a.lo = 0; a.lo < a.segs; a.lo = a.hi) {
+        a.hi = std::min(a.segs, a.lo + group);
+        const int ns = std::min(a.hi, a.segs - 1) - a.lo;
+        if (ns > 0) {
+            hipLaunchKernelGGL((ssd_wide<N, R, NCG, false>), dim3(npairs * ns), threads, 0, stream, a);
+            hipLaunchKernelGGL((seg_combine<N, NCG>), dim3((unsigned)(((int64_t)npairs * PW * NCG * N / 4 + 255) / 256)),
+                               dim3(256), 0, stream, a);
+        }
+        hipLaunchKernelGGL((ssd_wide<N, R, NCG, true>), dim3(npairs * (a.hi - a.lo)), threads, 0, stream, a);
     }
-    hipLaunchKernelGGL((ssd_wide<N, R, NCG, true>), dim3(npairs * a.segs), threads, 0, stream, a);
 }
 
 inline size_t al256(size_t n) { return (n + 255) & ~(size_t)255; }
 
+// What a call runs: the cuts of a sequence, and how much of it a workspace holds at a time.
 // Workspace: B^ and C^ rows, then the segments' states, log-decays and angle increments.
 struct Plan {
     int segs, seg0;
-    int ncg;  // column groups per workgroup
-    size_t rows, hseg, lseg, total;  // bytes of B^ (and of C^); offsets; bytes in all
+    int batch;         // sequences per slice
+    int slots, group;  // states kept, segments per group of launches
+    int ncg;           // column groups per workgroup
+    size_t rows, hseg, lseg, aseg, total;  // bytes of B^ (and of C^); offsets; bytes in all
 };
 
-// Segments of a call. The pairs alone fill the 256 CUs from about 192 on (a segmented walk
-// does 1.5x the work: its state pass). The cuts lie at fixed tokens, closer at the start, so
-// that a short prompt splits finely and a long one into few states, and no segment is much
-// longer than the mean of its sequence's share per CU; as they depend on neither the length
-// nor, below that pair count, the batch, a prefix or a sub-batch reproduces the same bits.
+void lay_out(const m3_layer_desc& d, Plan& p) {
+    const size_t n = p.segs - 1, bh = (size_t)p.batch * d.nheads;
+    p.rows = (size_t)p.batch * d.seqlen * d.ngroups * d.d_state * d.mimo_rank * sizeof(f16);
+    p.hseg = al256(2 * p.rows);
+    p.lseg = p.hseg + (n ? al256(p.slots * bh * d.headdim * d.d_state * sizeof(float)) : 0);
+    p.aseg = p.lseg + al256(n * bh * sizeof(float));
+    p.total = n ? p.aseg + n * bh * (d.d_state / 2) * sizeof(float) + 256 : 2 * p.rows + 256;
+}
+
+// The cuts of a sequence depend on nothing but its layer and its tokens: not on the batch, so
+// that a sequence gives the same bits alone and in any batch, nor on the workspace (but see
+// below), nor, as they lie at fixed tokens, on the length, so that a prefix gives the same
+// bits too. They are closer at the start, so that a short prompt splits finely and a long one
+// into few states. Heads whose column blocks alone nearly fill the 256 CUs are not cut: a
+// segmented walk does 1.5x the work (its state pass).
+//
+// A workspace that does not hold every segment's state takes the batch in slices, and one
+// that does not hold those of one sequence takes its segments in groups, from two states on:
+// the same arithmetic in more launches. Below that (no workspace of
+// m3_prefill_workspace_size bytes or of m3_prefill_fwd_noalloc) the sequence is one walk.
 Plan make_plan(const m3_layer_desc& d, size_t limit) {
-    const size_t BH = (size_t)d.batch * d.nheads;
     Plan p;
     p.ncg = column_groups(d.headdim, d.d_state, d.mimo_rank);
-    p.rows = (size_t)d.batch * d.seqlen * d.ngroups * d.d_state * d.mimo_rank * sizeof(f16);
+    const int64_t blocks = d.headdim / (PW * p.ncg);
     p.seg0 = std::max(256, d.headdim * d.d_state / 64);
     p.segs = 1;
-    p.hseg = al256(2 * p.rows);
-    p.lseg = p.hseg;
-    p.total = 2 * p.rows + 256;
-    if (BH * (d.headdim / (PW * p.ncg)) < 192 && d.seqlen > p.seg0) {
-        int segs = 1;
-        while (seg_start(segs, p.seg0) < d.seqlen) ++segs;
-        const size_t n = segs - 1;
-        const size_t lseg = p.hseg + al256(n * BH * d.headdim * d.d_state * sizeof(float));
-        const size_t total = lseg + al256(n * BH * sizeof(float)) + n * BH * (d.d_state / 2) * sizeof(float) + 256;
-        if (total <= limit) {  // else a caller's workspace without room for the states: one walk
-            p.segs = segs;
-            p.lseg = lseg;
-            p.total = total;
+    if (d.nheads * blocks < 192 && d.seqlen > p.seg0)
+        while (seg_start(p.segs, p.seg0) < d.seqlen) ++p.segs;
+    p.batch = d.batch;
+    p.slots = std::max(p.segs - 1, 1);
+    p.group = p.segs;
+    lay_out(d, p);
+    if (p.segs > 1 && p.total > limit) {
+        // the sequences of a slice, give or take alignment
+        p.batch = std::min(d.batch, 1 + (int)((double)limit / p.total * d.batch));
+        lay_out(d, p);
+        while (p.batch > 1 && p.total > limit) {
+            --p.batch;
+            lay_out(d, p);
+        }
+        while (p.slots > 2 && p.total > limit) {
+            --p.slots;
+            p.group = p.slots - 1;
+            lay_out(d, p);
+        }
+        if (p.total > limit) {
+            p.segs = p.slots = p.group = 1;
+            p.batch = d.batch;
+            lay_out(d, p);
         }
     }
     // Narrower blocks where the workgroups would leave CUs idle: they repeat the rotation and
     // the scores, but each walks its chunks faster (same bits: a column's arithmetic does not
     // depend on its block).
-    while (p.ncg > 1 && BH * (d.headdim / (PW * p.ncg)) * p.segs < 192) p.ncg /= 2;
+    const int64_t bh = (int64_t)p.batch * d.nheads * p.group;
+    while (p.ncg > 1 && bh * (d.headdim / (PW * p.ncg)) < 192) p.ncg /= 2;
     return p;
 }
 
+// One slice of the batch.
 template <int N, int R>
-int launch(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
-           const float* dt_scale, void* y_out, float* h_final, float* angle, float* prev_bx,
-           void* workspace, size_t limit, hipStream_t stream) {
-    const Plan plan = make_plan(d, limit);
+int launch_slice(const m3_layer_desc& d, const Plan& plan, const m3_layer_params& p, const bf16* proj,
+                 const float* dt_scale, bf16* y_out, float* h_final, float* angle, float* prev_bx,
+                 void* workspace, hipStream_t stream) {
     const int ncg = plan.ncg;
     char* ws = reinterpret_cast<char*>(workspace);
     Args a;
@@ -1012,22 +1054,23 @@ int launch(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
     a.rs = d.proj_row_stride;
     a.pl = proj_layout(d);
     a.prm = p;
-    a.proj = reinterpret_cast<const bf16*>(proj);
+    a.proj = proj;
     a.dt_scale = dt_scale;
     const int64_t nrows = (int64_t)d.batch * d.seqlen * d.ngroups;
     f16* bn = reinterpret_cast<f16*>(ws);
     f16* cn = reinterpret_cast<f16*>(ws + plan.rows);
     a.Bn = bn;
     a.Cn = cn;
-    a.y_out = reinterpret_cast<bf16*>(y_out);
+    a.y_out = y_out;
     a.h_final = h_final;
     a.angle = angle;
     a.prev_bx = prev_bx;
     a.segs = plan.segs;
     a.seg0 = plan.seg0;
+    a.slots = plan.slots;
     a.hseg = reinterpret_cast<f32x4*>(ws + plan.hseg);
     a.lseg = reinterpret_cast<float*>(ws + plan.lseg);
-    a.aseg = reinterpret_cast<float*>(ws + plan.lseg + al256((size_t)(plan.segs - 1) * d.batch * d.nheads * sizeof(float)));
+    a.aseg = reinterpret_cast<float*>(ws + plan.aseg);
     // vector loads of a pair's 2R raw values when every row offset keeps them aligned
     const int vec = a.rs % (2 * R) == 0 && a.pl.B % (2 * R) == 0 && a.pl.C % (2 * R) == 0 &&
                     reinterpret_cast<uintptr_t>(proj) % (4 * R) == 0;
@@ -1037,13 +1080,32 @@ int launch(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                        p.B_norm_w, p.B_bias, p.C_norm_w, p.C_bias, bn, cn);
     if constexpr (kMaxGroups<N, R> == 4) {
         if (ncg == 4) {
-            launch_ssd<N, R, 4>(a, stream);
+            launch_ssd<N, R, 4>(a, plan.group, stream);
             return hipGetLastError() == hipSuccess ? M3_OK : M3_ERR_LAUNCH;
         }
     }
-    if (ncg == 2) launch_ssd<N, R, 2>(a, stream);
-    else launch_ssd<N, R, 1>(a, stream);
+    if (ncg == 2) launch_ssd<N, R, 2>(a, plan.group, stream);
+    else launch_ssd<N, R, 1>(a, plan.group, stream);
     return hipGetLastError() == hipSuccess ? M3_OK : M3_ERR_LAUNCH;
+}
+
+template <int N, int R>
+int launch(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
+           const float* dt_scale, void* y_out, float* h_final, float* angle, float* prev_bx,
+           void* workspace, size_t limit, hipStream_t stream) {
+    const Plan plan = make_plan(d, limit);
+    const int64_t T = d.seqlen, H = d.nheads, PN = (int64_t)d.headdim * d.d_state;
+    for (int b = 0; b < d.batch; b += plan.batch) {
+        m3_layer_desc part = d;
+        part.batch = std::min(plan.batch, d.batch - b);
+        auto at = [&](auto* q, int64_t per_row) { return q ? q + b * per_row : nullptr; };
+        const int st = launch_slice<N, R>(part, plan, p, reinterpret_cast<const bf16*>(proj) + b * T * d.proj_row_stride,
+                                          at(dt_scale, T * H), reinterpret_cast<bf16*>(y_out) + b * T * H * d.headdim,
+                                          at(h_final, H * PN), at(angle, H * (d.d_state / 2)),
+                                          at(prev_bx, H * PN), workspace, stream);
+        if (st != M3_OK) return st;
+    }
+    return M3_OK;
 }
 
 }  // namespace wd
@@ -1059,9 +1121,9 @@ bool wide_prefill_supported(const m3_layer_desc& d) {
     return d.proj_row_stride < lim && (int64_t)d.ngroups * N * R < lim && (int64_t)d.nheads * d.headdim < lim;
 }
 
-size_t wide_prefill_workspace(const m3_layer_desc& d, size_t limit) {
-    return wd::make_plan(d, limit).total;
-}
+size_t wide_prefill_workspace(const m3_layer_desc& d) { return wd::make_plan(d, SIZE_MAX).total; }
+
+size_t wide_prefill_min_workspace(const m3_layer_desc& d) { return wd::make_plan(d, 0).total; }
 
 int launch_wide_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                         const float* dt_scale, void* y_out, float* h_final, float* angle,

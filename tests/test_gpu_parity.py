@@ -1066,3 +1066,73 @@ def test_general_kernel_segments_match_fp32_oracle(kw, T, cuda_device):
     for k, one in (("h", h1), ("prev_BX", b1), ("angle", a1)):
         assert max_rel(st[k], st_ref[k]) < BF16_TOL, k
         assert max_rel(one, st_ref[k]) < BF16_TOL, k
+
+
+@pytest.mark.parametrize("kw,T", [
+    (dict(d_model=512, d_state=64, headdim=64, mimo_rank=2), 257),    # two column groups a block
+    (dict(d_model=1024, d_state=64, headdim=128, mimo_rank=2), 300),  # four
+    (dict(d_model=1024, d_state=128, headdim=128, mimo_rank=1), 290),
+    (dict(d_model=1024, d_state=256, headdim=128, mimo_rank=4), 513),
+    (dict(d_model=512, d_state=256, headdim=64, mimo_rank=1), 257),
+])
+def test_general_kernel_segments_in_wide_blocks_and_any_batch(kw, T, cuda_device):
+    """Sequences cut into segments, in a batch whose 192 (batch, head) pairs run in blocks of
+    the whole headdim (state pass, combine and entering states of two and four column groups):
+    one row against the fp32 oracle, and bit for bit against that row alone, which runs in
+    blocks of 32 columns. The cuts do not depend on the batch."""
+    print(f"segments in wide blocks {kw} T {T}", flush=True)
+    dev = cuda_device
+    layer, cfg, p = _bf16_pair(kw, dev, seed=19)
+    B = 192 // layer.nheads
+    torch.manual_seed(T)
+    x = torch.randn(B, T, kw["d_model"]).to(torch.bfloat16)
+    with torch.no_grad():
+        y_ref, st_ref = ref.layer_forward(cfg, p, x[2:3].float(), return_state=True)
+        proj = layer.in_proj(x.to(dev)).contiguous()
+        assert _native.prefill_kernel_name(layer._desc(B, T, proj), proj) == "mfma_general"
+        y, st = layer.ssd_from_proj(proj, return_state=True)
+        assert max_rel(layer.out_proj(y[2:3]).float(), y_ref) < BF16_TOL
+        for b in (2, B - 1):
+            y1, st1 = layer.ssd_from_proj(proj[b:b + 1].contiguous(), return_state=True)
+            assert torch.equal(y1, y[b:b + 1])
+            for k in ("h", "prev_BX", "angle"):
+                assert torch.equal(st1[k], st[k][b:b + 1]), k
+    for k in ("h", "prev_BX", "angle"):
+        assert max_rel(st[k][2:3], st_ref[k]) < BF16_TOL, k
+
+
+@pytest.mark.parametrize("kw,T", [
+    (dict(d_model=512, d_state=64, headdim=64, mimo_rank=2), 1100),
+    (dict(d_model=512, d_state=256, headdim=128, mimo_rank=1), 3000),
+])
+def test_general_kernel_in_smaller_workspaces(kw, T, cuda_device):
+    """The general kernel's results do not depend on its workspace: two sequences at once, one
+    at a time (a workspace of one sequence's size), and one sequence's five segments in groups
+    (a workspace of one to two states less), bit for bit."""
+    print(f"smaller workspaces {kw} T {T}", flush=True)
+    dev = cuda_device
+    torch.manual_seed(23)
+    layer = mamba3_amd.KulaMamba(**kw).to(dev, torch.bfloat16).eval()
+    H, P, N = layer.nheads, layer.headdim, layer.d_state
+    with torch.no_grad():
+        proj = layer.in_proj(torch.randn(2, T, kw["d_model"], device=dev, dtype=torch.bfloat16))
+    ds = torch.rand(2, T, H, device=dev) + 0.5
+    one = _native.prefill_workspace_bytes(layer._desc(1, T, proj))
+
+    def call(B, nbytes):
+        desc = layer._desc(B, T, proj)
+        assert _native.prefill_kernel_name(desc, proj) == "mfma_general"
+        full = _native.prefill_workspace_bytes(desc)
+        outs = (torch.empty(B, T, layer.d_inner, device=dev, dtype=torch.bfloat16),
+                *(torch.empty(B, H, *s, device=dev) for s in ((P, N), (N // 2,), (P, N))))
+        nbytes = full if nbytes is None else nbytes
+        assert nbytes <= full
+        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+        _native.prefill_fwd(desc, layer._param_pack(), proj, ds, *outs, ws, nbytes)
+        return outs
+
+    whole = call(2, None)
+    state = H * P * N * 4
+    for B, nbytes in ((2, one), (1, one), (1, one - state), (1, one - 2 * state)):
+        for a, b in zip(call(B, nbytes), whole):
+            assert torch.equal(a, b[:B]), (B, nbytes)
