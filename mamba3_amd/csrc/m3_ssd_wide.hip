@@ -153,6 +153,12 @@ __host__ __device__ inline int64_t seg_start(int i, int seg0) {
 // Keeps the LDS reads issued above ahead of the LDS writes that follow.
 #define M3_LDS_ORDER() asm volatile("" ::: "memory")
 
+// v, rounded to fp32: keeps the product behind v out of a fused conversion.
+__device__ __forceinline__ float opaque_f(float v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
 __device__ __forceinline__ float readlane(float v, int l) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
@@ -323,12 +329,72 @@ __device__ __forceinline__ unsigned rotate_pair(unsigned word, f16x2 kA, f16x2 k
 
 __device__ __forceinline__ float bf(unsigned u) { return __builtin_bit_cast(float, u << 16); }
 
+// One of the causal score tiles (ti, ui), ui <= ti, listed row by row as 0..9. A lane's four u-rows
+// 16 ui + 4 g16 + v cover NU tokens; their mask factors are read (unconditionally: every index
+// is below Q) and formed before the contraction. The skip term D enters the masked scores,
+// which carry 1 / (sB sC).
+template <int N, int R, typename SM>
+__device__ __forceinline__ void score_tile(SM& sm, const Tok& tk, int idx, int l16, int g16, float Dh) {
+    constexpr int KN = N / 32;
+    const int ti = idx < 1 ? 0 : idx < 3 ? 1 : idx < 6 ? 2 : 3;
+    const int ui = idx - ti * (ti + 1) / 2;
+    constexpr int NU = R >= 4 ? 1 : 4 / R;
+    const unsigned trow = 16 * ti + l16, t = trow / R;
+    const unsigned ub = (unsigned)(16 * ui + 4 * g16) / R;
+    const f16* pa = &sm.B[16 * ui + l16][8 * g16];
+    const f16* pb = &sm.C[16 * ti + l16][8 * g16];
+    const float ct = tk.c2[t];
+    float fu[NU];
+#pragma unroll
+    for (int j = 0; j < NU; ++j) {
+        const unsigned u = ub + j;
+        const float e = __builtin_amdgcn_exp2f(ct - tk.c2[u]);
+        const float ab = fmaf(tk.bv[u], u < t ? 1.f : 0.f, tk.av[u]);
+        fu[j] = u <= t ? e * ab : 0.f;
+    }
+    f32x4 sacc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KN; ++s) {
+        const f16x8 A = *reinterpret_cast<const f16x8*>(pa + 32 * s);
+        const f16x8 Bo = *reinterpret_cast<const f16x8*>(pb + 32 * s);
+        sacc = mfma16(A, Bo, sacc);
+    }
+    // lane: u-row 16 ui + 4 g16 + v, t-row 16 ti + l16
+    f16x4 sv;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const float val = sacc[v] * fu[v * NU / 4];
+        sv[v] = (f16)(16 * ui + 4 * g16 + v == (int)trow ? val + Dh : val);
+    }
+    *reinterpret_cast<f16x4*>(&sm.S[trow][16 * ui + 4 * g16]) = sv;
+}
+
+// Waves beside the column and the helper waves: one computes the token scalars, the others take
+// score tiles. As many as registers and the 16 waves of a workgroup leave: none beside four
+// column groups of d_state 128 and 256 (helper 3 has the token scalars there) or where the
+// waves would spill. With few column waves a chunk's time is that of its longest helper: of
+// 6,650 cycles at d_state 128 rank 4 in one column group, the token wave's angles, scalars and
+// scores took 4,100.
 template <int N, int R, int NCG, bool FULL>
-__global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
-                             N == 256 ? (2 * NCG + Layout<N, R>::HELPERS + 3) / 4 : 4) void ssd_wide(Args a) {
+constexpr int extra_waves() {
+    if (N != 64 && (NCG == 4 || (N == 256 && NCG == 2))) return 0;
+    if (!FULL) return 1;
+    if (N == 64) return R == 1 && NCG == 4 ? 0 : 4;
+    return N == 256 ? 2 : NCG == 2 ? 4 : 6;
+}
+template <int N, int R, int NCG, bool FULL>
+constexpr int kExtra = extra_waves<N, R, NCG, FULL>();
+template <int N, int R, int NCG, bool FULL>
+constexpr int kWaves = 2 * NCG + Layout<N, R>::HELPERS + kExtra<N, R, NCG, FULL>;
+
+template <int N, int R, int NCG, bool FULL>
+__global__ __launch_bounds__((64 * kWaves<N, R, NCG, FULL>),
+                             (N == 256 ? (kWaves<N, R, NCG, FULL> + 3) / 4 : 4)) void ssd_wide(Args a) {
     using L = Layout<N, R>;
     constexpr int Q = L::Q, LPT = L::LPT, GR = L::GR, TPT = L::TPT, HELPERS = L::HELPERS;
     constexpr int CW = 2 * NCG;     // column waves
+    constexpr int EXTRA = kExtra<N, R, NCG, FULL>;
+    constexpr int TILERS = EXTRA > 0 ? EXTRA - 1 : 0;  // extra waves that take score tiles, two each
     constexpr int NH = N / 2;       // RoPE pairs
     constexpr int NR = N * R;
     constexpr int NT = N / 32;      // state row tiles of a wave (half of n)
@@ -377,7 +443,7 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
     const F16Scales scl = sm.scl.in_sgprs();
     const int hp = h * a.P + p0;  // first column of this block in x, z and y
     if constexpr (FULL) {
-        for (int e = tid; e < PC * R; e += 64 * (CW + HELPERS)) {
+        for (int e = tid; e < PC * R; e += 64 * (CW + HELPERS + EXTRA)) {
             sm.gate[e / R][0][e % R] = a.prm.mimo_z[(int64_t)hp * R + e];
             sm.gate[e / R][1][e % R] = a.prm.mimo_down[(int64_t)hp * R + e] * scl.out;
         }
@@ -413,6 +479,8 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
     static_assert(XT >= 1 && XV * XP == XT * R, "whole X pieces");
     typedef f16 xpiece __attribute__((ext_vector_type(XP)));
     xpiece xo[FULL ? XV : 1], xw[XV];
+    // (The weighted product rounds to fp32 before it rounds to f16, in both passes: the compiler
+    // may fuse the two into one rounding in either.)
     auto form_x = [&](int kk) {
         const Tok& tk = sm.tok[kk % 3];
 #pragma unroll
@@ -423,7 +491,7 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
             for (int r = 0; r < R; ++r) {
                 const float v = xval * mx[r];
                 if constexpr (FULL) xo[(m * R + r) / XP][(m * R + r) % XP] = (f16)v;
-                xw[(m * R + r) / XP][(m * R + r) % XP] = (f16)(v * w);
+                xw[(m * R + r) / XP][(m * R + r) % XP] = (f16)opaque_f(v * w);
             }
         }
     };
@@ -431,7 +499,7 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
 #pragma unroll
         for (int v = 0; v < XV; ++v) *reinterpret_cast<xpiece*>(&sm.XwT[xp][xt0 * R + XP * v]) = xw[v];
     };
-    // token scalars: lane t = token t of the chunk (helper 3)
+    // token scalars: lane t = token t of the chunk
     unsigned rdt0 = 0, rlam0 = 0, rdt1 = 0, rlam1 = 0;
     float sc0 = 1.f, sc1 = 1.f;
     auto load_tokens = [&](int kk) {
@@ -450,7 +518,9 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
             sc1 = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rd, od + a.H * 4, 0, 0));
         }
     };
+    // (No contraction, here and in the angles: the state pass and the full pass round alike.)
     auto prep_tokens = [&](int kk) {
+#pragma clang fp contract(off)
         const int s0 = tbeg + kk * Q;
         const int t = lane;
         const bool v0 = t < Q && s0 + t < T, v1 = t < Q && s0 + t + 1 < T;
@@ -660,11 +730,38 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
                 for (int pt = 0; pt < 2; ++pt) hs[(2 * t + pt) * 64] = hacc[t][pt];
             if (wave == 0 && lane == 0 && pblk == 0) a.lseg[(int64_t)seg * sbase + bh] = ldec;
         }
+    } else if (EXTRA > 0 && wave >= CW + HELPERS) {
+        // =============================== extra waves ===============================
+        __builtin_amdgcn_s_setprio(3);
+        const int ew = wave - CW - HELPERS;
+        const bool token_wave = ew == TILERS;
+        const float Dh = a.prm.D[h] * scl.inv_bc;
+        if (token_wave) {
+            load_tokens(0);
+            prep_tokens(0);
+            load_tokens(1);
+            prep_tokens(1);
+            load_tokens(2);
+        }
+        __syncthreads();  // token scalars of chunk 0 and 1
+        __syncthreads();  // angle sums of chunk 0
+        __syncthreads();  // angles of chunk 0
+        __syncthreads();  // tiles of chunk 0, angle sums of chunk 1
+        for (int k = 0; k < nchunks; ++k) {
+            if (token_wave) {
+                prep_tokens(k + 2);
+                load_tokens(k + 3);
+            } else if constexpr (FULL) {
+#pragma unroll 1
+                for (int idx = ew; idx < 2 * TILERS && idx < 10; idx += TILERS) score_tile<N, R>(sm, sm.tok[k % 3], idx, l16, g16, Dh);
+            }
+            __syncthreads();
+            __syncthreads();
+        }
     } else {
         // =============================== helper waves ===============================
         __builtin_amdgcn_s_setprio(3);  // the helpers' chains end both phases; the column waves have slack
         const int hw = wave - CW, htid = tid - 64 * CW;
-        // the skip term D enters the masked scores, which carry 1 / (sB sC)
         const float Dh = a.prm.D[h] * scl.inv_bc;
         const f16* Bn = a.Bn + (int64_t)b * T * nrs + (int64_t)grp * NR;
         const f16* Cn = a.Cn + (int64_t)b * T * nrs + (int64_t)grp * NR;
@@ -723,8 +820,8 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
 #pragma unroll
             for (int m = 0; m < TPT; ++m) {
                 const float dt = tk.dt[tg * TPT + m];
-                ps[0] += dt * bf(pth[1][m]);
-                ps[1] += dt * __builtin_bit_cast(float, pth[1][m] & 0xffff0000u);
+                ps[0] = fmaf(dt, bf(pth[1][m]), ps[0]);
+                ps[1] = fmaf(dt, __builtin_bit_cast(float, pth[1][m] & 0xffff0000u), ps[1]);
             }
             *reinterpret_cast<f32x2*>(&sm.part[tg][2 * hl]) = ps;
         };
@@ -753,8 +850,8 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
                 kA[m][0] = kA[m][1] = f16x2{(f16)1.f, (f16)0.f};
                 if (a.cplx) {
                     const float dt = tk.dt[tg * TPT + m];
-                    ph[0] -= dt * bf(pth[0][m]);
-                    ph[1] -= dt * __builtin_bit_cast(float, pth[0][m] & 0xffff0000u);
+                    ph[0] = fmaf(-dt, bf(pth[0][m]), ph[0]);
+                    ph[1] = fmaf(-dt, __builtin_bit_cast(float, pth[0][m] & 0xffff0000u), ph[1]);
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         float sn, cs;
@@ -786,7 +883,7 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
 #pragma unroll
             for (int m = 0; m < TPT; ++m) pth[0][m] = pth[1][m];
         };
-        const bool token_wave = hw == 3;
+        const bool token_wave = EXTRA == 0 && hw == 3;
 
         // Prologue: chunks 0 and 1's token scalars, chunk 0's tiles, chunk 1's angle sums and
         // reads (chunks past the end read as zero).
@@ -838,45 +935,8 @@ __global__ __launch_bounds__(64 * (2 * NCG + Layout<N, R>::HELPERS),
                 load_tokens(k + 3);
             }
             if constexpr (FULL) {
-                // Causal score tiles (ti, ui), ui <= ti, listed row by row as 0..9, dealt to the
-                // helpers in turn. A lane's four u-rows 16 ui + 4 g16 + v cover NU tokens; their
-                // mask factors are read (unconditionally: every index is below Q) and formed
-                // before the contraction.
-                const Tok& tk = sm.tok[k % 3];
 #pragma unroll 1
-                for (int idx = hw; idx < 10; idx += HELPERS) {
-                    const int ti = idx < 1 ? 0 : idx < 3 ? 1 : idx < 6 ? 2 : 3;
-                    const int ui = idx - ti * (ti + 1) / 2;
-                    constexpr int NU = R >= 4 ? 1 : 4 / R;
-                    const unsigned trow = 16 * ti + l16, t = trow / R;
-                    const unsigned ub = (unsigned)(16 * ui + 4 * g16) / R;
-                    const f16* pa = &sm.B[16 * ui + l16][8 * g16];
-                    const f16* pb = &sm.C[16 * ti + l16][8 * g16];
-                    const float ct = tk.c2[t];
-                    float fu[NU];
-#pragma unroll
-                    for (int j = 0; j < NU; ++j) {
-                        const unsigned u = ub + j;
-                        const float e = __builtin_amdgcn_exp2f(ct - tk.c2[u]);
-                        const float ab = fmaf(tk.bv[u], u < t ? 1.f : 0.f, tk.av[u]);
-                        fu[j] = u <= t ? e * ab : 0.f;
-                    }
-                    f32x4 sacc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int s = 0; s < KN; ++s) {
-                        const f16x8 A = *reinterpret_cast<const f16x8*>(pa + 32 * s);
-                        const f16x8 Bo = *reinterpret_cast<const f16x8*>(pb + 32 * s);
-                        sacc = mfma16(A, Bo, sacc);
-                    }
-                    // lane: u-row 16 ui + 4 g16 + v, t-row 16 ti + l16
-                    f16x4 sv;
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const float val = sacc[v] * fu[v * NU / 4];
-                        sv[v] = (f16)(16 * ui + 4 * g16 + v == (int)trow ? val + Dh : val);
-                    }
-                    *reinterpret_cast<f16x4*>(&sm.S[trow][16 * ui + 4 * g16]) = sv;
-                }
+                for (int idx = 2 * TILERS + hw; idx < 10; idx += HELPERS) score_tile<N, R>(sm, sm.tok[k % 3], idx, l16, g16, Dh);
             }
             __syncthreads();
             // ---- output ----
@@ -945,8 +1005,9 @@ __global__ __launch_bounds__(256) void seg_combine(Args a) {
         float s0, c0, s1, c1;
         fast_sincos(phi[0], s0, c0);
         fast_sincos(phi[1], s1, c1);
-        h = h * dec + f32x4{v[0] * c0 - v[1] * s0, v[0] * s0 + v[1] * c0,
-                            v[2] * c1 - v[3] * s1, v[2] * s1 + v[3] * c1};
+        // (the first segment's state is in the sequence's frame already)
+        h = j == 0 ? v : h * dec + f32x4{v[0] * c0 - v[1] * s0, v[0] * s0 + v[1] * c0,
+                                         v[2] * c1 - v[3] * s1, v[2] * s1 + v[3] * c1};
         *hj = h;
         phi += inc;
     }
@@ -956,16 +1017,15 @@ __global__ __launch_bounds__(256) void seg_combine(Args a) {
 template <int N, int R, int NCG>
 void launch_ssd(Args a, int group, hipStream_t stream) {
     const unsigned npairs = (unsigned)(a.B * a.H * a.PS);
-    const dim3 threads(64 * (2 * NCG + Layout<N, R>::HELPERS));
     for (a.lo = 0; a.lo < a.segs; a.lo = a.hi) {
         a.hi = std::min(a.segs, a.lo + group);
         const int ns = std::min(a.hi, a.segs - 1) - a.lo;
         if (ns > 0) {
-            hipLaunchKernelGGL((ssd_wide<N, R, NCG, false>), dim3(npairs * ns), threads, 0, stream, a);
+            hipLaunchKernelGGL((ssd_wide<N, R, NCG, false>), dim3(npairs * ns), dim3(64 * kWaves<N, R, NCG, false>), 0, stream, a);
             hipLaunchKernelGGL((seg_combine<N, NCG>), dim3((unsigned)(((int64_t)npairs * PW * NCG * N / 4 + 255) / 256)),
                                dim3(256), 0, stream, a);
         }
-        hipLaunchKernelGGL((ssd_wide<N, R, NCG, true>), dim3(npairs * (a.hi - a.lo)), threads, 0, stream, a);
+        hipLaunchKernelGGL((ssd_wide<N, R, NCG, true>), dim3(npairs * (a.hi - a.lo)), dim3(64 * kWaves<N, R, NCG, true>), 0, stream, a);
     }
 }
 
@@ -995,7 +1055,12 @@ void lay_out(const m3_layer_desc& d, Plan& p) {
 // below), nor, as they lie at fixed tokens, on the length, so that a prefix gives the same
 // bits too. They are closer at the start, so that a short prompt splits finely and a long one
 // into few states. Heads whose column blocks alone nearly fill the 256 CUs are not cut: a
-// segmented walk does 1.5x the work (its state pass).
+// segmented walk does 1.5x the work (its state pass). (us per call, cut / uncut: d_state 64
+// headdim 64 rank 2, one sequence of 2,048 tokens: 96 heads 130 / 190, 160 171 / 214, 190
+// 201 / 224, of 600 tokens 69 / 67, 78 / 75, 96 / 77; d_state 256 headdim 128 rank 4, 32
+// heads: (1, 16384) 1,030 / 2,789, (2, 16384) 2,072 / 2,956, but (8, 2048) 1,068 / 656.)
+// The first cut is free, as the state at it is the walk's own: up to two segments a sequence
+// is walked in one piece with the same bits ((1, 600) of that layer 132 us, 199 cut).
 //
 // A workspace that does not hold every segment's state takes the batch in slices, and one
 // that does not hold those of one sequence takes its segments in groups, from two states on:
@@ -1007,7 +1072,7 @@ Plan make_plan(const m3_layer_desc& d, size_t limit) {
     const int64_t blocks = d.headdim / (PW * p.ncg);
     p.seg0 = std::max(256, d.headdim * d.d_state / 64);
     p.segs = 1;
-    if (d.nheads * blocks < 192 && d.seqlen > p.seg0)
+    if (d.nheads * blocks < 192 && d.seqlen > 2 * p.seg0)
         while (seg_start(p.segs, p.seg0) < d.seqlen) ++p.segs;
     p.batch = d.batch;
     p.slots = std::max(p.segs - 1, 1);

@@ -1031,16 +1031,17 @@ def test_general_kernel_column_blocks_agree(N, R, P, cuda_device):
 
 
 @pytest.mark.parametrize("kw,T", [
-    (dict(d_model=64, d_state=64, headdim=64, mimo_rank=2), 257),     # second segment of one token
+    (dict(d_model=64, d_state=64, headdim=64, mimo_rank=2), 513),     # third segment of one token
     (dict(d_model=64, d_state=64, headdim=32, mimo_rank=1, ngroups=2), 1100),  # into the 512-token segments
     (dict(d_model=64, d_state=128, headdim=64, mimo_rank=4, use_trapezoidal=False), 600),
-    (dict(d_model=64, d_state=256, headdim=128, mimo_rank=4, use_complex_ssm=False), 520),
-    (dict(d_model=128, d_state=256, headdim=128, mimo_rank=1), 513),
+    (dict(d_model=64, d_state=256, headdim=128, mimo_rank=4, use_complex_ssm=False), 1040),
+    (dict(d_model=128, d_state=256, headdim=128, mimo_rank=1), 1025),
 ])
 def test_general_kernel_segments_match_fp32_oracle(kw, T, cuda_device):
     """Sequences cut into segments (state pass, combine, full pass) with dt_scale against the
     fp32 oracle, and as one walk in a workspace without room for the segments' states; a
-    prefix that ends inside the segmented run reproduces it bit for bit."""
+    prefix reproduces the segmented run bit for bit, also one that is short enough to be
+    walked in one piece."""
     print(f"segments {kw} T {T}", flush=True)
     dev = cuda_device
     layer, cfg, p = _bf16_pair(kw, dev, seed=17)
@@ -1069,11 +1070,11 @@ def test_general_kernel_segments_match_fp32_oracle(kw, T, cuda_device):
 
 
 @pytest.mark.parametrize("kw,T", [
-    (dict(d_model=512, d_state=64, headdim=64, mimo_rank=2), 257),    # two column groups a block
-    (dict(d_model=1024, d_state=64, headdim=128, mimo_rank=2), 300),  # four
-    (dict(d_model=1024, d_state=128, headdim=128, mimo_rank=1), 290),
-    (dict(d_model=1024, d_state=256, headdim=128, mimo_rank=4), 513),
-    (dict(d_model=512, d_state=256, headdim=64, mimo_rank=1), 257),
+    (dict(d_model=512, d_state=64, headdim=64, mimo_rank=2), 513),    # two column groups a block
+    (dict(d_model=1024, d_state=64, headdim=128, mimo_rank=2), 600),  # four
+    (dict(d_model=1024, d_state=128, headdim=128, mimo_rank=1), 577),
+    (dict(d_model=1024, d_state=256, headdim=128, mimo_rank=4), 1025),
+    (dict(d_model=512, d_state=256, headdim=64, mimo_rank=1), 513),
 ])
 def test_general_kernel_segments_in_wide_blocks_and_any_batch(kw, T, cuda_device):
     """Sequences cut into segments, in a batch whose 192 (batch, head) pairs run in blocks of
