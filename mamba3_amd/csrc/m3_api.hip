@@ -74,11 +74,12 @@ PrefillPath prefill_path(const m3_layer_desc& d, const void* proj, const void* y
     return PrefillPath::kGeneric;
 }
 
+// The least workspace that a path runs in (within `limit`, the staged bf16 path).
 size_t prefill_path_workspace(const m3_layer_desc& d, PrefillPath path, size_t limit) {
     switch (path) {
         case PrefillPath::kMfma: return m3::mfma_prefill_workspace(d);
         case PrefillPath::kWide: return m3::wide_prefill_min_workspace(d);
-        case PrefillPath::kFp32Fused: return m3::fused_fp32_prefill_workspace(d, limit);
+        case PrefillPath::kFp32Fused: return m3::fused_fp32_prefill_min_workspace(d);
         case PrefillPath::kFp32FusedTrain:
         case PrefillPath::kFp32: return m3::fp32_layer_workspace(d);
         case PrefillPath::kStagedBf16: return m3::staged_bf16_workspace(d, limit);
@@ -110,13 +111,9 @@ int launch_prefill_path(PrefillPath path, const m3_layer_desc& d, const m3_layer
         case PrefillPath::kFp32Fused:
             return m3::launch_fused_fp32_prefill(d, p, proj, dt_scale, y_out, h_final, angle,
                                                  prev_bx, ws, limit, stream);
-        case PrefillPath::kFp32FusedTrain: {
-            const m3::Fp32LayerParts parts = m3::fp32_layer_parts(d, ws);
-            size_t bytes = 0;
-            void* scratch_rows = m3::fp32_layer_scratch(d, ws, &bytes);
-            return m3::launch_fused_fp32_prefill(d, p, proj, dt_scale, y_out, h_final, angle,
-                                                 prev_bx, scratch_rows, bytes, stream, &parts);
-        }
+        case PrefillPath::kFp32FusedTrain:
+            return m3::launch_fused_fp32_train(d, p, proj, dt_scale, y_out, h_final, angle,
+                                               prev_bx, ws, limit, stream);
         case PrefillPath::kFp32:
             return m3::launch_fp32_layer(d, p, proj, dt_scale, y_out, h_final, angle, prev_bx,
                                          ws, stream) == 0
@@ -248,7 +245,9 @@ static size_t prefill_workspace(const m3_layer_desc& d) {
     size_t n = m3::generic_prefill_workspace(d);
     n = std::max(n, m3::fp32_layer_workspace(d));
     if (m3::fused_fp32_prefill_supported(d, nullptr, nullptr, nullptr, nullptr))
-        n = std::max(n, m3::fused_fp32_prefill_workspace(d, SIZE_MAX));
+        n = std::max(n, m3::fused_fp32_prefill_workspace(d));
+    if ((d.flags & M3_FLAG_FOR_BACKWARD) && m3::fused_fp32_train_supported(d, nullptr, nullptr, nullptr, nullptr))
+        n = std::max(n, m3::fused_fp32_train_workspace(d));
     if (m3::mfma_prefill_supported(d, nullptr, nullptr)) n = std::max(n, m3::mfma_prefill_workspace(d));
     if (m3::wide_prefill_supported(d)) n = std::max(n, m3::wide_prefill_workspace(d));
     else n = std::max(n, m3::staged_bf16_workspace(d, SIZE_MAX));

@@ -133,13 +133,18 @@ bool fused_fp32_train_supported(const m3_layer_desc& d, const void* proj, const 
                                 const void* h_final, const void* prev_bx);
 // The chunk-kernel region of the fp32 layer workspace (pointer into ws, and its size).
 void* fp32_layer_scratch(const m3_layer_desc& d, void* ws, size_t* bytes);
-// Workspace within `limit` bytes where its segments' states fit, else that of one walk per
-// (batch, head); the launcher takes the bytes of its workspace.
-size_t fused_fp32_prefill_workspace(const m3_layer_desc& d, size_t limit);
+// Workspace of a call in one piece, and the least one that it runs in; the launchers take the
+// bytes of their workspace. The training forward's is the fp32 layer's and, where that has no
+// gap for the segments' states, those behind it.
+size_t fused_fp32_prefill_workspace(const m3_layer_desc& d);
+size_t fused_fp32_prefill_min_workspace(const m3_layer_desc& d);
+size_t fused_fp32_train_workspace(const m3_layer_desc& d);
 int launch_fused_fp32_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                               const float* dt_scale, void* y_out, float* h_final, float* angle,
-                              float* prev_bx, void* workspace, size_t limit, hipStream_t stream,
-                              const Fp32LayerParts* stage = nullptr);
+                              float* prev_bx, void* workspace, size_t limit, hipStream_t stream);
+int launch_fused_fp32_train(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
+                            const float* dt_scale, void* y_out, float* h_final, float* angle,
+                            float* prev_bx, void* workspace, size_t limit, hipStream_t stream);
 size_t fp32_layer_workspace(const m3_layer_desc& d);
 int launch_fp32_layer(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                       const float* dt_scale, void* y_out, float* h_final, float* angle,

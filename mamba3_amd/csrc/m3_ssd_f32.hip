@@ -11,7 +11,7 @@
 // Launches:
 //   1. bc_norm_f32: per (token, group), B^ = RMSNorm(B) * w + bias and C^ likewise, fp32, in
 //      the reference's (n, r) order (mamba3/mamba3.py:19-35, 147-157).
-//   2. with few (batch, head) pairs (seg_plan), ssd_f32<false>: a state-only walk of every
+//   2. for sequences of more than two segments, ssd_f32<false>: a state-only walk of every
 //      segment of the sequence but the last, from a zero state in its own RoPE frame, and
 //      seg_combine_f32, which turns the end states into the states entering each segment;
 //   3. ssd_f32<true>: one 768-thread workgroup per (batch, head, segment) walks its chunks of
@@ -48,6 +48,7 @@
 #include "m3_common.h"
 #include "m3_kernels.h"
 #include "m3_mfma.h"
+#include "m3_segments.h"
 
 namespace m3 {
 namespace f32k {
@@ -115,21 +116,18 @@ struct Args {
     // backward's chunking: the state entering every hs_every-th chunk k at entry k / hs_every
     // of (B, hs_K + 1, H, P, N) (the zero start at entry 0), and the final state at entry hs_K.
     int hs_every, hs_K;
-    // segments of the sequence (segs = 1: none) and the state pass's results, per segment but
-    // the last and (batch, head): end state [wave][tile][lane] (seg_combine_f32 turns it into
-    // the state entering the next segment), log-decay, RoPE angle increments
+    // segments of the sequence (segs = 1: none), of which a launch takes lo .. hi - 1, and the
+    // state pass's results, per segment but the last and (batch, head): end state
+    // [slot][wave][tile][lane] (seg_combine_f32 turns it into the state entering the next
+    // segment; that entering segment e is in slot (e - 1) % slots), log-decay, RoPE angle increments
     int segs;
+    int lo, hi, slots;
     f32x4* hseg;
     float* lseg;
     float* aseg;
 };
 
-// First token of segment i: four segments each of kSeg0, 2 kSeg0 and 4 kSeg0 tokens, then 16 kSeg0.
-constexpr int kSeg0 = 128;
-__host__ __device__ inline int64_t seg_start(int i) {
-    const int u = i <= 4 ? i : i <= 8 ? 4 + 2 * (i - 4) : i <= 12 ? 12 + 4 * (i - 8) : 28 + 16 * (i - 12);
-    return (int64_t)u * kSeg0;
-}
+constexpr int kSeg0 = 128;  // tokens of the first segments (seg_start)
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -223,13 +221,13 @@ __global__ __launch_bounds__(THREADS, 3) void ssd_f32(Args a) {
     const int npairs = a.B * a.H;
     // Segments longest first; within one, consecutive (batch, head) pairs share an XCD.
     const int j0 = blockIdx.x % npairs;
-    const int seg = (FULL ? a.segs : a.segs - 1) - 1 - (int)(blockIdx.x / npairs);
+    const int seg = (FULL ? a.hi : min(a.hi, a.segs - 1)) - 1 - (int)(blockIdx.x / npairs);
     const int bh = (npairs % 8 == 0) ? (j0 % 8) * (npairs / 8) + j0 / 8 : j0;
     const int b = bh / a.H, h = bh % a.H;
     const int grp = h / (a.H / a.G);
     const int T = a.T;
-    const int tbeg = (int)seg_start(seg);
-    const int tend = seg + 1 < a.segs ? (int)seg_start(seg + 1) : T;
+    const int tbeg = (int)seg_start(seg, kSeg0);
+    const int tend = seg + 1 < a.segs ? (int)seg_start(seg + 1, kSeg0) : T;
     const int K = (tend - tbeg + Q - 1) / Q;
     const int k0 = tbeg / Q;              // the segment's first chunk in the sequence
     const int KT = (T + Q - 1) / Q;
@@ -251,7 +249,7 @@ __global__ __launch_bounds__(THREADS, 3) void ssd_f32(Args a) {
 #pragma unroll
         for (int t = 0; t < NT; ++t) hacc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (FULL && seg > 0) {
-            const f32x4* hs = a.hseg + (((int64_t)(seg - 1) * npairs + bh) * CW + wave) * (NT * 64) + lane;
+            const f32x4* hs = a.hseg + (((int64_t)((seg - 1) % a.slots) * npairs + bh) * CW + wave) * (NT * 64) + lane;
 #pragma unroll
             for (int t = 0; t < NT; ++t) hacc[t] = hs[t * 64];
         }
@@ -424,7 +422,7 @@ __global__ __launch_bounds__(THREADS, 3) void ssd_f32(Args a) {
                 }
             }
         } else {
-            f32x4* hs = a.hseg + (((int64_t)seg * npairs + bh) * CW + wave) * (NT * 64) + lane;
+            f32x4* hs = a.hseg + (((int64_t)(seg % a.slots) * npairs + bh) * CW + wave) * (NT * 64) + lane;
 #pragma unroll
             for (int t = 0; t < NT; ++t) hs[t * 64] = hacc[t];
             if (wave == 0 && lane == 0) a.lseg[(int64_t)seg * npairs + bh] = ldec;
@@ -785,43 +783,40 @@ __global__ __launch_bounds__(256) void seg_combine_f32(Args a) {
     const int i = (16 * t + 4 * g16) / 2;  // first RoPE pair
     f32x4 h = f32x4{0.f, 0.f, 0.f, 0.f};
     f32x2 phi = f32x2{0.f, 0.f};
+    auto slot = [&](int j) { return a.hseg + (int64_t)(j % a.slots) * npairs * PER + e; };
+    auto angle_inc = [&](int j) {
+        return *reinterpret_cast<const f32x2*>(a.aseg + ((int64_t)j * npairs + bh) * NH + i);
+    };
+    if (a.lo > 0) h = *slot(a.lo - 1);
+    for (int j = 0; j < a.lo; ++j) phi += angle_inc(j);
+    const int hi = min(a.hi, a.segs - 1);
 #pragma unroll 2
-    for (int j = 0; j < a.segs - 1; ++j) {
-        f32x4* hj = a.hseg + (int64_t)j * npairs * PER + e;
+    for (int j = a.lo; j < hi; ++j) {
+        f32x4* hj = slot(j);
         const f32x4 v = *hj;
-        const f32x2 inc = *reinterpret_cast<const f32x2*>(a.aseg + ((int64_t)j * npairs + bh) * NH + i);
+        const f32x2 inc = angle_inc(j);
         const float dec = expf(a.lseg[(int64_t)j * npairs + bh]);
         float s0, c0, s1, c1;
         sincosf(phi[0], &s0, &c0);
         sincosf(phi[1], &s1, &c1);
-        h = h * dec + f32x4{v[0] * c0 - v[1] * s0, v[0] * s0 + v[1] * c0,
-                            v[2] * c1 - v[3] * s1, v[2] * s1 + v[3] * c1};
+        // (the first segment's state is in the sequence's frame already)
+        h = j == 0 ? v : h * dec + f32x4{v[0] * c0 - v[1] * s0, v[0] * s0 + v[1] * c0,
+                                         v[2] * c1 - v[3] * s1, v[2] * s1 + v[3] * c1};
         *hj = h;
         phi += inc;
     }
 }
 
-// Segments of a call (1: one walk per (batch, head)) and the bytes of their states, log-decays
-// and angle increments. The state pass costs about half a walk, so segments pay only while the
-// pairs leave more than half of the 256 CUs idle and the walk is long: whole d_model 768
-// forward, one walk against segments, 48 pairs x 500 tokens 223 / 159 us, 96 x 1024 551 / 475;
-// but 24 x 129 80 / 98, 96 x 200 139 / 146, 144 x 1024 680 / 697, 192 x 1024 782 / 864.
-struct SegPlan {
-    int segs;
-    size_t lseg, aseg, bytes;  // offsets behind the states
-};
-inline size_t al256(size_t n) { return (n + 255) & ~(size_t)255; }
-SegPlan seg_plan(const m3_layer_desc& d, size_t limit) {
-    SegPlan p = {1, 0, 0, 0};
-    const size_t BH = (size_t)d.batch * d.nheads;
-    if (BH >= 128 || d.seqlen <= 2 * kSeg0) return p;
-    int segs = 1;
-    while (seg_start(segs) < d.seqlen) ++segs;
-    const size_t n = segs - 1;
-    const size_t lseg = n * BH * P * N * sizeof(float);
-    const size_t aseg = lseg + al256(n * BH * sizeof(float));
-    const size_t bytes = aseg + al256(n * BH * NH * sizeof(float));
-    return bytes <= limit ? SegPlan{segs, lseg, aseg, bytes} : p;
+// Segments of a sequence, by its heads and tokens alone: not by the batch, so that a sequence
+// gives the same bits alone and in any batch. The state pass costs about half a walk, so segments
+// pay while the (batch, head) pairs leave more than half of the 256 CUs idle, and more pairs pay
+// for it. us per call at 24 heads, cut / uncut: (1, 300) 70 / 94, (1, 1000) 125 / 276, (4, 600)
+// 136 / 169, (4, 4096) 681 / 1085; but (8, 300) 157 / 97, (8, 1000) 354 / 279, (8, 2048) 670 / 563.
+int segments(const m3_layer_desc& d) { return d.nheads < 128 ? seg_count(d.seqlen, kSeg0) : 1; }
+
+SegSizes seg_sizes(const m3_layer_desc& d, bool rows) {
+    return {rows ? (size_t)d.seqlen * d.ngroups * NR * sizeof(float) : 0, (size_t)d.nheads * P * N * sizeof(float),
+            d.nheads * sizeof(float), (size_t)d.nheads * NH * sizeof(float)};
 }
 
 }  // namespace f32k
@@ -852,50 +847,55 @@ bool fused_fp32_train_supported(const m3_layer_desc& d, const void* proj, const 
     if (!fused_fp32_shape_ok(d, proj, y_out, h_final, prev_bx) || !fp32_layer_supported(d)) return false;
     size_t bytes = 0;
     fp32_layer_scratch(d, nullptr, &bytes);
-    return bytes >= fused_fp32_prefill_workspace(d, 0);
+    return bytes >= fused_fp32_prefill_min_workspace(d);
 }
 
-// B^ and C^ rows, then the segments' states where `limit` bytes hold them.
-static size_t fused_fp32_rows(const m3_layer_desc& d) {
-    return f32k::al256((size_t)d.batch * d.seqlen * d.ngroups * f32k::NR * sizeof(float));
+static SegPlan fused_fp32_plan(const m3_layer_desc& d, size_t limit) {
+    return plan_segments(d.batch, f32k::segments(d), f32k::seg_sizes(d, true), limit, true);
 }
-size_t fused_fp32_prefill_workspace(const m3_layer_desc& d, size_t limit) {
-    const size_t rows = 2 * fused_fp32_rows(d);
-    return rows + f32k::seg_plan(d, limit > rows ? limit - rows : 0).bytes;
+size_t fused_fp32_prefill_workspace(const m3_layer_desc& d) { return fused_fp32_plan(d, SIZE_MAX).total; }
+size_t fused_fp32_prefill_min_workspace(const m3_layer_desc& d) { return fused_fp32_plan(d, 0).total; }
+
+// The training forward's parts of the fp32 layer workspace's chunk-kernel region: with room for
+// the chunk-start states (Fp32LayerParts::Hs) the C^ rows lie past them and the segments'
+// states between the B^ rows and them, else the segments' states follow both rows.
+struct TrainRegion {
+    size_t cn, seg, room;  // offsets in the region; bytes for the segments' states
+    bool hs;
+};
+static TrainRegion train_region(const m3_layer_desc& d) {
+    const size_t rows = al256((size_t)d.batch * d.seqlen * d.ngroups * f32k::NR * sizeof(float));
+    size_t bytes = 0;
+    fp32_layer_scratch(d, nullptr, &bytes);
+    if (!fp32_layer_hs_ok(d)) return {rows, 2 * rows, bytes > 2 * rows ? bytes - 2 * rows : 0, false};
+    const size_t off = chunked_fwd_hs_offset(d.batch, d.seqlen, d.nheads, d.headdim, d.d_state, d.mimo_rank,
+                                             d.use_trapezoidal != 0);
+    return {off + al256(fp32_layer_hs_bytes(d)), rows, off > rows ? off - rows : 0, true};
 }
 
-int launch_fused_fp32_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
-                              const float* dt_scale, void* y_out, float* h_final, float* angle,
-                              float* prev_bx, void* workspace, size_t limit, hipStream_t stream,
-                              const Fp32LayerParts* stage) {
+size_t fused_fp32_train_workspace(const m3_layer_desc& d) {
+    const SegPlan p = plan_segments(d.batch, f32k::segments(d), f32k::seg_sizes(d, false), SIZE_MAX, false);
+    const bool inside = p.segs == 1 || p.total <= train_region(d).room;
+    return al256(fp32_layer_workspace(d)) + (inside ? 0 : p.total);
+}
+
+// One slice of the batch: B^ rows at bn, C^ rows at cn, the segments' states as the plan lays
+// them out from `seg` on.
+static int launch_fused_fp32_slice(const m3_layer_desc& d, const m3_layer_params& p, const float* proj,
+                                   const float* dt_scale, float* y_out, float* h_final, float* angle,
+                                   float* prev_bx, float* bn, float* cn, char* seg, const SegPlan& sp,
+                                   hipStream_t stream, const Fp32LayerParts* stage, bool hs) {
     const ProjLayout pl = proj_layout(d);
     const int64_t nrows = (int64_t)d.batch * d.seqlen * d.ngroups;
-    const size_t rows = fused_fp32_rows(d);
-    char* ws = reinterpret_cast<char*>(workspace);
-    float* bn = reinterpret_cast<float*>(ws);
-    float* cn = reinterpret_cast<float*>(ws + rows);
-    char* seg = ws + 2 * rows;  // the segments' states, in room bytes
-    size_t room = limit > 2 * rows ? limit - 2 * rows : 0;
-    // Training forward with room for the chunk-start states (workspace = the fp32 layer
-    // workspace's chunk-kernel region, whose Hs part is stage->Hs): C^ rows past them, the
-    // segments' states between the B^ rows and them.
-    const bool hs = stage && stage->Hs && fp32_layer_hs_ok(d);
     int hs_every = 0, hs_K = 0;
     if (hs) {
-        const bool trap = d.use_trapezoidal != 0;
-        const size_t off = chunked_fwd_hs_offset(d.batch, d.seqlen, d.nheads, d.headdim, d.d_state,
-                                                 d.mimo_rank, trap);
-        const size_t hsb = f32k::al256(fp32_layer_hs_bytes(d));
-        cn = reinterpret_cast<float*>(ws + off + hsb);
-        seg = ws + rows;
-        room = off > rows ? off - rows : 0;
-        const int qb = chunked_chunk_tokens(d.mimo_rank, trap);
+        const int qb = chunked_chunk_tokens(d.mimo_rank, d.use_trapezoidal != 0);
         if (qb % f32k::Q != 0) return M3_ERR_UNSUPPORTED;
         hs_every = qb / f32k::Q;
         hs_K = (d.seqlen + qb - 1) / qb;
     }
     hipLaunchKernelGGL(f32k::bc_norm_f32, dim3((unsigned)((nrows + 3) / 4)), dim3(256), 0, stream,
-                       reinterpret_cast<const float*>(proj), d.proj_row_stride, pl.B, pl.C, d.ngroups,
+                       proj, d.proj_row_stride, pl.B, pl.C, d.ngroups,
                        nrows, d.rms_eps, p.B_norm_w, p.B_bias, p.C_norm_w, p.C_bias, bn, cn);
     f32k::Args a;
     a.B = d.batch; a.T = d.seqlen; a.H = d.nheads; a.G = d.ngroups;
@@ -903,11 +903,11 @@ int launch_fused_fp32_prefill(const m3_layer_desc& d, const m3_layer_params& p, 
     a.rs = d.proj_row_stride;
     a.pl = pl;
     a.prm = p;
-    a.proj = reinterpret_cast<const float*>(proj);
+    a.proj = proj;
     a.dt_scale = dt_scale;
     a.Bn = bn;
     a.Cn = cn;
-    a.y_out = reinterpret_cast<float*>(y_out);
+    a.y_out = y_out;
     a.h_final = h_final;
     a.angle = angle;
     a.prev_bx = prev_bx;
@@ -915,19 +915,65 @@ int launch_fused_fp32_prefill(const m3_layer_desc& d, const m3_layer_params& p, 
     a.stage = stage != nullptr;
     a.hs_every = hs_every;
     a.hs_K = hs_K;
-    const f32k::SegPlan sp = f32k::seg_plan(d, room);
     a.segs = sp.segs;
-    a.hseg = reinterpret_cast<f32x4*>(seg);
+    a.slots = sp.slots;
+    a.hseg = reinterpret_cast<f32x4*>(seg + sp.hseg);
     a.lseg = reinterpret_cast<float*>(seg + sp.lseg);
     a.aseg = reinterpret_cast<float*>(seg + sp.aseg);
     const unsigned bh = (unsigned)(d.batch * d.nheads);
-    if (sp.segs > 1) {
-        hipLaunchKernelGGL(f32k::ssd_f32<false>, dim3(bh * (sp.segs - 1)), dim3(f32k::THREADS), 0, stream, a);
-        hipLaunchKernelGGL(f32k::seg_combine_f32, dim3((unsigned)(((int64_t)bh * f32k::P * f32k::N / 4 + 255) / 256)),
-                           dim3(256), 0, stream, a);
+    for (a.lo = 0; a.lo < a.segs; a.lo = a.hi) {
+        a.hi = std::min(a.segs, a.lo + sp.group);
+        const int ns = std::min(a.hi, a.segs - 1) - a.lo;
+        if (ns > 0) {
+            hipLaunchKernelGGL(f32k::ssd_f32<false>, dim3(bh * ns), dim3(f32k::THREADS), 0, stream, a);
+            hipLaunchKernelGGL(f32k::seg_combine_f32,
+                               dim3((unsigned)(((int64_t)bh * f32k::P * f32k::N / 4 + 255) / 256)), dim3(256), 0,
+                               stream, a);
+        }
+        hipLaunchKernelGGL(f32k::ssd_f32<true>, dim3(bh * (a.hi - a.lo)), dim3(f32k::THREADS), 0, stream, a);
     }
-    hipLaunchKernelGGL(f32k::ssd_f32<true>, dim3(bh * sp.segs), dim3(f32k::THREADS), 0, stream, a);
     return hipGetLastError() == hipSuccess ? M3_OK : M3_ERR_LAUNCH;
+}
+
+int launch_fused_fp32_prefill(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
+                              const float* dt_scale, void* y_out, float* h_final, float* angle,
+                              float* prev_bx, void* workspace, size_t limit, hipStream_t stream) {
+    const SegPlan sp = fused_fp32_plan(d, limit);
+    char* ws = reinterpret_cast<char*>(workspace);
+    const int64_t T = d.seqlen, H = d.nheads;
+    for (int b = 0; b < d.batch; b += sp.batch) {
+        m3_layer_desc part = d;
+        part.batch = std::min(sp.batch, d.batch - b);
+        auto at = [&](auto* q, int64_t per_row) { return q ? q + b * per_row : nullptr; };
+        const int st = launch_fused_fp32_slice(
+            part, p, reinterpret_cast<const float*>(proj) + b * T * d.proj_row_stride, at(dt_scale, T * H),
+            reinterpret_cast<float*>(y_out) + b * T * H * f32k::P, at(h_final, H * f32k::P * f32k::N),
+            at(angle, H * f32k::NH), at(prev_bx, H * f32k::P * f32k::N), reinterpret_cast<float*>(ws),
+            reinterpret_cast<float*>(ws + sp.rows), ws, sp, stream, nullptr, false);
+        if (st != M3_OK) return st;
+    }
+    return M3_OK;
+}
+
+int launch_fused_fp32_train(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
+                            const float* dt_scale, void* y_out, float* h_final, float* angle,
+                            float* prev_bx, void* workspace, size_t limit, hipStream_t stream) {
+    const Fp32LayerParts parts = fp32_layer_parts(d, workspace);
+    size_t bytes = 0;
+    char* region = reinterpret_cast<char*>(fp32_layer_scratch(d, workspace, &bytes));
+    const TrainRegion r = train_region(d);
+    char* seg = region + r.seg;
+    size_t room = r.room;
+    const size_t own = al256(fp32_layer_workspace(d));
+    if (fused_fp32_train_workspace(d) > own && limit > own) {  // behind the layer's workspace
+        seg = reinterpret_cast<char*>(workspace) + own;
+        room = limit - own;
+    }
+    const SegPlan sp = plan_segments(d.batch, f32k::segments(d), f32k::seg_sizes(d, false), room, false);
+    return launch_fused_fp32_slice(d, p, reinterpret_cast<const float*>(proj), dt_scale,
+                                   reinterpret_cast<float*>(y_out), h_final, angle, prev_bx,
+                                   reinterpret_cast<float*>(region), reinterpret_cast<float*>(region + r.cn), seg,
+                                   sp, stream, &parts, r.hs);
 }
 
 }  // namespace m3

@@ -60,6 +60,7 @@
 #include "m3_common.h"
 #include "m3_kernels.h"
 #include "m3_mfma.h"
+#include "m3_segments.h"
 
 namespace m3 {
 namespace wd {
@@ -143,12 +144,6 @@ struct Args {
     float* lseg;  // log2 of the segment's decay, [seg][b h]
     float* aseg;  // its RoPE angle increment, [seg][b h][pair]
 };
-
-// First token of segment i: four segments each of seg0, 2 seg0 and 4 seg0 tokens, then 16 seg0.
-__host__ __device__ inline int64_t seg_start(int i, int seg0) {
-    const int u = i <= 4 ? i : i <= 8 ? 4 + 2 * (i - 4) : i <= 12 ? 12 + 4 * (i - 8) : 28 + 16 * (i - 12);
-    return (int64_t)u * seg0;
-}
 
 // Keeps the LDS reads issued above ahead of the LDS writes that follow.
 #define M3_LDS_ORDER() asm volatile("" ::: "memory")
@@ -1029,30 +1024,9 @@ void launch_ssd(Args a, int group, hipStream_t stream) {
     }
 }
 
-inline size_t al256(size_t n) { return (n + 255) & ~(size_t)255; }
-
-// What a call runs: the cuts of a sequence, and how much of it a workspace holds at a time.
-// Workspace: B^ and C^ rows, then the segments' states, log-decays and angle increments.
-struct Plan {
-    int segs, seg0;
-    int batch;         // sequences per slice
-    int slots, group;  // states kept, segments per group of launches
-    int ncg;           // column groups per workgroup
-    size_t rows, hseg, lseg, aseg, total;  // bytes of B^ (and of C^); offsets; bytes in all
-};
-
-void lay_out(const m3_layer_desc& d, Plan& p) {
-    const size_t n = p.segs - 1, bh = (size_t)p.batch * d.nheads;
-    p.rows = (size_t)p.batch * d.seqlen * d.ngroups * d.d_state * d.mimo_rank * sizeof(f16);
-    p.hseg = al256(2 * p.rows);
-    p.lseg = p.hseg + (n ? al256(p.slots * bh * d.headdim * d.d_state * sizeof(float)) : 0);
-    p.aseg = p.lseg + al256(n * bh * sizeof(float));
-    p.total = n ? p.aseg + n * bh * (d.d_state / 2) * sizeof(float) + 256 : 2 * p.rows + 256;
-}
-
 // The cuts of a sequence depend on nothing but its layer and its tokens: not on the batch, so
 // that a sequence gives the same bits alone and in any batch, nor on the workspace (but see
-// below), nor, as they lie at fixed tokens, on the length, so that a prefix gives the same
+// plan_segments), nor, as they lie at fixed tokens, on the length, so that a prefix gives the same
 // bits too. They are closer at the start, so that a short prompt splits finely and a long one
 // into few states. Heads whose column blocks alone nearly fill the 256 CUs are not cut: a
 // segmented walk does 1.5x the work (its state pass). (us per call, cut / uncut: d_state 64
@@ -1061,42 +1035,21 @@ void lay_out(const m3_layer_desc& d, Plan& p) {
 // heads: (1, 16384) 1,030 / 2,789, (2, 16384) 2,072 / 2,956, but (8, 2048) 1,068 / 656.)
 // The first cut is free, as the state at it is the walk's own: up to two segments a sequence
 // is walked in one piece with the same bits ((1, 600) of that layer 132 us, 199 cut).
-//
-// A workspace that does not hold every segment's state takes the batch in slices, and one
-// that does not hold those of one sequence takes its segments in groups, from two states on:
-// the same arithmetic in more launches. Below that (no workspace of
-// m3_prefill_workspace_size bytes or of m3_prefill_fwd_noalloc) the sequence is one walk.
+struct Plan : SegPlan {
+    int seg0;
+    int ncg;  // column groups per workgroup
+};
+
 Plan make_plan(const m3_layer_desc& d, size_t limit) {
     Plan p;
     p.ncg = column_groups(d.headdim, d.d_state, d.mimo_rank);
     const int64_t blocks = d.headdim / (PW * p.ncg);
     p.seg0 = std::max(256, d.headdim * d.d_state / 64);
-    p.segs = 1;
-    if (d.nheads * blocks < 192 && d.seqlen > 2 * p.seg0)
-        while (seg_start(p.segs, p.seg0) < d.seqlen) ++p.segs;
-    p.batch = d.batch;
-    p.slots = std::max(p.segs - 1, 1);
-    p.group = p.segs;
-    lay_out(d, p);
-    if (p.segs > 1 && p.total > limit) {
-        // the sequences of a slice, give or take alignment
-        p.batch = std::min(d.batch, 1 + (int)((double)limit / p.total * d.batch));
-        lay_out(d, p);
-        while (p.batch > 1 && p.total > limit) {
-            --p.batch;
-            lay_out(d, p);
-        }
-        while (p.slots > 2 && p.total > limit) {
-            --p.slots;
-            p.group = p.slots - 1;
-            lay_out(d, p);
-        }
-        if (p.total > limit) {
-            p.segs = p.slots = p.group = 1;
-            p.batch = d.batch;
-            lay_out(d, p);
-        }
-    }
+    const int segs = d.nheads * blocks < 192 ? seg_count(d.seqlen, p.seg0) : 1;
+    const SegSizes z = {(size_t)d.seqlen * d.ngroups * d.d_state * d.mimo_rank * sizeof(f16),
+                        (size_t)d.nheads * d.headdim * d.d_state * sizeof(float),
+                        d.nheads * sizeof(float), d.nheads * (d.d_state / 2) * sizeof(float)};
+    static_cast<SegPlan&>(p) = plan_segments(d.batch, segs, z, limit, true);
     // Narrower blocks where the workgroups would leave CUs idle: they repeat the rotation and
     // the scores, but each walks its chunks faster (same bits: a column's arithmetic does not
     // depend on its block).

@@ -1137,3 +1137,51 @@ def test_general_kernel_in_smaller_workspaces(kw, T, cuda_device):
     for B, nbytes in ((2, one), (1, one), (1, one - state), (1, one - 2 * state)):
         for a, b in zip(call(B, nbytes), whole):
             assert torch.equal(a, b[:B]), (B, nbytes)
+
+
+@pytest.mark.parametrize("extra,T", [
+    (dict(), 450),
+    (dict(use_complex_ssm=False), 390),
+    (dict(use_trapezoidal=False, ngroups=2), 700),
+    (dict(ngroups=24), 400),
+])
+def test_fp32_fused_segments_in_any_batch_and_workspace(extra, T, cuda_device):
+    """The fused fp32 kernel cuts a sequence by its layer and tokens alone: bit for bit, a row
+    alone is that row in a batch of 192 (batch, head) pairs, a prefix too short to be cut is
+    that of the cut run, a workspace of one sequence takes the batch in slices, one of a state
+    less takes the segments in groups, and the training forward gives the same outputs."""
+    print(f"fp32 fused batches {extra} T {T}", flush=True)
+    dev = cuda_device
+    torch.manual_seed(29)
+    layer = mamba3_amd.KulaMamba(768, d_state=128, headdim=64, mimo_rank=2, **extra).to(dev).eval()
+    H, P, N, B = layer.nheads, layer.headdim, layer.d_state, 8
+    with torch.no_grad():
+        proj = layer.in_proj(torch.randn(B, T, 768, device=dev))
+    ds = torch.rand(B, T, H, device=dev) + 0.5
+    state = H * P * N * 4
+
+    def call(rows, ntok, nbytes=None, train=False):
+        src, scale = proj[rows, :ntok].contiguous(), ds[rows, :ntok].contiguous()
+        n = src.shape[0]
+        desc = layer._desc(n, ntok, src)
+        if train:
+            desc.flags |= _native.M3_FLAG_FOR_BACKWARD
+        outs = (torch.empty(n, ntok, layer.d_inner, device=dev),
+                *(torch.empty(n, H, *s, device=dev) for s in ((P, N), (N // 2,), (P, N))))
+        name = _native.prefill_kernel_name(desc, src, outs[0], outs[1], outs[3])
+        assert name == ("fp32_fused_train" if train else "fp32_fused")
+        nbytes = _native.prefill_workspace_bytes(desc) if nbytes is None else nbytes
+        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+        _native.prefill_fwd(desc, layer._param_pack(), src, scale, *outs, ws, nbytes)
+        return outs
+
+    every, one = slice(0, B), slice(3, 4)
+    whole = call(every, T)
+    rows = 2 * T * layer.ngroups * N * layer.mimo_rank * 4  # of one sequence
+    segs = 4 + (T > 512)
+    seq = rows + (segs - 1) * (state + 256 + H * N * 2)
+    for got, sub in ((call(one, T), one), (call(one, T, seq - state), one),
+                     (call(every, T, max(seq, B * rows)), every), (call(every, T, train=True), every)):
+        for a, b in zip(got, whole):
+            assert torch.equal(a, b[sub])
+    assert torch.equal(call(every, 200)[0], whole[0][:, :200])
