@@ -45,6 +45,8 @@ enum m3_status {
 
 /* Size of the static per-device scratch of m3_prefill_fwd_noalloc (64 MiB). */
 #define M3_NOALLOC_SCRATCH_BYTES ((size_t)64 << 20)
+/* ... and beyond it, for the states of a sequence's segments. */
+#define M3_NOALLOC_STATE_BYTES ((size_t)64 << 20)
 
 /* Static description of one KulaMamba layer and of the activation tensor it reads.
  * Mirrors the constructor of KulaMamba (mamba3/mamba3.py:50-112). */
@@ -204,7 +206,10 @@ int m3_prefill_workspace_size(const m3_layer_desc* desc, size_t* bytes);
  *   h_final   [B,H,P,N] fp32 or NULL   (state 'h')
  *   angle     [B,H,N/2] fp32 or NULL   (state 'angle' = cumulative RoPE angle at T-1)
  *   prev_bx   [B,H,P,N] fp32 or NULL   (state 'prev_BX' = B~_{T-1} x_{T-1}^T)
- *   workspace of at least m3_prefill_workspace_size() bytes, 256-byte aligned.
+ *   workspace of at least m3_prefill_workspace_size() bytes, 256-byte aligned. (A smaller one
+ *   that still holds the call's operands is taken: the batch then runs in slices, or a
+ *   sequence's segments in groups; one that holds no two segments' states walks each sequence
+ *   in one piece, which moves its results by rounding.)
  */
 int m3_prefill_fwd(const m3_layer_desc* desc, const m3_layer_params* params,
                    const void* proj, const float* dt_scale, void* y_out,
@@ -214,14 +219,16 @@ int m3_prefill_fwd(const m3_layer_desc* desc, const m3_layer_params* params,
 /*
  * m3_prefill_fwd without a caller workspace: no counterpart in the reference. For callers
  * that cannot allocate device memory (code under HIP graph capture, tight serving loops,
- * harnesses that forbid hipMalloc). Same arguments, dispatch, kernels and results as
- * m3_prefill_fwd, but the workspace is a static array of the library on each GPU
- * (M3_NOALLOC_SCRATCH_BYTES, held from the first call on that GPU until the process
- * ends; bf16 layers outside the MFMA kernels take what it holds, see
- * m3_prefill_workspace_size; the general MFMA and the fused fp32 kernel walk each sequence in
- * one piece where the states of its segments do not fit, which moves results by rounding);
- * calls needing more return M3_ERR_SCRATCH_LIMIT and launch nothing. It calls no allocator. M3_FLAG_FOR_BACKWARD is refused (M3_ERR_UNSUPPORTED): the backward's operands
- * would be left in the shared scratch, which the next call overwrites. The scratch keeps the last call's contents and needs no clearing (every
+ * harnesses that forbid hipMalloc). Same arguments, dispatch, kernels and results, bit for bit,
+ * as m3_prefill_fwd in a workspace of m3_prefill_workspace_size bytes (bf16 layers outside the
+ * MFMA kernels take what the scratch holds, see there), but the workspace is a static array of
+ * the library on each GPU (M3_NOALLOC_SCRATCH_BYTES for the operands and M3_NOALLOC_STATE_BYTES
+ * for the states of the segments, held from the first call on that GPU until the process ends).
+ * Calls whose operands need more than M3_NOALLOC_SCRATCH_BYTES return M3_ERR_SCRATCH_LIMIT and
+ * launch nothing; calls whose segments' states do not fit run in slices of the batch, or in
+ * groups of segments. It calls no allocator. M3_FLAG_FOR_BACKWARD is refused
+ * (M3_ERR_UNSUPPORTED): the backward's operands would be left in the shared scratch, which the
+ * next call overwrites. The scratch keeps the last call's contents and needs no clearing (every
  * kernel writes what it later reads). All calls on one GPU share the array: calls that
  * overlap in time on one GPU (other streams or threads) race and must be serialised by
  * the caller.

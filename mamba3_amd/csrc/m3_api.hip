@@ -135,7 +135,11 @@ int launch_prefill_path(PrefillPath path, const m3_layer_desc& d, const m3_layer
 // that GPU until the process ends. Host code never uses the array's name as an address:
 // its device address is looked up once per device (hipGetSymbolAddress, with that device
 // current) and kept in g_scratch.
-static __device__ __align__(256) unsigned char scratch[M3_NOALLOC_SCRATCH_BYTES];
+// Behind the M3_NOALLOC_SCRATCH_BYTES that a call's operands may take lies room for the states of
+// its segments, so that every call that fits runs the same cuts as m3_prefill_fwd: two states
+// (plan_segments) of the widest layer that is cut, 191 x 128 columns of d_state 256, are 50 MB.
+constexpr size_t kScratchBytes = M3_NOALLOC_SCRATCH_BYTES + M3_NOALLOC_STATE_BYTES;
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -286,7 +290,7 @@ int m3_prefill_fwd_noalloc(const m3_layer_desc* desc, const m3_layer_params* par
     // The backward's operands would land in the shared scratch, which the next call
     // overwrites and no caller can hand to m3_layer_bwd.
     if (desc->flags & M3_FLAG_FOR_BACKWARD) return M3_ERR_UNSUPPORTED;
-    const size_t limit = M3_NOALLOC_SCRATCH_BYTES;
+    const size_t limit = kScratchBytes;
     const PrefillPath path = prefill_path(*desc, proj, y_out, h_final, prev_bx, limit);
     const size_t need = prefill_path_workspace(*desc, path, limit);
     if (need > M3_NOALLOC_SCRATCH_BYTES) return M3_ERR_SCRATCH_LIMIT;

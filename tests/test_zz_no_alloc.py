@@ -69,6 +69,27 @@ def test_noalloc_equals_prefill_fwd_on_two_calls(kw, dtype, path, cuda_device):
             assert torch.equal(a, b), (path, B, T, name)
 
 
+@pytest.mark.parametrize("kw,dtype,B,T", [
+    # more states of segments than a 64 MiB scratch holds beside the normalised B / C rows
+    (dict(d_model=2048, d_state=256, headdim=128, mimo_rank=4), torch.bfloat16, 1, 9000),
+    # and more than the library's whole scratch: slices of the batch
+    (dict(d_model=2048, d_state=256, headdim=128, mimo_rank=4), torch.bfloat16, 7, 2000),
+    (dict(d_model=768, d_state=128, headdim=64, mimo_rank=2), torch.float32, 15, 2000),
+])
+def test_noalloc_equals_prefill_fwd_with_many_segment_states(kw, dtype, B, T, cuda_device):
+    print(f"no-alloc prefill, segment states: {kw} {dtype} {B} x {T}", flush=True)
+    layer = _layer(kw, dtype, cuda_device)
+    with torch.no_grad():
+        proj = layer.in_proj(torch.randn(B, T, kw["d_model"], device=cuda_device, dtype=dtype)).contiguous()
+        assert _native.prefill_workspace_bytes(layer._desc(B, T, proj)) > _native.NOALLOC_SCRATCH_BYTES
+        got, want = (_outputs(layer, B, T, cuda_device, dtype) for _ in range(2))
+        _call(layer, proj, got, noalloc=True)
+        _call(layer, proj, want, noalloc=False)
+    torch.cuda.synchronize()
+    for name, a, b in zip(("y", "h", "angle", "prev_BX"), got, want):
+        assert torch.equal(a, b), (B, T, name)
+
+
 def test_noalloc_refuses_a_workspace_beyond_its_scratch(cuda_device):
     """The (8, 8192) d768 prefill needs 64 MiB of normalised B/C rows plus 256 bytes: one
     more than the scratch holds, so the call returns M3_ERR_SCRATCH_LIMIT and launches
