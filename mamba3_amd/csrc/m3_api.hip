@@ -293,7 +293,8 @@ int m3_prefill_fwd_noalloc(const m3_layer_desc* desc, const m3_layer_params* par
     const size_t limit = kScratchBytes;
     const PrefillPath path = prefill_path(*desc, proj, y_out, h_final, prev_bx, limit);
     const size_t need = prefill_path_workspace(*desc, path, limit);
-    if (need > M3_NOALLOC_SCRATCH_BYTES) return M3_ERR_SCRATCH_LIMIT;
+    // (the staged bf16 path was chosen because its slices fit)
+    if (path != PrefillPath::kStagedBf16 && need > M3_NOALLOC_SCRATCH_BYTES) return M3_ERR_SCRATCH_LIMIT;
     void* ws = nullptr;
     if (need > 0) {
         st = scratch_for_stream(as_stream(stream), &ws);

@@ -38,6 +38,10 @@ struct Args {
     float *dt, *A, *phi, *phi_sum, *xg, *xb, *xr, *Bt, *Bb, *Ct, *ys;  // workspace
     void* y;                                                           // outputs
     float *h_final, *angle, *prev_bx;
+    // A token slice of one sequence: the sums of dt theta and the last token's B~ before it and,
+    // for the next slice, after it (null at the sequence's start and end).
+    const float *sum_in, *b_in;
+    float *sum_out, *b_out;
 };
 
 template <typename T>
@@ -111,8 +115,9 @@ __global__ __launch_bounds__(NTH) void lp_angles(Args a) {
     if (e >= n) return;
     int b, c, h, i;
     angle_job(a, e, b, c, h, i);
-    float s = 0.f;
+    float s = a.sum_in ? a.sum_in[(int64_t)h * NH + i] : 0.f;
     for (int cc = 0; cc < c; ++cc) s += a.phi_sum[(((int64_t)b * nc + cc) * a.H + h) * NH + i];
+    if (a.sum_out && c == nc - 1) a.sum_out[(int64_t)h * NH + i] = s + a.phi_sum[e];
     const int t1 = min(a.T, (c + 1) * kAC);
     const float* dtp = a.dt + (int64_t)b * a.T * a.H + h;                  // stride H
     const T* thp = proj_of<T>(a) + (int64_t)b * a.T * a.rs + a.pl.theta + i;  // stride rs
@@ -209,7 +214,8 @@ __global__ __launch_bounds__(NTH) void lp_prep(Args a) {
                 a.Ct[tok * NR + e] = vc;
                 if (a.trap) {
                     if (t + 1 < a.T) a.Bb[(tok + a.H) * NR + e] = vb;  // B_b[t+1] = B~[t]
-                    if (t == 0) a.Bb[tok * NR + e] = 0.f;
+                    if (t == 0) a.Bb[tok * NR + e] = a.b_in ? a.b_in[(int64_t)h * NR + e] : 0.f;
+                    if (a.b_out && t + 1 == a.T) a.b_out[(int64_t)h * NR + e] = vb;
                 }
             }
         }
@@ -226,7 +232,7 @@ __global__ __launch_bounds__(NTH) void lp_prep(Args a) {
         a.xg[tok * PR + e] = xr * lam;
         if (a.trap) {
             const float sb = (1.f - lam) * expf(a.A[h] * a.dt[tok]);
-            const float xp = t > 0 ? ld_f32(row + a.pl.x + (int64_t)h * a.P + p - a.rs) * mx : 0.f;
+            const float xp = t > 0 || a.b_in ? ld_f32(row + a.pl.x + (int64_t)h * a.P + p - a.rs) * mx : 0.f;
             a.xb[tok * PR + e] = xp * sb;
         }
     }
@@ -376,8 +382,9 @@ size_t fp32_layer_workspace(const m3_layer_desc& d) {
 }
 
 // bf16 layers outside the bf16 MFMA kernels: the batch rows are independent, so they run in
-// slices whose staged operands stay within kStagedBf16Cap; a layer of which one row does not
-// fit runs on the generic kernel, and so do short sequences. That kernel walks the sequence on
+// slices whose staged operands stay within kStagedBf16Cap, and a row that does not fit in slices
+// of its tokens, which hand on the state, the angle sums and the last B~ (the slices end with
+// chunks: the same bits). Short sequences run on the generic kernel. That kernel walks the sequence on
 // the VALU, one workgroup per (batch, head, column block), at 30-50 us per LDS chunk of its own
 // (64 tokens of a small layer, 16 of d_state 128 rank 3); the ten launches here cost 50-60 us
 // before the tokens count (125 us at d_state 128 rank 3). us per call, generic / staged, bf16,
@@ -394,38 +401,69 @@ static int staged_bf16_min_chunks(const m3_layer_desc& d) {
     return d.d_state * d.headdim * d.mimo_rank >= 256 ? 2 : 8;
 }
 
-static int staged_bf16_rows(const m3_layer_desc& d, size_t cap) {
-    m3_layer_desc one = d;
-    one.batch = 1;
-    if (lp::plan(one).total > cap) return 0;
-    int rows = d.batch;
-    for (;;) {  // the plan grows with the rows, up to each part's alignment
-        one.batch = rows;
-        const size_t need = lp::plan(one).total;
-        if (need <= cap) return rows;
-        rows = std::max(1, std::min(rows - 1, (int)((double)rows * cap / need)));
+// A slice: batch rows, tokens of each (all, unless one row alone does not fit), bytes of its
+// staged operands, and behind them twice the floats that a token slice hands on.
+struct StagedSlices {
+    int rows, tokens;
+    size_t staged, h, sum, b, total;  // (rows 0: nothing fits)
+};
+
+static StagedSlices staged_bf16_slices(const m3_layer_desc& d, size_t cap) {
+    m3_layer_desc part = d;
+    const size_t H = d.nheads;
+    StagedSlices z = {d.batch, d.seqlen, 0, H * d.headdim * d.d_state, H * (d.d_state / 2),
+                      d.use_trapezoidal ? H * d.d_state * d.mimo_rank : 0, 0};
+    while (z.rows > 0) {  // the plan grows with the rows, up to each part's alignment
+        part.batch = z.rows;
+        z.staged = z.total = lp::plan(part).total;
+        if (z.total <= cap) return z;
+        z.rows = z.rows == 1 ? 0 : std::max(1, std::min(z.rows - 1, (int)((double)z.rows * cap / z.total)));
     }
+    const size_t carry = 2 * lp::al((z.h + z.sum + z.b) * sizeof(float));
+    part.batch = 1;
+    auto bytes = [&](int slices) {  // of a slice of so many angle chunks
+        part.seqlen = slices * lp::kAC;
+        return lp::plan(part).total + carry;
+    };
+    int lo = 0, hi = d.seqlen / lp::kAC;  // the longest that fits
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) / 2;
+        if (bytes(mid) <= cap) lo = mid;
+        else hi = mid - 1;
+    }
+    if (lo > 0) {
+        z.rows = 1;
+        z.tokens = lo * lp::kAC;
+        z.total = bytes(lo);
+        z.staged = z.total - carry;
+    }
+    return z;
 }
 
 size_t staged_bf16_workspace(const m3_layer_desc& d, size_t limit) {
     if (d.dtype != M3_DTYPE_BF16 || (d.flags & M3_FLAG_NO_F16_OPERANDS) || !staged_shape_ok(d)) return 0;
     if (d.seqlen <= (int64_t)staged_bf16_min_chunks(d) * generic_prefill_chunk(d)) return 0;
-    const int rows = staged_bf16_rows(d, std::min(limit, kStagedBf16Cap));
-    if (rows == 0) return 0;
-    m3_layer_desc part = d;
-    part.batch = rows;
-    return lp::plan(part).total;
+    const StagedSlices z = staged_bf16_slices(d, std::min(limit, kStagedBf16Cap));
+    return z.rows > 0 ? z.total : 0;
 }
+
+// What one token slice hands to the next.
+struct Carry {
+    const float *sum_in = nullptr, *b_in = nullptr, *h_in = nullptr;
+    float *sum_out = nullptr, *b_out = nullptr;
+};
 
 template <typename T>
 static int launch_staged(const m3_layer_desc& d, const m3_layer_params& p, const T* proj,
                          const float* dt_scale, T* y_out, float* h_final, float* angle,
-                         float* prev_bx, void* workspace, hipStream_t stream) {
+                         float* prev_bx, void* workspace, hipStream_t stream,
+                         const Carry& carry = Carry()) {
     using namespace lp;
     const Plan pl = plan(d);
     char* ws = reinterpret_cast<char*>(workspace);
     auto part = [&](int i) { return reinterpret_cast<float*>(ws + pl.off[i]); };
     Args a;
+    a.sum_in = carry.sum_in, a.sum_out = carry.sum_out, a.b_in = carry.b_in, a.b_out = carry.b_out;
     a.B = d.batch, a.T = d.seqlen, a.H = d.nheads, a.P = d.headdim, a.N = d.d_state;
     a.R = d.mimo_rank, a.G = d.ngroups, a.trap = d.use_trapezoidal, a.cplx = d.use_complex;
     a.rs = d.proj_row_stride, a.pl = proj_layout(d), a.eps = d.rms_eps, a.prm = p;
@@ -451,7 +489,7 @@ static int launch_staged(const m3_layer_desc& d, const m3_layer_params& p, const
     }
     hipLaunchKernelGGL(lp_prep<T>, dim3(d.batch * d.seqlen), dim3(NTH), lds, stream, a);
     if (launch_chunked_fwd_mfma(a.B, a.T, a.H, a.P, a.N, a.R, a.xg, a.xb, a.Bt, a.Bb, a.Ct, a.dt,
-                                a.A, p.D, a.xr, nullptr, a.ys, h_final, ws + pl.chunk_off,
+                                a.A, p.D, a.xr, carry.h_in, a.ys, h_final, ws + pl.chunk_off,
                                 stream) != 0)
         return 1;
     const int64_t n = (int64_t)d.batch * d.seqlen * d.nheads * d.headdim;
@@ -471,19 +509,32 @@ int launch_fp32_layer(const m3_layer_desc& d, const m3_layer_params& p, const vo
 int launch_staged_bf16(const m3_layer_desc& d, const m3_layer_params& p, const void* proj,
                        const float* dt_scale, void* y_out, float* h_final, float* angle,
                        float* prev_bx, void* workspace, size_t limit, hipStream_t stream) {
-    const int rows = staged_bf16_rows(d, std::min(limit, kStagedBf16Cap));
-    if (rows <= 0) return 1;
+    const StagedSlices z = staged_bf16_slices(d, std::min(limit, kStagedBf16Cap));
+    if (z.rows <= 0) return 1;
     const int64_t T = d.seqlen, H = d.nheads;
-    for (int b = 0; b < d.batch; b += rows) {
-        m3_layer_desc part = d;
-        part.batch = std::min(rows, d.batch - b);
-        auto at = [&](float* q, int64_t per_row) { return q ? q + b * per_row : nullptr; };
-        if (launch_staged(part, p, reinterpret_cast<const bf16*>(proj) + b * T * d.proj_row_stride,
-                          dt_scale ? dt_scale + b * T * H : nullptr,
-                          reinterpret_cast<bf16*>(y_out) + b * T * H * d.headdim,
-                          at(h_final, H * d.headdim * d.d_state), at(angle, H * (d.d_state / 2)),
-                          at(prev_bx, H * d.headdim * d.d_state), workspace, stream) != 0)
-            return 1;
+    const size_t set = lp::al((z.h + z.sum + z.b) * sizeof(float)) / sizeof(float);
+    float* hand = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + z.staged);
+    for (int b = 0; b < d.batch; b += z.rows) {
+        for (int64_t t = 0; t < T; t += z.tokens) {
+            m3_layer_desc part = d;
+            part.batch = std::min(z.rows, d.batch - b);
+            part.seqlen = (int)std::min<int64_t>(z.tokens, T - t);
+            const bool last = t + z.tokens >= T;
+            const int k = (int)(t / z.tokens);  // the slices alternate between two sets
+            const float* in = hand + (k + 1) % 2 * set;
+            float* out = hand + k % 2 * set;
+            Carry c;
+            if (t > 0) c.h_in = in, c.sum_in = in + z.h, c.b_in = d.use_trapezoidal ? in + z.h + z.sum : nullptr;
+            if (!last) c.sum_out = out + z.h, c.b_out = d.use_trapezoidal ? out + z.h + z.sum : nullptr;
+            auto at = [&](auto* q, int64_t per_row) { return q && last ? q + b * per_row : nullptr; };
+            float* h = last ? at(h_final, H * d.headdim * d.d_state) : out;
+            if (launch_staged(part, p, reinterpret_cast<const bf16*>(proj) + (b * T + t) * d.proj_row_stride,
+                              dt_scale ? dt_scale + (b * T + t) * H : nullptr,
+                              reinterpret_cast<bf16*>(y_out) + (b * T + t) * H * d.headdim, h,
+                              at(angle, H * (d.d_state / 2)), at(prev_bx, H * d.headdim * d.d_state), workspace,
+                              stream, c) != 0)
+                return 1;
+        }
     }
     return 0;
 }

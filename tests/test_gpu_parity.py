@@ -1185,3 +1185,37 @@ def test_fp32_fused_segments_in_any_batch_and_workspace(extra, T, cuda_device):
         for a, b in zip(got, whole):
             assert torch.equal(a, b[sub])
     assert torch.equal(call(every, 200)[0], whole[0][:, :200])
+
+
+@pytest.mark.parametrize("kw,T", [
+    (dict(d_model=64, d_state=16, headdim=16, mimo_rank=2), 1000),
+    (dict(d_model=64, d_state=18, headdim=32, mimo_rank=3, ngroups=2), 777),
+    (dict(d_model=48, d_state=70, headdim=24, mimo_rank=5, use_complex_ssm=False), 640),
+    (dict(d_model=64, d_state=18, headdim=32, mimo_rank=8, use_trapezoidal=False), 961),
+])
+def test_bf16_staged_prefill_in_token_slices(kw, T, cuda_device):
+    """bf16 layers outside the bf16 MFMA kernels in a workspace that does not hold one row: the
+    tokens run in slices, whose state, angles and last B~ carry over, bit for bit the whole."""
+    print(f"token slices {kw} T {T}", flush=True)
+    dev = cuda_device
+    torch.manual_seed(37)
+    layer = mamba3_amd.KulaMamba(**kw).to(dev, torch.bfloat16).eval()
+    H, P, N, B = layer.nheads, layer.headdim, layer.d_state, 2
+    with torch.no_grad():
+        proj = layer.in_proj(torch.randn(B, T, kw["d_model"], device=dev, dtype=torch.bfloat16))
+    ds = torch.rand(B, T, H, device=dev) + 0.5
+    desc = layer._desc(B, T, proj)
+    assert _native.prefill_kernel_name(desc, proj) == "fp32_layer"
+
+    def call(nbytes):
+        outs = (torch.empty(B, T, layer.d_inner, device=dev, dtype=torch.bfloat16),
+                *(torch.empty(B, H, *s, device=dev) for s in ((P, N), (N // 2,), (P, N))))
+        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+        _native.prefill_fwd(desc, layer._param_pack(), proj, ds, *outs, ws, nbytes)
+        return outs
+
+    whole = call(_native.prefill_workspace_bytes(desc))
+    row = _native.prefill_workspace_bytes(layer._desc(1, T, proj))
+    for nbytes in (row - 256, row // 2, row // 4):
+        for a, b in zip(call(nbytes), whole):
+            assert torch.equal(a, b), nbytes

@@ -75,9 +75,11 @@ def test_noalloc_equals_prefill_fwd_on_two_calls(kw, dtype, path, cuda_device):
     # and more than the library's whole scratch: slices of the batch
     (dict(d_model=2048, d_state=256, headdim=128, mimo_rank=4), torch.bfloat16, 7, 2000),
     (dict(d_model=768, d_state=128, headdim=64, mimo_rank=2), torch.float32, 15, 2000),
+    # staged operands of which the scratch holds a part: slices of the tokens
+    (dict(d_model=768, d_state=128, headdim=64, mimo_rank=3), torch.bfloat16, 1, 1500),
 ])
-def test_noalloc_equals_prefill_fwd_with_many_segment_states(kw, dtype, B, T, cuda_device):
-    print(f"no-alloc prefill, segment states: {kw} {dtype} {B} x {T}", flush=True)
+def test_noalloc_equals_prefill_fwd_in_slices(kw, dtype, B, T, cuda_device):
+    print(f"no-alloc prefill in slices: {kw} {dtype} {B} x {T}", flush=True)
     layer = _layer(kw, dtype, cuda_device)
     with torch.no_grad():
         proj = layer.in_proj(torch.randn(B, T, kw["d_model"], device=cuda_device, dtype=dtype)).contiguous()
