@@ -49,12 +49,15 @@ EXPORTED_SYMBOLS = (
 )
 
 M3_ERR_UNSUPPORTED = 3
+M3_ERR_WORKSPACE = 4
 M3_ERR_SCRATCH_LIMIT = 8
 NOALLOC_SCRATCH_BYTES = 64 << 20
 
 
 class NativeError(RuntimeError):
-    """A native entry point returned a non-zero m3_status."""
+    """A native entry point returned a non-zero m3_status (in `status`)."""
+
+    status = None
 
 
 class LayerDesc(ctypes.Structure):
@@ -181,7 +184,9 @@ def lib() -> ctypes.CDLL:
 def check(status: int, what: str) -> None:
     if status != 0:
         msg = lib().m3_status_string(status).decode()
-        raise NativeError(f"{what}: {msg} (m3_status {status})")
+        err = NativeError(f"{what}: {msg} (m3_status {status})")
+        err.status = status
+        raise err
 
 
 def dtype_code(dtype: torch.dtype) -> int:

@@ -74,6 +74,10 @@ def _state_shapes(B, nheads, headdim, d_state):
 
 
 # ---------------------------------------------------------------------------- prefill
+def _scratch(nbytes: int, device) -> torch.Tensor:
+    return torch.empty(max(nbytes, 1), device=device, dtype=torch.uint8)
+
+
 def _prefill_eager(proj, A_log, D, dt_bias, B_norm_w, C_norm_w, B_bias, C_bias, mimo_x, mimo_z,
                    mimo_down, dt_scale, nheads, headdim, d_state, mimo_rank, ngroups, trap, cplx,
                    eps, return_state):
@@ -96,8 +100,27 @@ def _prefill_eager(proj, A_log, D, dt_bias, B_norm_w, C_norm_w, B_bias, C_bias, 
     else:
         h = angle = prev = None
     ws_bytes = _native.prefill_workspace_bytes(desc)
-    ws = torch.empty(max(ws_bytes, 1), device=dev, dtype=torch.uint8)
-    _native.prefill_fwd(desc, pack, proj, dt_scale, y, h, angle, prev, ws, ws_bytes)
+    try:
+        ws = _scratch(ws_bytes, dev)
+    except torch.OutOfMemoryError as e:
+        oom = e
+    else:
+        _native.prefill_fwd(desc, pack, proj, dt_scale, y, h, angle, prev, ws, ws_bytes)
+        return y, h, angle, prev
+    # The kernels take a smaller workspace too (slices of the batch or the sequence).
+    ws = None
+    while ws is None and ws_bytes:
+        ws_bytes = ws_bytes * 7 // 8
+        try:
+            ws = _scratch(ws_bytes, dev) if ws_bytes else None
+        except torch.OutOfMemoryError:
+            pass
+    try:
+        _native.prefill_fwd(desc, pack, proj, dt_scale, y, h, angle, prev, ws, ws_bytes)
+    except _native.NativeError as e:
+        if e.status == _native.M3_ERR_WORKSPACE:  # not even the operands fit
+            raise oom from None
+        raise
     return y, h, angle, prev
 
 

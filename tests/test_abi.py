@@ -423,3 +423,41 @@ def test_prefill_kernel_name_and_noalloc_refusal(lib):
     d = desc(dtype=0, flags=_native.M3_FLAG_FOR_BACKWARD)
     assert lib.m3_prefill_fwd_noalloc(ctypes.byref(d), ctypes.byref(params), fake, None, fake,
                                       None, None, None, None) == 3
+
+
+def test_prefill_short_of_memory_takes_a_smaller_workspace(monkeypatch):
+    """Where the advertised workspace cannot be allocated the prefill runs in the largest of the
+    ones tried below it that can, and raises the allocator's error when that holds no call
+    (host only: the allocator and the library's entry are stand-ins)."""
+    import torch
+    import mamba3_amd
+    from mamba3_amd import _native, ops
+    layer = mamba3_amd.KulaMamba(d_model=64, d_state=16, headdim=16, mimo_rank=3).bfloat16()
+    proj = torch.zeros(2, 300, layer.in_proj.out_features, dtype=torch.bfloat16)
+    full = _native.prefill_workspace_bytes(layer._desc(2, 300, proj))
+    calls = []
+
+    def scratch(n, dev):
+        if n > free:
+            raise torch.OutOfMemoryError(f"no {n} bytes")
+        return n
+
+    def prefill_fwd(desc, pack, proj, scale, y, h, angle, prev, ws, nbytes):
+        assert ws == nbytes or (ws is None and nbytes == 0)
+        calls.append(nbytes)
+        if nbytes < need:
+            _native.check(_native.M3_ERR_WORKSPACE, "m3_prefill_fwd")
+
+    monkeypatch.setattr(_native, "require_gpu", lambda *t: None)
+    monkeypatch.setattr(_native, "prefill_fwd", prefill_fwd)
+    monkeypatch.setattr(ops, "_scratch", scratch)
+    args = (proj, *layer._small_params(), None, *ops.layer_args(layer), True)
+    for free, need, expect in ((full, full, full), (full - 1, 1, None), (full // 3, 1, None),
+                               (0, 0, 0)):
+        calls.clear()
+        ops._prefill_eager(*args)
+        assert len(calls) == 1 and calls[0] <= free
+        assert calls[0] == expect if expect is not None else calls[0] > free * 7 // 8 - 1
+    free, need = full // 3, full // 2
+    with pytest.raises(torch.OutOfMemoryError):
+        ops._prefill_eager(*args)
