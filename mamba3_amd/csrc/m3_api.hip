@@ -87,6 +87,21 @@ size_t prefill_path_workspace(const m3_layer_desc& d, PrefillPath path, size_t l
     }
 }
 
+// Workspace for whichever prefill kernel the shape may dispatch to (the pointers' alignment
+// is not known here, so the largest of the candidates).
+size_t prefill_workspace(const m3_layer_desc& d) {
+    size_t n = m3::generic_prefill_workspace(d);
+    n = std::max(n, m3::fp32_layer_workspace(d));
+    if (m3::fused_fp32_prefill_supported(d, nullptr, nullptr, nullptr, nullptr))
+        n = std::max(n, m3::fused_fp32_prefill_workspace(d));
+    if ((d.flags & M3_FLAG_FOR_BACKWARD) && m3::fused_fp32_train_supported(d, nullptr, nullptr, nullptr, nullptr))
+        n = std::max(n, m3::fused_fp32_train_workspace(d));
+    if (m3::mfma_prefill_supported(d, nullptr, nullptr)) n = std::max(n, m3::mfma_prefill_workspace(d));
+    if (m3::wide_prefill_supported(d)) n = std::max(n, m3::wide_prefill_workspace(d));
+    else n = std::max(n, m3::staged_bf16_workspace(d, SIZE_MAX));
+    return n;
+}
+
 int check_prefill_args(const m3_layer_desc* desc, const m3_layer_params* params,
                        const void* proj, const void* y_out) {
     int st = check_desc(desc);
@@ -194,7 +209,7 @@ int m3_version(void) { return 200; }
 const char* m3_prefill_kernel_name(const m3_layer_desc* desc, const void* proj, const void* y_out,
                                    const float* h_final, const float* prev_bx) {
     if (check_desc(desc) != M3_OK) return nullptr;
-    switch (prefill_path(*desc, proj, y_out, h_final, prev_bx, SIZE_MAX)) {
+    switch (prefill_path(*desc, proj, y_out, h_final, prev_bx, prefill_workspace(*desc))) {
         case PrefillPath::kMfma: return "mfma_d128_p64_r2";
         case PrefillPath::kWide: return "mfma_general";
         case PrefillPath::kFp32Fused: return "fp32_fused";
@@ -241,21 +256,6 @@ int m3_scan_bwd(const float* decay, const float* h_states, const float* grad, fl
                                as_stream(stream)) == 0
                ? M3_OK
                : M3_ERR_LAUNCH;
-}
-
-// Workspace for whichever prefill kernel the shape may dispatch to (the pointers' alignment
-// is not known here, so the largest of the candidates).
-static size_t prefill_workspace(const m3_layer_desc& d) {
-    size_t n = m3::generic_prefill_workspace(d);
-    n = std::max(n, m3::fp32_layer_workspace(d));
-    if (m3::fused_fp32_prefill_supported(d, nullptr, nullptr, nullptr, nullptr))
-        n = std::max(n, m3::fused_fp32_prefill_workspace(d));
-    if ((d.flags & M3_FLAG_FOR_BACKWARD) && m3::fused_fp32_train_supported(d, nullptr, nullptr, nullptr, nullptr))
-        n = std::max(n, m3::fused_fp32_train_workspace(d));
-    if (m3::mfma_prefill_supported(d, nullptr, nullptr)) n = std::max(n, m3::mfma_prefill_workspace(d));
-    if (m3::wide_prefill_supported(d)) n = std::max(n, m3::wide_prefill_workspace(d));
-    else n = std::max(n, m3::staged_bf16_workspace(d, SIZE_MAX));
-    return n;
 }
 
 int m3_prefill_workspace_size(const m3_layer_desc* desc, size_t* bytes) {

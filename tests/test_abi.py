@@ -461,3 +461,21 @@ def test_prefill_short_of_memory_takes_a_smaller_workspace(monkeypatch):
     free, need = full // 3, full // 2
     with pytest.raises(torch.OutOfMemoryError):
         ops._prefill_eager(*args)
+
+
+def test_kernel_name_of_a_misaligned_state_follows_the_advertised_workspace():
+    """A general-MFMA shape whose h_final is not 16-byte aligned leaves that kernel. The name is
+    that of the kernel which m3_prefill_fwd runs in the advertised workspace, sized for the
+    general kernel: slices of the staged operands where it holds one of 64 tokens, else the
+    generic kernel."""
+    one_slice = _native.LayerDesc(8, 4096, 2, 64, 64, 1, 1, 1, 1, _native.M3_DTYPE_BF16, 600, 1e-5, 0)
+    none = _native.LayerDesc(1, 200, 48, 128, 256, 4, 1, 1, 1, _native.M3_DTYPE_BF16, 16384, 1e-5, 0)
+    lib = _native.lib()
+
+    def name(desc, h):
+        return lib.m3_prefill_kernel_name(ctypes.byref(desc), 4096, 4096, h, 4096)
+
+    for desc in (one_slice, none):
+        assert name(desc, 4096) == b"mfma_general"
+    assert name(one_slice, 4100) == b"fp32_layer"
+    assert name(none, 4100) == b"generic"
