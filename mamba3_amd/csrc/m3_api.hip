@@ -405,8 +405,8 @@ static bool norm_dtypes_ok(int xd, int wd, int yd) {
     return yd == ((xd == M3_DTYPE_BF16 && wd == M3_DTYPE_BF16) ? M3_DTYPE_BF16 : M3_DTYPE_F32);
 }
 
-// Grid limits of the norm kernels: rows / 4 blocks (x) forward, d / 256 column blocks (y)
-// for the dweight partials.
+// 2^33 rows are what 32-bit block counts hold at four rows a block; from 2^26 rows on the runtime
+// rejects the forward's grid (64 threads a row).
 static bool norm_shape_ok(int64_t rows, int32_t d) {
     return rows > 0 && rows < ((int64_t)1 << 33) && d > 0 && d <= (1 << 24);
 }

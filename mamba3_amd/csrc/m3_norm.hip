@@ -290,20 +290,34 @@ static void launch_bwd_t(const void* x, const void* w, const float* rstd, const 
     const int64_t nparts = (rows + kNormRowsPerPart - 1) / kNormRowsPerPart;
     const int64_t cb = (d + 63) / 64;
     constexpr int W = kNormBwdThreads / 64;
-    // at most 65536 dw blocks, so that the grid stays within 2^32 threads for every row count
-    // that dx alone allows
     const unsigned ndw = (unsigned)std::min<int64_t>(nparts * cb, 65536);
-    const dim3 grid((unsigned)(ndw + (rows + W - 1) / W));
     // four-element pieces need whole, aligned pieces in every row
     auto al = [](const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; };
     const bool vec = d % 4 == 0 && al(x, 4 * sizeof(TX)) && al(dx, 4 * sizeof(TX)) &&
                      al(w, 4 * sizeof(TW)) && al(g, 4 * sizeof(TG));
-    if (vec)
-        hipLaunchKernelGGL((rmsnorm_bwd_kernel<TX, TW, TG, true>), grid, dim3(kNormBwdThreads), 0,
+    // dx of rows r0 .. r1 - 1 behind ndw blocks of dw
+    auto run = [&](int64_t r0, int64_t r1, unsigned ndw) {
+        const dim3 grid((unsigned)(ndw + (r1 - r0 + W - 1) / W));
+        const TX* xr = reinterpret_cast<const TX*>(x) + r0 * d;
+        const TG* gr = reinterpret_cast<const TG*>(g) + r0 * d;
+        TX* dr = reinterpret_cast<TX*>(dx) + r0 * d;
+        if (vec)
+            hipLaunchKernelGGL((rmsnorm_bwd_kernel<TX, TW, TG, true>), grid, dim3(kNormBwdThreads), 0,
+                               stream, xr, w, rstd + r0, gr, dr, part, r1 - r0, d, (int)nparts, ndw);
+        else
+            hipLaunchKernelGGL((rmsnorm_bwd_kernel<TX, TW, TG, false>), grid, dim3(kNormBwdThreads), 0,
+                               stream, xr, w, rstd + r0, gr, dr, part, r1 - r0, d, (int)nparts, ndw);
+    };
+    // A grid holds less than 2^32 threads: from 2^26 - 2^20 rows on dw is a launch of its own, and
+    // dx launches of at most 2^25 rows (a multiple of four, so that pieces stay aligned).
+    if (ndw + (rows + W - 1) / W < ((int64_t)1 << 32) / kNormBwdThreads) {
+        run(0, rows, ndw);
+    } else {
+        hipLaunchKernelGGL((rmsnorm_bwd_kernel<TX, TW, TG, false>), dim3(ndw), dim3(kNormBwdThreads), 0,
                            stream, x, w, rstd, g, dx, part, rows, d, (int)nparts, ndw);
-    else
-        hipLaunchKernelGGL((rmsnorm_bwd_kernel<TX, TW, TG, false>), grid, dim3(kNormBwdThreads), 0,
-                           stream, x, w, rstd, g, dx, part, rows, d, (int)nparts, ndw);
+        constexpr int64_t kRows = (int64_t)1 << 25;
+        for (int64_t r = 0; r < rows; r += kRows) run(r, std::min(rows, r + kRows), 0);
+    }
     hipLaunchKernelGGL((rmsnorm_dw_sum_kernel<TW>), dim3((unsigned)cb), dim3(kNormThreads), 0, stream,
                        part, dw, (int)nparts, d);
 }

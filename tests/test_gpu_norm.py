@@ -189,3 +189,23 @@ def test_block_prefill_then_steps_match_oracle(cuda_device):
             y_ref, st_ref = ref.block_step(cfg, p, "", toks[i].double(), st_ref, 0.5, True)
             assert max_rel(y, y_ref) < FP32_TOL, i
             assert max_rel(st["h"], st_ref["h"]) < FP32_TOL, i
+
+
+def test_rmsnorm_backward_of_almost_2_to_26_rows(cuda_device):
+    """The last row count that one wave per row allows in a grid of less than 2^32 threads: the
+    launch with dw's blocks beside dx's no longer fits and is split. dx element by element, dw
+    of non-negative terms: fp32 sums of 65,536 serial additions per wave, 2^-24 each."""
+    rows = (1 << 26) - 4
+    print(f"rmsnorm backward, {rows} rows", flush=True)
+    g = torch.Generator(device=cuda_device).manual_seed(3)
+    x = torch.rand(rows, 1, device=cuda_device, generator=g) + 0.5
+    grad = torch.rand(rows, 1, device=cuda_device, generator=g)
+    w = torch.full((1,), 1.25, device=cuda_device)
+    rstd = torch.rsqrt(x[:, 0] * x[:, 0] + 1e-5)
+    dx, dw = ops.rmsnorm_bwd(x, w, rstd, grad)
+    # d = 1: dx = s w g - x s^3 w g x = s w g (1 - x^2 s^2), a difference of terms of s w g
+    s = rstd[:, None]
+    want = s * w * grad * (1e-5 * s * s)
+    assert float((dx - want).abs().max()) < 8 * 2.0 ** -24 * float((s * w * grad).max())
+    exact = float((grad * x * s).sum(dtype=torch.float64))
+    assert abs(float(dw) - exact) < 65536 * 2.0 ** -24 * exact
