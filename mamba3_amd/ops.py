@@ -706,44 +706,57 @@ def _(gate_up, d_ff):
 
 
 # ---------------------------------------------------------------- eager calls
-_PLAIN = (torch.Tensor, torch.nn.Parameter)
+# What a direct call may be given: a subclass's own dispatch has to see it.
+_PLAIN = frozenset((torch.Tensor, torch.nn.Parameter, type(None)))
 
 
-def _direct(a: torch.Tensor, b: torch.Tensor) -> bool:
+def _direct(tensors) -> bool:
     """Eager calls with autograd off bypass the dispatcher: its per-call host time (16 us for
     the prefill op) is what a per-token decode loop and a short prompt wait on. Traced calls,
     calls under autograd, a dispatch or function mode, a functorch transform or forward-mode
-    AD, and calls on tensor subclasses go through the registered ops and their formulas. `a`
-    and `b` stand for the activations and the parameters."""
-    return not (torch.is_grad_enabled() or torch.compiler.is_compiling()
-                or _C._len_torch_dispatch_stack() or _C._len_torch_function_stack()
-                or _C._get_tracing_state() is not None
-                or _C._functorch.peek_interpreter_stack() is not None
-                or _forward_ad._current_level >= 0
-                or type(a) not in _PLAIN or type(b) not in _PLAIN)
+    AD, and calls with a tensor subclass among `tensors` (all tensor arguments of the op) go
+    through the registered ops and their formulas."""
+    if _is_grad_enabled() or _is_compiling():
+        return False
+    if (_in_dispatch_mode() or _in_function_mode() or _tracing_state() is not None
+            or _functorch_stack() is not None or _forward_ad._current_level >= 0):
+        return False
+    return _PLAIN.issuperset(map(type, tensors))
+
+
+_is_grad_enabled, _is_compiling = torch.is_grad_enabled, torch.compiler.is_compiling
+# torch's private counters of the modes and transforms that a direct call would pass by; on a
+# torch version that lacks one of them every call goes through the ops.
+try:
+    _in_dispatch_mode, _in_function_mode = _C._len_torch_dispatch_stack, _C._len_torch_function_stack
+    _tracing_state, _functorch_stack = _C._get_tracing_state, _C._functorch.peek_interpreter_stack
+    _forward_ad._current_level
+except AttributeError:
+    def _direct(tensors) -> bool:
+        return False
 
 
 def prefill_fast(*args):
-    return (_prefill_eager if _direct(args[0], args[1]) else prefill)(*args)
+    return (_prefill_eager if _direct(args[:12]) else prefill)(*args)
 
 
 def step_fast(*args):
-    return (_step_eager if _direct(args[0], args[1]) else step)(*args)
+    return (_step_eager if _direct(args[:15]) else step)(*args)
 
 
 def small_linear_fast(x, norm_w, eps, weight, residual, scale):
-    fn = _small_linear_eager if _direct(x, weight) else small_linear
+    fn = _small_linear_eager if _direct((x, norm_w, weight, residual)) else small_linear
     return fn(x, norm_w, eps, weight, residual, scale)
 
 
 def small_swiglu_fast(x, norm_w, eps, w_gate, w_up):
-    fn = _small_swiglu_eager if _direct(x, w_gate) else small_swiglu
+    fn = _small_swiglu_eager if _direct((x, norm_w, w_gate, w_up)) else small_swiglu
     return fn(x, norm_w, eps, w_gate, w_up)
 
 
 def silu_mul_fast(gate_up, d_ff):
-    return (_silu_mul_eager if _direct(gate_up, gate_up) else silu_mul)(gate_up, d_ff)
+    return (_silu_mul_eager if _direct((gate_up,)) else silu_mul)(gate_up, d_ff)
 
 
 def rmsnorm_fast(x, weight, eps):
-    return (_rmsnorm_eager if _direct(x, weight) else rmsnorm)(x, weight, eps)[0]
+    return (_rmsnorm_eager if _direct((x, weight)) else rmsnorm)(x, weight, eps)[0]

@@ -282,16 +282,16 @@ def test_module_calls_under_a_dispatch_mode_go_through_the_ops():
         out, st = layer.step(x[:, 0], st)
         assert out.shape == (2, 64) and st["angle"].shape == (2, layer.nheads, 8)
     t = torch.ones(3)
-    assert not ops._direct(t, t)
+    assert not ops._direct((t, t))
     with torch.no_grad():
-        assert ops._direct(t, torch.nn.Parameter(t))
-        assert not ops._direct(t.as_subclass(type("Sub", (torch.Tensor,), {})), t)
+        assert ops._direct((t, torch.nn.Parameter(t)))
+        assert not ops._direct((t.as_subclass(type("Sub", (torch.Tensor,), {})), t))
         seen = []
-        torch.func.vmap(lambda v: seen.append(ops._direct(t, t)) or v)(t)
+        torch.func.vmap(lambda v: seen.append(ops._direct((t, t))) or v)(t)
         with torch.autograd.forward_ad.dual_level():
-            seen.append(ops._direct(t, t))
+            seen.append(ops._direct((t, t)))
         with torch.device("cpu"):
-            seen.append(ops._direct(t, t))
+            seen.append(ops._direct((t, t)))
         assert seen == [False] * 3
 
 
@@ -479,3 +479,54 @@ def test_kernel_name_of_a_misaligned_state_follows_the_advertised_workspace():
         assert name(desc, 4096) == b"mfma_general"
     assert name(one_slice, 4100) == b"fp32_layer"
     assert name(none, 4100) == b"generic"
+
+
+def test_a_subclass_in_any_tensor_argument_goes_through_the_op(monkeypatch):
+    """The direct eager calls look at every tensor argument of the op they stand for: a subclass
+    among the parameters, dt_scale, the decode state, a norm weight or the residual takes the
+    registered op, and so does every call under a mode."""
+    import torch
+    from mamba3_amd import ops
+
+    class Sub(torch.Tensor):
+        pass
+
+    seen = []
+    calls = {  # direct entry, op, eager body, tensor arguments, the rest
+        "prefill_fast": ("prefill", "_prefill_eager", 12, (0,) * 9),
+        "step_fast": ("step", "_step_eager", 15, (0,) * 8),
+        "rmsnorm_fast": ("rmsnorm", "_rmsnorm_eager", 2, (1e-5,)),
+    }
+    for op, eager, *_ in calls.values():
+        monkeypatch.setattr(ops, op, lambda *a: seen.append("op") or (None,))
+        monkeypatch.setattr(ops, eager, lambda *a: seen.append("direct") or (None,))
+    for name in ("small_linear", "small_swiglu"):
+        monkeypatch.setattr(ops, name, lambda *a: seen.append("op"))
+        monkeypatch.setattr(ops, f"_{name}_eager", lambda *a: seen.append("direct"))
+
+    def routes(call, n):
+        plain = [torch.zeros(2) for _ in range(n)]
+        out = []
+        for i in (None, *range(n)):
+            ts = list(plain)
+            if i is not None:
+                ts[i] = ts[i].as_subclass(Sub)
+            seen.clear()
+            call(*ts)
+            out += seen
+        return out
+
+    def all_routes():
+        with torch.no_grad():
+            for fast, (_, _, n, rest) in calls.items():
+                yield n, routes(lambda *ts: getattr(ops, fast)(*ts, *rest), n)
+            yield 4, routes(lambda x, n, w, r: ops.small_linear_fast(x, n, 1e-5, w, r, 1.0), 4)
+            yield 4, routes(lambda x, n, g, u: ops.small_swiglu_fast(x, n, 1e-5, g, u), 4)
+
+    for n, got in all_routes():
+        assert got == ["direct"] + ["op"] * n
+    for counter in ("_in_dispatch_mode", "_in_function_mode"):
+        with monkeypatch.context() as m:
+            m.setattr(ops, counter, lambda: 1)
+            for n, got in all_routes():
+                assert got == ["op"] * (n + 1)
