@@ -111,7 +111,7 @@ __device__ __forceinline__ int64_t row(const Shape& s, int b, int tg, int h) {
 template <int TN>
 struct Lds {
     float A[KT][TT + 17];
-    float B[KT][TN + 17];
+    float B[KT][TN == 16 ? TN + 1 : TN + 17];
 };
 
 // Tile layout of the fp32 MFMA accumulators (v_mfma_f32_16x16x4_f32: lane l holds rows
