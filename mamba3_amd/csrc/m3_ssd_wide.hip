@@ -87,11 +87,9 @@ struct Tok {
 
 // Column groups per workgroup: headdim in blocks of 128, 64 or 32 columns (128 columns of
 // d_state 256 at rank 1, whose helper threads each prepare 16 tokens, would spill).
-template <int N, int R>
-constexpr int kMaxGroups = N == 256 && R == 1 ? 2 : 4;
+constexpr int max_groups(int N, int R) { return N == 256 && R == 1 ? 2 : 4; }
 inline int column_groups(int P, int N, int R) {
-    const int most = N == 256 && R == 1 ? 2 : 4;
-    return std::min(most, P % 128 == 0 ? 4 : P % 64 == 0 ? 2 : 1);
+    return std::min(max_groups(N, R), P % 128 == 0 ? 4 : P % 64 == 0 ? 2 : 1);
 }
 
 // Helper thread layout: N/4 lanes (one 4-column group, two RoPE pairs, each) share a token
@@ -144,9 +142,6 @@ struct Args {
     float* lseg;  // log2 of the segment's decay, [seg][b h]
     float* aseg;  // its RoPE angle increment, [seg][b h][pair]
 };
-
-// Keeps the LDS reads issued above ahead of the LDS writes that follow.
-#define M3_LDS_ORDER() asm volatile("" ::: "memory")
 
 // v, rounded to fp32: keeps the product behind v out of a fused conversion.
 __device__ __forceinline__ float opaque_f(float v) {
@@ -1096,7 +1091,7 @@ int launch_slice(const m3_layer_desc& d, const Plan& plan, const m3_layer_params
     hipLaunchKernelGGL((bc_norm_wide<N, R>), dim3((unsigned)((nrows + rows_per_block - 1) / rows_per_block)),
                        dim3(256), 0, stream, a.proj, a.rs, a.pl.B, a.pl.C, a.G, nrows, d.rms_eps, vec,
                        p.B_norm_w, p.B_bias, p.C_norm_w, p.C_bias, bn, cn);
-    if constexpr (kMaxGroups<N, R> == 4) {
+    if constexpr (max_groups(N, R) == 4) {
         if (ncg == 4) {
             launch_ssd<N, R, 4>(a, plan.group, stream);
             return hipGetLastError() == hipSuccess ? M3_OK : M3_ERR_LAUNCH;
