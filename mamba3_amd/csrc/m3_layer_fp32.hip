@@ -38,10 +38,14 @@ struct Args {
     float *dt, *A, *phi, *phi_sum, *xg, *xb, *xr, *Bt, *Bb, *Ct, *ys;  // workspace
     void* y;                                                           // outputs
     float *h_final, *angle, *prev_bx;
-    // A token slice of one sequence: the sums of dt theta and the last token's B~ before it and,
-    // for the next slice, after it (null at the sequence's start and end).
-    const float *sum_in, *b_in;
-    float *sum_out, *b_out;
+};
+
+// A token slice of one sequence: the state, the sums of dt theta and the last token's B~ before it
+// and, for the next slice, after it (null at the sequence's start and end; the state after it is
+// its h_final).
+struct Carry {
+    const float *h_in = nullptr, *sum_in = nullptr, *b_in = nullptr;
+    float *sum_out = nullptr, *b_out = nullptr;
 };
 
 template <typename T>
@@ -106,8 +110,8 @@ __global__ __launch_bounds__(NTH) void lp_angle_sums(Args a) {
     a.phi_sum[e] = s;
 }
 
-template <typename T>
-__global__ __launch_bounds__(NTH) void lp_angles(Args a) {
+template <typename T, bool CARRY>
+__global__ __launch_bounds__(NTH) void lp_angles(Args a, const float* __restrict__ sum_in) {
     const int nc = (a.T + kAC - 1) / kAC;
     const int NH = a.N / 2;
     const int64_t n = (int64_t)a.B * nc * a.H * NH;
@@ -115,9 +119,8 @@ __global__ __launch_bounds__(NTH) void lp_angles(Args a) {
     if (e >= n) return;
     int b, c, h, i;
     angle_job(a, e, b, c, h, i);
-    float s = a.sum_in ? a.sum_in[(int64_t)h * NH + i] : 0.f;
+    float s = CARRY ? sum_in[(int64_t)h * NH + i] : 0.f;
     for (int cc = 0; cc < c; ++cc) s += a.phi_sum[(((int64_t)b * nc + cc) * a.H + h) * NH + i];
-    if (a.sum_out && c == nc - 1) a.sum_out[(int64_t)h * NH + i] = s + a.phi_sum[e];
     const int t1 = min(a.T, (c + 1) * kAC);
     const float* dtp = a.dt + (int64_t)b * a.T * a.H + h;                  // stride H
     const T* thp = proj_of<T>(a) + (int64_t)b * a.T * a.rs + a.pl.theta + i;  // stride rs
@@ -214,8 +217,7 @@ __global__ __launch_bounds__(NTH) void lp_prep(Args a) {
                 a.Ct[tok * NR + e] = vc;
                 if (a.trap) {
                     if (t + 1 < a.T) a.Bb[(tok + a.H) * NR + e] = vb;  // B_b[t+1] = B~[t]
-                    if (t == 0) a.Bb[tok * NR + e] = a.b_in ? a.b_in[(int64_t)h * NR + e] : 0.f;
-                    if (a.b_out && t + 1 == a.T) a.b_out[(int64_t)h * NR + e] = vb;
+                    if (t == 0) a.Bb[tok * NR + e] = 0.f;
                 }
             }
         }
@@ -232,9 +234,33 @@ __global__ __launch_bounds__(NTH) void lp_prep(Args a) {
         a.xg[tok * PR + e] = xr * lam;
         if (a.trap) {
             const float sb = (1.f - lam) * expf(a.A[h] * a.dt[tok]);
-            const float xp = t > 0 || a.b_in ? ld_f32(row + a.pl.x + (int64_t)h * a.P + p - a.rs) * mx : 0.f;
+            const float xp = t > 0 ? ld_f32(row + a.pl.x + (int64_t)h * a.P + p - a.rs) * mx : 0.f;
             a.xb[tok * PR + e] = xp * sb;
         }
+    }
+}
+
+// What a token slice of one sequence takes from the one before it, into the first token's beta
+// operands, and hands on (one thread per element; after lp_prep).
+template <typename T>
+__global__ __launch_bounds__(NTH) void lp_hand(Args a, Carry k) {
+    const int NH = a.N / 2, NR = a.N * a.R, PR = a.P * a.R;
+    const int j = blockIdx.x * NTH + threadIdx.x;
+    if (a.cplx && k.sum_out && j < a.H * NH) {
+        const int nc = (a.T + kAC - 1) / kAC;
+        float s = k.sum_in ? k.sum_in[j] : 0.f;
+        for (int c = 0; c < nc; ++c) s += a.phi_sum[(int64_t)c * a.H * NH + j];
+        k.sum_out[j] = s;
+    }
+    if (k.b_out && j < a.H * NR) k.b_out[j] = a.Bt[(int64_t)(a.T - 1) * a.H * NR + j];
+    if (k.b_in && j < a.H * NR) a.Bb[j] = k.b_in[j];
+    if (k.b_in && j < a.H * PR) {
+        const int h = j / PR, p = j % PR / a.R;
+        const T* row = proj_of<T>(a);
+        const float lam = 1.f / (1.f + expf(-ld_f32(row + a.pl.lam + h)));
+        const float sb = (1.f - lam) * expf(a.A[h] * a.dt[h]);
+        const float xp = ld_f32(row + a.pl.x + (int64_t)h * a.P + p - a.rs) * a.prm.mimo_x[j];
+        a.xb[j] = xp * sb;
     }
 }
 
@@ -447,23 +473,16 @@ size_t staged_bf16_workspace(const m3_layer_desc& d, size_t limit) {
     return z.rows > 0 ? z.total : 0;
 }
 
-// What one token slice hands to the next.
-struct Carry {
-    const float *sum_in = nullptr, *b_in = nullptr, *h_in = nullptr;
-    float *sum_out = nullptr, *b_out = nullptr;
-};
-
 template <typename T>
 static int launch_staged(const m3_layer_desc& d, const m3_layer_params& p, const T* proj,
                          const float* dt_scale, T* y_out, float* h_final, float* angle,
                          float* prev_bx, void* workspace, hipStream_t stream,
-                         const Carry& carry = Carry()) {
+                         const lp::Carry& carry = lp::Carry()) {
     using namespace lp;
     const Plan pl = plan(d);
     char* ws = reinterpret_cast<char*>(workspace);
     auto part = [&](int i) { return reinterpret_cast<float*>(ws + pl.off[i]); };
     Args a;
-    a.sum_in = carry.sum_in, a.sum_out = carry.sum_out, a.b_in = carry.b_in, a.b_out = carry.b_out;
     a.B = d.batch, a.T = d.seqlen, a.H = d.nheads, a.P = d.headdim, a.N = d.d_state;
     a.R = d.mimo_rank, a.G = d.ngroups, a.trap = d.use_trapezoidal, a.cplx = d.use_complex;
     a.rs = d.proj_row_stride, a.pl = proj_layout(d), a.eps = d.rms_eps, a.prm = p;
@@ -485,9 +504,14 @@ static int launch_staged(const m3_layer_desc& d, const m3_layer_params& p, const
         const int64_t na = (int64_t)d.batch * ((d.seqlen + kAC - 1) / kAC) * d.nheads * (d.d_state / 2);
         const unsigned ga = (unsigned)((na + NTH - 1) / NTH);
         hipLaunchKernelGGL(lp_angle_sums<T>, dim3(ga), dim3(NTH), 0, stream, a);
-        hipLaunchKernelGGL(lp_angles<T>, dim3(ga), dim3(NTH), 0, stream, a);
+        if (carry.sum_in) hipLaunchKernelGGL((lp_angles<T, true>), dim3(ga), dim3(NTH), 0, stream, a, carry.sum_in);
+        else hipLaunchKernelGGL((lp_angles<T, false>), dim3(ga), dim3(NTH), 0, stream, a, nullptr);
     }
     hipLaunchKernelGGL(lp_prep<T>, dim3(d.batch * d.seqlen), dim3(NTH), lds, stream, a);
+    if (carry.h_in || carry.sum_out) {
+        const int n = a.H * a.R * std::max(a.N, a.P);
+        hipLaunchKernelGGL(lp_hand<T>, dim3((n + NTH - 1) / NTH), dim3(NTH), 0, stream, a, carry);
+    }
     if (launch_chunked_fwd_mfma(a.B, a.T, a.H, a.P, a.N, a.R, a.xg, a.xb, a.Bt, a.Bb, a.Ct, a.dt,
                                 a.A, p.D, a.xr, carry.h_in, a.ys, h_final, ws + pl.chunk_off,
                                 stream) != 0)
@@ -523,7 +547,7 @@ int launch_staged_bf16(const m3_layer_desc& d, const m3_layer_params& p, const v
             const int k = (int)(t / z.tokens);  // the slices alternate between two sets
             const float* in = hand + (k + 1) % 2 * set;
             float* out = hand + k % 2 * set;
-            Carry c;
+            lp::Carry c;
             if (t > 0) c.h_in = in, c.sum_in = in + z.h, c.b_in = d.use_trapezoidal ? in + z.h + z.sum : nullptr;
             if (!last) c.sum_out = out + z.h, c.b_out = d.use_trapezoidal ? out + z.h + z.sum : nullptr;
             auto at = [&](auto* q, int64_t per_row) { return q && last ? q + b * per_row : nullptr; };
