@@ -10,8 +10,8 @@
 // Work decomposition. A workgroup owns (batch, head, PC = 32 NCG headdim columns, segment of
 // the sequence) and walks its chunks of 64 (t, r) rows, Q = 64 / R tokens. PC is the whole
 // headdim (128 or 64) where enough workgroups remain, so the RoPE rotation and the scores,
-// which every column block of a head repeats, are done once per head. Shapes whose (batch,
-// head) pairs do not fill the GPU are cut along the sequence (make_plan): a state-only pass
+// which every column block of a head repeats, are done once per head. Sequences of layers whose
+// heads do not fill the GPU are cut (make_plan): a state-only pass
 // walks every segment but the last from a zero state in its own RoPE frame and leaves its end
 // state, log-decay and angle increment, and seg_combine turns those into the state entering
 // each segment.
@@ -20,16 +20,18 @@
 // state rows, H^T [n][p], in MFMA accumulators (N/32 x 2 tiles), contracts that half for all
 // 64 output rows, swaps the partial sums of half the rows with the other wave through LDS and
 // finishes its own rows. Helper waves (8; 4 for d_state 64) compute the scores and prepare the
-// next chunk's operand tiles. Sixteen waves, four per SIMD: one wave alone issues a VALU
+// next chunk's operand tiles; workgroups of fewer column waves have extra ones for the token
+// scalars and score tiles (extra_waves). Sixteen waves, four per SIMD: one wave alone issues a VALU
 // instruction only every ~9 cycles, so eight waves of 256 registers (whole state rows per
 // wave, no swap) left the VALU and the matrix cores idle (2.6 ms against 2.2 for both passes
 // of the (2, 16384) d_model 2048 call).
 //
-// Bound: VALU issue and LDS bandwidth together. Per chunk of that call 10.5K cycles, in which
-// the SIMDs issue 5.7K cycles of VALU and 2.6K of MFMA and the LDS is busy 6.5K. The call (both
-// passes, seg_combine and the B / C normalisation) takes 2.30 ms, 0.29 of the bf16 MFMA peak;
+// Bound: VALU issue and LDS bandwidth together. A chunk of that call takes a CU 12.2K cycles in
+// the full pass, in which the SIMDs issue 5.1K cycles of VALU and 2.6K of MFMA and the LDS is
+// busy 6.1K (profiles/pmc_segmented_prefill_kernels.md). The call (B / C normalisation 68 us,
+// state pass 640, seg_combine 32, full pass 1,323) takes 2.06 ms, 0.32 of the bf16 MFMA peak;
 // in blocks of 32 columns without segments (256 workgroups, every block repeating the rotation
-// and the scores) it took 2.84 ms.
+// and the scores) it took 2.74 ms.
 //
 // Per chunk, in LDS (f16 unless noted):
 //   C [(t,r)][n], B [(u,r')][n]       C~ / B~: normalised B^ / C^ (bc_norm_wide) rotated
@@ -1045,11 +1047,14 @@ Plan make_plan(const m3_layer_desc& d, size_t limit) {
                         (size_t)d.nheads * d.headdim * d.d_state * sizeof(float),
                         d.nheads * sizeof(float), d.nheads * (d.d_state / 2) * sizeof(float)};
     static_cast<SegPlan&>(p) = plan_segments(d.batch, segs, z, limit, true);
-    // Narrower blocks where the workgroups would leave CUs idle: they repeat the rotation and
-    // the scores, but each walks its chunks faster (same bits: a column's arithmetic does not
-    // depend on its block).
+    // Narrower blocks where they still run at once, one a CU: they repeat the rotation and the
+    // scores, but each walks its chunks faster (same bits: a column's arithmetic does not depend
+    // on its block). us per call in blocks of 128 / 64 / 32 columns, d_state 256 rank 4, headdim
+    // 128, 32 heads, 600 tokens: one sequence 202 / 150 / 134, two 202 / 151 / 134, four 205 / 156
+    // / 263, five 207 / 303 / 391; d_state 128 rank 4, headdim 64, 24 heads, 300 tokens: four
+    // - / 61 / 58, six - / 62 / 112.
     const int64_t bh = (int64_t)p.batch * d.nheads * p.group;
-    while (p.ncg > 1 && bh * (d.headdim / (PW * p.ncg)) < 192) p.ncg /= 2;
+    while (p.ncg > 1 && 2 * bh * (d.headdim / (PW * p.ncg)) <= 256) p.ncg /= 2;
     return p;
 }
 
