@@ -38,11 +38,13 @@
 // holds, the per-token operands the layer backward reads, in the staged fp32 layer path's
 // layouts (m3_layer_fp32.hip), and its chunk-start states.
 //
-// Bound by SIMD issue: 1,500 v_mfma_f32_16x16x4_f32 of 32 cycles per chunk are 12K cycles on
-// four SIMDs, and the helpers' VALU work (about 4K) and the phase tails do not hide under them:
-// 19.7K measured, 8.2 us per chunk and workgroup. d_model 768 over 4 x 1024 tokens (96 (batch,
-// head) pairs): 300 us with two workgroups of 32 columns per pair, state and operands through
-// LDS, all eight waves in step; 212 us with this split (135 + 70 state pass + 7).
+// Bound by SIMD issue: 1,504 v_mfma_f32_16x16x4_f32 of 32 cycles per chunk are 12.0K cycles on
+// four SIMDs, 5,000 other VALU instructions 5.0K, and they add up, with 2.7K of waits at the two
+// barriers, to 19.7K, 8.2 us per chunk and workgroup (profiles/pmc_segmented_prefill_kernels.md).
+// d_model 768 over 4 x 1024 tokens (96 (batch, head) pairs), from a cool clock: 300 us with two
+// workgroups of 32 columns per pair, state and operands through LDS, all eight waves in step;
+// 212 us with this split (135 + 70 state pass + 7); 193 at the sustained clock (118 + 62 + 7 and
+// the normalisation).
 #include <algorithm>
 
 #include "m3_common.h"
