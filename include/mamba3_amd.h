@@ -188,8 +188,9 @@ int m3_layer_bwd(const m3_layer_desc* desc, const m3_layer_params* params, const
 /*
  * Bytes of device workspace m3_prefill_fwd needs for `desc` (0 is possible). bf16 layers that
  * no bf16 MFMA kernel takes run the fp32 layer path in this workspace ("fp32_layer"), in
- * slices of the batch where it is smaller, and the generic kernel, which needs none, where it
- * does not hold one batch row; all of them compute in fp32, so results agree to its rounding.
+ * slices of the batch or of a row's tokens where it is smaller (the same bits), and the generic
+ * kernel, which needs none, where it does not hold a slice of 64 tokens; both compute in fp32,
+ * so their results agree to its rounding.
  * No counterpart in the reference, which allocates inside ATen.
  */
 int m3_prefill_workspace_size(const m3_layer_desc* desc, size_t* bytes);

@@ -912,10 +912,10 @@ def test_bf16_d768_long_prefill_properties(cuda_device):
 
 
 def test_bf16_d2048_long_prefill_properties(cuda_device):
-    """x (2, 16384, 2048) bf16 (the wide-layer workload): every (batch, head, column
-    block) runs independently and chunks start at fixed positions, so a sub-batch and a
-    prefix reproduce the full run bit for bit; the prefill -> step hand-off agrees with
-    the full prefill."""
+    """x (2, 16384, 2048) bf16 (the wide-layer workload): every (batch, head, column block)
+    runs independently, its chunks start at fixed positions, and the cuts of a sequence into
+    segments depend on neither the batch nor the length, so a sub-batch and a prefix reproduce
+    the full run bit for bit; the prefill -> step hand-off agrees with the full prefill."""
     kw = dict(d_model=2048, d_state=256, headdim=128, mimo_rank=4)
     torch.manual_seed(0)
     layer = mamba3_amd.KulaMamba(**kw).to(cuda_device, torch.bfloat16).eval()
