@@ -710,7 +710,7 @@ def _(gate_up, d_ff):
 _PLAIN = frozenset((torch.Tensor, torch.nn.Parameter, type(None)))
 
 
-def _direct(tensors) -> bool:
+def _direct(*tensors) -> bool:
     """Eager calls with autograd off bypass the dispatcher: its per-call host time (16 us for
     the prefill op) is what a per-token decode loop and a short prompt wait on. Traced calls,
     calls under autograd, a dispatch or function mode, a functorch transform or forward-mode
@@ -732,31 +732,31 @@ try:
     _tracing_state, _functorch_stack = _C._get_tracing_state, _C._functorch.peek_interpreter_stack
     _forward_ad._current_level
 except AttributeError:
-    def _direct(tensors) -> bool:
+    def _direct(*tensors) -> bool:
         return False
 
 
 def prefill_fast(*args):
-    return (_prefill_eager if _direct(args[:12]) else prefill)(*args)
+    return (_prefill_eager if _direct(*args[:12]) else prefill)(*args)
 
 
 def step_fast(*args):
-    return (_step_eager if _direct(args[:15]) else step)(*args)
+    return (_step_eager if _direct(*args[:15]) else step)(*args)
 
 
 def small_linear_fast(x, norm_w, eps, weight, residual, scale):
-    fn = _small_linear_eager if _direct((x, norm_w, weight, residual)) else small_linear
+    fn = _small_linear_eager if _direct(x, norm_w, weight, residual) else small_linear
     return fn(x, norm_w, eps, weight, residual, scale)
 
 
 def small_swiglu_fast(x, norm_w, eps, w_gate, w_up):
-    fn = _small_swiglu_eager if _direct((x, norm_w, w_gate, w_up)) else small_swiglu
+    fn = _small_swiglu_eager if _direct(x, norm_w, w_gate, w_up) else small_swiglu
     return fn(x, norm_w, eps, w_gate, w_up)
 
 
 def silu_mul_fast(gate_up, d_ff):
-    return (_silu_mul_eager if _direct((gate_up,)) else silu_mul)(gate_up, d_ff)
+    return (_silu_mul_eager if _direct(gate_up) else silu_mul)(gate_up, d_ff)
 
 
 def rmsnorm_fast(x, weight, eps):
-    return (_rmsnorm_eager if _direct((x, weight)) else rmsnorm)(x, weight, eps)[0]
+    return (_rmsnorm_eager if _direct(x, weight) else rmsnorm)(x, weight, eps)[0]

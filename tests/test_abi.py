@@ -282,16 +282,16 @@ def test_module_calls_under_a_dispatch_mode_go_through_the_ops():
         out, st = layer.step(x[:, 0], st)
         assert out.shape == (2, 64) and st["angle"].shape == (2, layer.nheads, 8)
     t = torch.ones(3)
-    assert not ops._direct((t, t))
+    assert not ops._direct(t, t)
     with torch.no_grad():
-        assert ops._direct((t, torch.nn.Parameter(t)))
-        assert not ops._direct((t.as_subclass(type("Sub", (torch.Tensor,), {})), t))
+        assert ops._direct(t, torch.nn.Parameter(t))
+        assert not ops._direct(t.as_subclass(type("Sub", (torch.Tensor,), {})), t)
         seen = []
-        torch.func.vmap(lambda v: seen.append(ops._direct((t, t))) or v)(t)
+        torch.func.vmap(lambda v: seen.append(ops._direct(t, t)) or v)(t)
         with torch.autograd.forward_ad.dual_level():
-            seen.append(ops._direct((t, t)))
+            seen.append(ops._direct(t, t))
         with torch.device("cpu"):
-            seen.append(ops._direct((t, t)))
+            seen.append(ops._direct(t, t))
         assert seen == [False] * 3
 
 
