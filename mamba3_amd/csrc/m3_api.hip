@@ -152,7 +152,7 @@ int launch_prefill_path(PrefillPath path, const m3_layer_desc& d, const m3_layer
 // current) and kept in g_scratch.
 // Behind the M3_NOALLOC_SCRATCH_BYTES that a call's operands may take lies room for the states of
 // its segments, so that every call that fits runs the same cuts as m3_prefill_fwd: two states
-// (plan_segments) of the widest layer that is cut, 191 x 128 columns of d_state 256, are 50 MB.
+// (plan_segments) of the widest layer that is cut, 95 x 128 columns of d_state 256, are 25 MB.
 constexpr size_t kScratchBytes = M3_NOALLOC_SCRATCH_BYTES + M3_NOALLOC_STATE_BYTES;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 

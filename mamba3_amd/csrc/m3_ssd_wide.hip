@@ -1025,11 +1025,13 @@ void launch_ssd(Args a, int group, hipStream_t stream) {
 // that a sequence gives the same bits alone and in any batch, nor on the workspace (but see
 // plan_segments), nor, as they lie at fixed tokens, on the length, so that a prefix gives the same
 // bits too. They are closer at the start, so that a short prompt splits finely and a long one
-// into few states. Heads whose column blocks alone nearly fill the 256 CUs are not cut: a
-// segmented walk does 1.5x the work (its state pass). (us per call, cut / uncut: d_state 64
-// headdim 64 rank 2, one sequence of 2,048 tokens: 96 heads 130 / 190, 160 171 / 214, 190
-// 201 / 224, of 600 tokens 69 / 67, 78 / 75, 96 / 77; d_state 256 headdim 128 rank 4, 32
-// heads: (1, 16384) 1,030 / 2,789, (2, 16384) 2,072 / 2,956, but (8, 2048) 1,068 / 656.)
+// into few states. Layers of 96 or more column blocks (heads times headdim / 128, 64 or 32) are
+// not cut: a segmented walk does 1.5x the work (its state pass) and repeats its prologue. us per
+// call, cut / uncut, one sequence of 2,048 and 4,096 tokens, d_state 64 headdim 64 rank 2: 8
+// heads 75 / 135 and 110 / 258, 96 122 / 139 and 207 / 260, 128 150 / 140 and 265 / 261, 190 213 /
+// 157 and 387 / 297; d_state 256 headdim 128 rank 4: 32 heads 236 / 372 and 513 / 716, 64 314 /
+// 385 and 574 / 737, 96 569 / 441 and 802 / 847, 128 584 / 449 and 969 / 859. Batches of the
+// 32-head layer: (1, 16384) 1,030 / 2,789, (2, 16384) 2,072 / 2,956, but (8, 2048) 1,068 / 656.
 // The first cut is free, as the state at it is the walk's own: up to two segments a sequence
 // is walked in one piece with the same bits ((1, 600) of that layer 132 us, 199 cut).
 struct Plan : SegPlan {
@@ -1042,7 +1044,7 @@ Plan make_plan(const m3_layer_desc& d, size_t limit) {
     p.ncg = column_groups(d.headdim, d.d_state, d.mimo_rank);
     const int64_t blocks = d.headdim / (PW * p.ncg);
     p.seg0 = std::max(256, d.headdim * d.d_state / 64);
-    const int segs = d.nheads * blocks < 192 ? seg_count(d.seqlen, p.seg0) : 1;
+    const int segs = d.nheads * blocks < 96 ? seg_count(d.seqlen, p.seg0) : 1;
     const SegSizes z = {(size_t)d.seqlen * d.ngroups * d.d_state * d.mimo_rank * sizeof(f16),
                         (size_t)d.nheads * d.headdim * d.d_state * sizeof(float),
                         d.nheads * sizeof(float), d.nheads * (d.d_state / 2) * sizeof(float)};
